@@ -28,10 +28,22 @@ def run(cmd):
     subprocess.check_call(cmd)
 
 
+HIP_SRCS = ["phylo_hip.hip", "prune_mfma.hip", "nni.hip", "learn.hip"]
+
+
 def build_hip(verbose: bool = True) -> str:
-    srcs = [os.path.join(CSRC, "phylo_hip.hip"), os.path.join(CSRC, "learn.hip")]
+    """Compiles the HIP sources side by side, then links them."""
+    from concurrent.futures import ThreadPoolExecutor
+    inc = "-I" + os.path.join(ROOT, "include")
+    obj_dir = os.path.join(CSRC, "_build")
+    os.makedirs(obj_dir, exist_ok=True)
+    objs = [os.path.join(obj_dir, f + ".o") for f in HIP_SRCS]
+    flags = [f for f in HIP_FLAGS if f != "-shared"]
+    with ThreadPoolExecutor(len(HIP_SRCS)) as ex:
+        list(ex.map(lambda p: run([HIPCC, *flags, inc, "-c", "-o", p[1], os.path.join(CSRC, p[0])]),
+                    zip(HIP_SRCS, objs)))
     tmp = LIB + ".tmp"
-    run([HIPCC, *HIP_FLAGS, "-I" + os.path.join(ROOT, "include"), "-o", tmp, *srcs])
+    run([HIPCC, *HIP_FLAGS, "-o", tmp, *objs])
     os.replace(tmp, LIB)
     return LIB
 

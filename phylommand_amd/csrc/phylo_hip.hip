@@ -39,247 +39,12 @@
 
 #include "../../include/phylo_hip.h"
 #include "model_math.h"
+#include "nni.h"
+#include "prune_mfma.h"
+#include "prune_device.h"
 
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kMaxCat = 8;
-constexpr int kMaxStates = 32;
-constexpr double kLn2 = 0.69314718055994530942;
-constexpr int kRootCatOff = 32;   // roots[]: per-state weights [0, 32), category weights after
-
-// Workgroups per CU below which a whole-tree launch has too few waves to
-// hide its dependent chain: every site block is then walked as subtree
-// pieces plus the top program (the tail split applied to all blocks), which
-// multiplies the independent waves by the number of pieces.
-constexpr int kSplitAllBelowPerCu = 4;
-
-// Site groups per wave of the MFMA walker: two independent MFMA chains per
-// wave share each P operand load and overlap their memory latency.
-constexpr int kMfmaGroups = 2;
-
-enum SrcKind : int { SRC_TIP = 0, SRC_CLV = 1, SRC_CARRY_A = 2, SRC_CARRY_B = 3, SRC_NONE = 4 };
-// OP_SWAP: the children were swapped into kind order (order_children); the
-// stochastic rounding of a stored result is keyed by them in their original
-// order.
-// OP_SH_*: one-hot hints for the four commonest child shapes (children in
-// kind order), set by order_children; the DNA walker tests them before its
-// switch, the matrix walker runs a specialised op for each.
-enum OpFlags : int {
-    OP_ROOT = 1, OP_TO_B = 2, OP_SWAP = 4,
-    OP_SH_AT = 8, OP_SH_TT = 16, OP_SH_AB = 32, OP_SH_AC = 64,
-    OP_SH_ALL = OP_SH_AT | OP_SH_TT | OP_SH_AB | OP_SH_AC
-};
-
-struct alignas(16) Op {
-    int l_node, r_node;   // child node ids: P matrices are per (child node, category)
-    int l_kind, r_kind;   // SrcKind
-    int l_idx, r_idx;     // tip row or partial slot
-    int out_slot;         // slot to store the result in, -1 for none
-    int flags;            // OpFlags
-};
-
-// ---------------------------------------------------------------------------
-// Device helpers
-// ---------------------------------------------------------------------------
-
-__device__ inline void load4(const float* p, double v[4]) {
-    const float4 x = *reinterpret_cast<const float4*>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-}
-__device__ inline void load4(const double* p, double v[4]) {
-    const double2 a = reinterpret_cast<const double2*>(p)[0];
-    const double2 b = reinterpret_cast<const double2*>(p)[1];
-    v[0] = a.x; v[1] = a.y; v[2] = b.x; v[3] = b.y;
-}
-__device__ inline void load_raw4(const float* p, float v[4]) {
-    const float4 x = *reinterpret_cast<const float4*>(p);
-    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
-}
-__device__ inline void load_raw4(const double* p, double v[4]) { load4(p, v); }
-__device__ inline void store4(float* p, const float v[4]) {
-    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-}
-__device__ inline void store4(double* p, const double v[4]) {
-    reinterpret_cast<double2*>(p)[0] = make_double2(v[0], v[1]);
-    reinterpret_cast<double2*>(p)[1] = make_double2(v[2], v[3]);
-}
-
-// 32-bit integer hash (Wellons' "lowbias32" xorshift-multiply mix).
-__device__ inline uint32_t mix32(uint32_t x) {
-    x ^= x >> 16;
-    x *= 0x7feb352du;
-    x ^= x >> 15;
-    x *= 0x846ca68bu;
-    x ^= x >> 16;
-    return x;
-}
-
-// Rounding of a partial (x >= 0) to the storage type.  FP32 storage rounds
-// stochastically: 29 random bits are added below the float's last mantissa
-// bit of the FP64 value and the bits a float does not hold are cut off, so x
-// rounds up with probability equal to its distance from the float below.  A
-// subtree with few tips produces the same few values at every site, so
-// round-to-nearest would repeat the same error at thousands of sites and the
-// total lnL would drift (+4.6e-3 at 128 taxa x 100,000 sites); with
-// per-site random bits the errors average out.  The bits come from a hash of
-// (site, node, category) stepped by a Weyl sequence per state, so results
-// are reproducible and the same node rounds the same way in every program
-// that computes it.  (Zero stays zero; values below the float normal range
-// end as the nearest float of the truncated value.)
-// The dithered cut and the power-of-two scaling commute (the cut reads only
-// mantissa bits), so a walker may cut before or after scaling a partial.
-__device__ inline double round_cut(double x, uint32_t bits, float) {
-    // 64-bit add of the 29 dither bits, written on 32-bit halves
-    const uint32_t lo = (uint32_t)__double2loint(x);
-    const uint32_t sum = lo + (bits >> 3);
-    const uint32_t hi = (uint32_t)__double2hiint(x) + (sum < lo ? 1u : 0u);
-    return __hiloint2double((int)hi, (int)(sum & 0xe0000000u));   // <= 24 significant bits
-}
-__device__ inline double round_cut(double x, uint32_t, double) { return x; }
-
-// Random bits for the partials of one (site, node, category); state i uses
-// key + i * 0x9e3779b9.  The node is identified by its two children, in the
-// order the program builder gave them.
-__device__ inline uint32_t round_key(int s, int l_node, int r_node, int cat) {
-    return mix32((uint32_t)s * 0x9e3779b1u ^ ((uint32_t)l_node * 0x85ebca77u + (uint32_t)r_node * 0x27d4eb2fu +
-                                              (uint32_t)cat * 0xc2b2ae3du));
-}
-__device__ inline uint32_t round_key(int s, const Op& op, int cat) {
-    return (op.flags & OP_SWAP) ? round_key(s, op.r_node, op.l_node, cat) : round_key(s, op.l_node, op.r_node, cat);
-}
-
-__device__ inline double wave_sum(double v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
-}
-
-// Compensated sum of partial[0, n) by one wave in a fixed order: lane l adds
-// partial[l], partial[l + 64], ... with Kahan compensation, then the lanes'
-// (sum, error) pairs meet in a two-sum butterfly.  Every lane returns the
-// same total (two-sum gives the exact error whichever operand comes first).
-// Adds b + bl to the compensated pair (hi, lo) by Knuth's two-sum.
-__device__ inline void two_sum_add(double& hi, double& lo, double b, double bl) {
-    const double t = hi + b;
-    const double bb = t - hi;
-    const double err = (hi - (t - bb)) + (b - bb);
-    hi = t;
-    lo = (lo + bl) + err;
-}
-
-// Threads of the compensated sum: one workgroup per program.
-constexpr int kSumThreads = 256;
-
-// Compensated fixed-order sum of partial[0, n) by one workgroup of
-// kSumThreads.  Each thread issues its loads eight at a time before adding
-// them (Kahan), so their latencies overlap instead of queueing; the threads'
-// (sum, error) pairs then meet by two-sum, in a butterfly within each wave
-// and in LDS across the waves.  Thread 0 returns the total.
-__device__ inline double block_total(const double* partial, int n) {
-    double s = 0.0, comp = 0.0;
-    for (int base = threadIdx.x; base < n; base += 8 * kSumThreads) {
-        double v[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = base + u * kSumThreads;
-            v[u] = i < n ? partial[i] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (base + u * kSumThreads < n) {
-                const double x = v[u] - comp;
-                const double t = s + x;
-                comp = (t - s) - x;
-                s = t;
-            }
-        }
-    }
-    double hi = s, lo = -comp;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) two_sum_add(hi, lo, __shfl_xor(hi, o, 64), __shfl_xor(lo, o, 64));
-    __shared__ double red_hi[kSumThreads / 64], red_lo[kSumThreads / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) { red_hi[wid] = hi; red_lo[wid] = lo; }
-    __syncthreads();
-    hi = red_hi[0];
-    lo = red_lo[0];
-#pragma unroll
-    for (int w = 1; w < kSumThreads / 64; ++w) two_sum_add(hi, lo, red_hi[w], red_lo[w]);
-    return hi + lo;
-}
-
-// Sums v over the workgroup (any multiple of 64 threads); thread 0 stores it.
-__device__ inline void block_sum_store(double v, double* dst) {
-    __shared__ double red[16];
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) red[wid] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < (int)(blockDim.x >> 6); ++w) t += red[w];
-        *dst = t;
-    }
-}
-
-// The top launch of a tail split (its workgroups are the last blocks to
-// finish an evaluation) folds in the final sum: each workgroup, once its
-// partial is stored, counts itself in; the last one sums every block's
-// partial in block_total's order (so the total equals final_sum_kernel's),
-// writes it to the host-mapped total and returns the counter to zero.  The
-// fences publish the few partials this launch wrote and drop stale copies
-// before the sum reads them.  Workgroups of kSumThreads threads only.
-__device__ inline void fold_total(const double* partial, int n_part, unsigned* counter, double* total) {
-    __shared__ int last;
-    if (threadIdx.x == 0) {
-        __threadfence();
-        last = atomicAdd(counter, 1u) == gridDim.x - 1;
-        if (last) __threadfence();
-    }
-    __syncthreads();
-    if (last) {
-        const double t = block_total(partial, n_part);
-        if (threadIdx.x == 0) {
-            *total = t;
-            *counter = 0u;
-        }
-    }
-}
-
-// Bit j of a tip's state set as 1.0 or 0.0: a bit-field extract and an
-// integer-to-double conversion.  (Building the double's high word from a
-// mask needs a third instruction to copy the zero low word into each
-// register pair; the conversion form ran the C2 kernel 1 % faster.)
-template <int J>
-__device__ inline double tip_bit(unsigned code) {
-    return (double)((code >> J) & 1u);
-}
-
-// frexp exponent of the largest of four values (0 if none is positive): as
-// signed integers the high words of positive doubles order like the values,
-// and those of negative ones (P(t) from the eigen system can leave tiny
-// negative partials) are negative, so they never win.
-__device__ inline int max_exponent(const double (&L)[4]) {
-    const int h = max(max(__double2hiint(L[0]), __double2hiint(L[1])), max(__double2hiint(L[2]), __double2hiint(L[3])));
-    int e = (h >> 20) - 1022;
-    if (h < 0x00100000) {   // no positive normal value: zero, subnormal or negative maximum
-        const double mx = fmax(fmax(L[0], L[1]), fmax(L[2], L[3]));
-        e = 0;
-        if (mx > 0.0) (void)frexp(mx, &e);
-    }
-    return e;
-}
-
-// The largest high word of four doubles, as signed integers: for positive
-// values it orders like the values (negative ones never win).
-__device__ inline int max_hi_word(const double (&L)[4]) {
-    return max(max(__double2hiint(L[0]), __double2hiint(L[1])), max(__double2hiint(L[2]), __double2hiint(L[3])));
-}
-
-// High word of 2^-256: carried DNA partials whose largest entry is below it
-// are rescaled (walk4).
-constexpr int kLazyRescaleHi = (1023 - 256) << 20;
 
 // One child's operand for a walker op, by source kind (compile-time).
 // With TL the tip's state set comes from the workgroup's LDS copy, one byte
@@ -570,21 +335,8 @@ __device__ inline double combine_categories(double lc, int sc, int cat, int lane
     return log(lc) + sc * kLn2;
 }
 
-// Taxa whose tip codes a DNA workgroup stages in LDS (one byte per site,
-// sized at launch).
-constexpr int kTipLdsTaxa = 256;
-inline size_t tip_lds_bytes(int n_taxa) { return (size_t)n_taxa * 64; }
-
-// Plain launch (prog_main < 0): grid = (m_pad / 64, n_programs); workgroup
+// Plain launch (prog_main = -1): grid = (m_pad / 64, n_programs); workgroup
 // (x, y) runs ops[prog_begin[y] .. prog_begin[y+1]) over site block x.
-// Program-major launch (prog_main = -2, n_main site blocks, n_tail
-// programs, blk0 programs a workgroup; 1-D grid of 8 ceil(n_main / 8)
-// ceil(n_tail / blk0) workgroups): workgroup i runs on XCD i % 8
-// (workgroups are dealt to the XCDs in turn), and XCD k's workgroups take
-// site blocks k, k + 8, ... each with every group of blk0 consecutive
-// programs in turn, so the programs of one site block read its stored
-// partials through one L2.  Program p over block b writes
-// partial[p n_main + b], as a plain launch does.
 // Split launch (prog_main >= 0, grid.y = 1; build_split_programs): workgroups
 // x < n_main run program prog_main over site block blk0 + x; the others run
 // piece program prog_piece + (x - n_main) / n_tail over site block
@@ -621,11 +373,6 @@ __global__ __launch_bounds__(64 * C) void prune4_kernel(
             prog = prog_piece + r / n_tail;
             has_root = false;
         }
-    } else if (prog_main == -2) {
-        const int slot = (int)blockIdx.x >> 3, n_pg = (n_tail + blk0 - 1) / blk0;
-        prog = slot % n_pg * blk0;
-        bx = slot / n_pg * 8 + ((int)blockIdx.x & 7);
-        if (bx >= n_main) return;        // the last group's padding (uniform per workgroup)
     }
     const int s = bx * 64 + lane;
     if (TL) {
@@ -639,26 +386,6 @@ __global__ __launch_bounds__(64 * C) void prune4_kernel(
             reinterpret_cast<uint32_t*>(tl)[i] = (w << 4) & 0xF0F0F0F0u;
         }
         __syncthreads();
-    }
-    if constexpr (!TL) {
-        if (prog_main == -2) {
-            // blk0 programs of one site block, one after another
-            const int p_end = min(prog + blk0, n_tail);
-            for (int p = prog; p < p_end; ++p) {
-                double lc;
-                int sc;
-                walk4<T, C, false>(ops, prog_begin[p], prog_begin[p + 1], tips, tl, tipv, clv, scl, P, roots, m_pad,
-                                   s, lane, cat, xb, lc, sc);
-                const double lnl = combine_categories<C, true>(lc, sc, cat, lane, xroot, xsc);
-                const bool live = s < m && cat == 0;
-                if (live && site_lnl) site_lnl[(size_t)p * m + s] = lnl;
-                if (cat == 0) {
-                    const double v = wave_sum(live ? (site_w ? site_w[s] : 1.0) * lnl : 0.0);
-                    if (lane == 0) partial[(size_t)p * n_main + bx] = v;
-                }
-            }
-            return;
-        }
     }
     double lc;
     int sc;
@@ -771,598 +498,6 @@ __global__ __launch_bounds__(64) void segment_sum_kernel(const double* __restric
         s = t;
     }
     out[k] = s;
-}
-
-// ---------------------------------------------------------------------------
-// Wide-state walker on the matrix cores (4 < S <= 32, FP64 arithmetic).
-//
-// One wave = G groups of 16 sites x one rate category; a workgroup holds the
-// C category waves of the same G site groups.  Each child product is a GEMM
-//     out[state row][site] = sum_k P[row][k] * L[k][site]
-// done as v_mfma_f64_16x16x4f64 steps (A = P: 16 rows x 4 k, B = L: 4 k x 16
-// sites, D = 16 rows x 16 sites; D[i][j] sits in lane j + 16 (i % 4),
-// register i / 4).  Lane l serves site l % 16 and lane group g = l / 16; slot
-// t of a lane holds state 4t + g, and row i of tile T is state 16T + i, so an
-// MFMA result (tile T, register r) is slot 4T + r of the next op's operand
-// with no shuffles.  V = ceil(S / 4) slots cover the S states; tile 1 exists
-// for S > 16 (for 17..20 states as v_mfma_f64_4x4x4f64 blocks, see
-// pmfma_kernel).  Partials are stored as [slot][cat][site group][V][64 lanes]
-// (every load and store a full row), P as [node][cat][tile][V][64] doubles
-// (pmfma_kernel).  FP64 matrix cores rather than FP32 ones: the FP32 MFMA
-// dot products truncate small addends (about -0.1 ulp per 5-step chain on
-// transition-matrix-shaped operands), which biases every site the same way.
-// Scalers as in the DNA walker: one int32 power of two per (node, category,
-// site), the categories meeting only at the root.
-// ---------------------------------------------------------------------------
-
-typedef double mfma_d4 __attribute__((ext_vector_type(4)));
-
-__host__ __device__ constexpr int mfma_slots(int S) { return (S + 3) / 4; }
-
-// Pm[node][cat][T][t][lane] = P[16T + lane % 16][4t + lane / 16] (0 outside S),
-// the A operand of v_mfma_f64_16x16x4f64 for row tile T and K-step t.  With
-// V = 5 (17..20 states) tile 1 holds only rows 16..19 and is instead the A
-// operand of v_mfma_f64_4x4x4f64 (four 4x4 blocks, one per 4 sites): lane l
-// = 4b + 16k + i holds P[16 + i][4t + k] for every block b.  That product
-// lands as D[lane j + 16 i] = row 16 + i of site j, the operand slot of
-// states 16..19, with no padded rows.
-__global__ void pmfma_kernel(const double* __restrict__ P, int S, int Sp, int C, int n_nodes, int V, int TN,
-                             double* __restrict__ Pm) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)n_nodes * C * TN * V * 64;
-    if (gid >= total) return;
-    const int l = gid % 64;
-    const int t = (gid / 64) % V;
-    const int T = (gid / (64L * V)) % TN;
-    const long mat = gid / (64L * V * TN);          // node * C + cat
-    const bool short_tile = V == 5 && T == 1;
-    const int row = 16 * T + (short_tile ? l % 4 : l % 16), col = 4 * t + l / 16;
-    Pm[gid] = (row < S && col < S) ? P[(mat * Sp + row) * Sp + col] : 0.0;
-}
-
-// PTm[node][cat][k][i] = P[i][k] for k < S, PTm[..][S][i] = sum_q P[i][q]
-// (the product with an all-states tip), i < 4V (0 for i >= S): the columns a
-// single-state or all-states tip selects.
-__global__ void ptm_kernel(const double* __restrict__ P, int S, int Sp, int C, int n_nodes, int W,
-                           double* __restrict__ PTm) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)n_nodes * C * (S + 1) * W;
-    if (gid >= total) return;
-    const int i = gid % W;
-    const int k = (gid / W) % (S + 1);
-    const long mat = gid / ((long)W * (S + 1));
-    const double* row = P + (mat * Sp + i) * Sp;
-    double v = 0.0;
-    if (i < S) {
-        if (k < S) v = row[k];
-        else
-            for (int q = 0; q < S; ++q) v += row[q];
-    }
-    PTm[gid] = v;
-}
-
-__device__ inline double to_d(float x) { return (double)x; }
-__device__ inline double to_d(double x) { return x; }
-
-// Largest state value of a site in the matrix walker's layout (states 4t + g
-// in slot t of lane group g, so the maximum runs over the slots and then the
-// four lane groups: lanes l ^ 16, l ^ 32), and its frexp exponent (0 when no
-// state is positive).  Every lane of the wave must take part.
-template <int V>
-__device__ inline double site_max(const double (&v)[V]) {
-    double mx = 0.0;
-#pragma unroll
-    for (int t = 0; t < V; ++t) mx = fmax(mx, v[t]);
-    mx = fmax(mx, __shfl_xor(mx, 16, 64));
-    return fmax(mx, __shfl_xor(mx, 32, 64));
-}
-template <int V>
-__device__ inline int site_exponent(const double (&v)[V]) {
-    const double mx = site_max<V>(v);
-    int e = 0;
-    if (mx > 0.0) (void)frexp(mx, &e);
-    return e;
-}
-
-// One child for the G site groups of a wave: acc[q][T] = P . x for tile T,
-// x in operand order.  The P operand of each K-step is loaded once and used by
-// every group.
-template <typename T, int C, int V, int G, bool TL>
-__device__ inline void mfma_child(int kind, int idx, int node, int cat, const int (&s)[G], int sg0, int n_sg,
-                                  int lane, int g, int m_pad, int S, uint32_t full,
-                                  const uint32_t* __restrict__ tips, const uint32_t* tl, const T* clv,
-                                  size_t slot_stride,
-                                  const int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm,
-                                  const double (&cA)[G][V], const int (&sA)[G], const double* cB,
-                                  const int (&sB)[G], mfma_d4 (&acc)[G][2], int (&sc)[G]) {
-    constexpr int TN = V > 4 ? 2 : 1;
-    double x[G][V];
-    if (kind == SRC_TIP) {
-        uint32_t mk[G];
-        bool simple = true;
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            mk[q] = TL ? tl[idx * 16 * G + 16 * q + (lane & 15)] : tips[(size_t)idx * m_pad + s[q]];
-            simple = simple && (mk[q] == full || __popc(mk[q]) == 1);
-        }
-        // a wave whose sites are all single states or gaps selects columns of P
-        if (__all(simple)) {
-            const double* base = PTm + ((size_t)node * C + cat) * (S + 1) * (4 * V) + g;
-#pragma unroll
-            for (int q = 0; q < G; ++q) {
-                const int col = mk[q] == full ? S : __ffs(mk[q]) - 1;
-                const double* pt = base + (size_t)col * (4 * V);
-#pragma unroll
-                for (int t = 0; t < V; ++t) acc[q][t / 4][t % 4] = pt[4 * t];
-            }
-            return;
-        }
-#pragma unroll
-        for (int q = 0; q < G; ++q)
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = (mk[q] >> (4 * t + g)) & 1u ? 1.0 : 0.0;
-    } else if (kind == SRC_CLV) {
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const T* src = clv + (size_t)idx * slot_stride + ((size_t)cat * n_sg + sg0 + q) * V * 64 + lane;
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = to_d(src[t * 64]);
-            sc[q] += scl[((size_t)idx * C + cat) * m_pad + s[q]];
-        }
-    } else if (kind == SRC_CARRY_A) {
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = to_d(cA[q][t]);
-            sc[q] += sA[q];
-        }
-    } else {
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = cB[(q * V + t) * 64];
-            sc[q] += sB[q];
-        }
-    }
-    const double* pm = Pm + ((size_t)node * C + cat) * TN * V * 64 + lane;
-#pragma unroll
-    for (int T2 = 0; T2 < TN; ++T2) {
-#pragma unroll
-        for (int q = 0; q < G; ++q) acc[q][T2] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-        if (V == 5 && T2 == 1) {
-            // states 16..19: four 4x4x4 blocks give exactly the 4 rows
-            double d[G];
-#pragma unroll
-            for (int q = 0; q < G; ++q) d[q] = 0.0;
-#pragma unroll
-            for (int t = 0; t < V; ++t) {
-                const double a = pm[(V + t) * 64];
-#pragma unroll
-                for (int q = 0; q < G; ++q) d[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(a, x[q][t], d[q], 0, 0, 0);
-            }
-#pragma unroll
-            for (int q = 0; q < G; ++q) acc[q][1][0] = d[q];
-            continue;
-        }
-#pragma unroll
-        for (int t = 0; t < V; ++t) {
-            const double a = pm[(T2 * V + t) * 64];
-#pragma unroll
-            for (int q = 0; q < G; ++q)
-                acc[q][T2] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, x[q][t], acc[q][T2], 0, 0, 0);
-        }
-    }
-}
-
-// The P operand of one child for every row tile and K-step (Pm order: tile
-// T, K-step t at register T V + t).
-template <int C, int V>
-__device__ __forceinline__ void load_pm(int node, int cat, int lane, const double* __restrict__ Pm,
-                                        double (&pf)[(V > 4 ? 2 : 1) * V]) {
-    constexpr int TN = V > 4 ? 2 : 1;
-    const double* pm = Pm + ((size_t)node * C + cat) * TN * V * 64 + lane;
-#pragma unroll
-    for (int i = 0; i < TN * V; ++i) pf[i] = pm[i * 64];
-}
-
-// r = P . x for the G site groups with the P operand in registers: the same
-// matrix instructions in the same order as mfma_child; r[q][t] is state
-// 4t + g of group q's site.
-template <int V, int G>
-__device__ __forceinline__ void mfma_products(const double (&pf)[(V > 4 ? 2 : 1) * V], const double (&x)[G][V],
-                                              double (&r)[G][V]) {
-    constexpr int TN = V > 4 ? 2 : 1;
-    mfma_d4 acc[G][2];
-#pragma unroll
-    for (int T2 = 0; T2 < TN; ++T2) {
-        if (V == 5 && T2 == 1) {
-            double d[G];
-#pragma unroll
-            for (int q = 0; q < G; ++q) d[q] = 0.0;
-#pragma unroll
-            for (int t = 0; t < V; ++t)
-#pragma unroll
-                for (int q = 0; q < G; ++q) d[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(pf[V + t], x[q][t], d[q], 0, 0, 0);
-#pragma unroll
-            for (int q = 0; q < G; ++q) acc[q][1][0] = d[q];
-            continue;
-        }
-#pragma unroll
-        for (int q = 0; q < G; ++q) acc[q][T2] = mfma_d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int t = 0; t < V; ++t)
-#pragma unroll
-            for (int q = 0; q < G; ++q)
-                acc[q][T2] = __builtin_amdgcn_mfma_f64_16x16x4f64(pf[T2 * V + t], x[q][t], acc[q][T2], 0, 0, 0);
-    }
-#pragma unroll
-    for (int q = 0; q < G; ++q)
-#pragma unroll
-        for (int t = 0; t < V; ++t) r[q][t] = acc[q][t / 4][t % 4];
-}
-
-// A tip child's state masks for the G site groups, and whether every site of
-// the wave is a single state or a gap (then the child's factor is a column
-// of P).
-template <int G, bool TL>
-__device__ __forceinline__ bool tip_masks(int idx, const int (&s)[G], int lane, int m_pad, uint32_t full,
-                                          const uint32_t* __restrict__ tips, const uint32_t* tl, uint32_t (&mk)[G]) {
-    bool simple = true;
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        mk[q] = TL ? tl[idx * 16 * G + 16 * q + (lane & 15)] : tips[(size_t)idx * m_pad + s[q]];
-        simple = simple && (mk[q] == full || __popc(mk[q]) == 1);
-    }
-    return __all(simple);
-}
-
-// One child's factor in a shape-specialised op: a tip's P columns (col) or
-// products with its state indicators, a stored or carried partial's products.
-template <int K, typename T, int C, int V, int G>
-__device__ __forceinline__ void mfma_factor(bool col, const double (&cols)[G][V], const uint32_t (&mk)[G], int node,
-                                            int cat, int lane, int g, const double* __restrict__ Pm,
-                                            const double (&pf)[(V > 4 ? 2 : 1) * V], const T (&xr)[G][V],
-                                            const double (&cA)[G][V], const double* cB, double (&r)[G][V]) {
-    if constexpr (K == SRC_TIP) {
-        if (col) {
-#pragma unroll
-            for (int q = 0; q < G; ++q)
-#pragma unroll
-                for (int t = 0; t < V; ++t) r[q][t] = cols[q][t];
-            return;
-        }
-        double pt[(V > 4 ? 2 : 1) * V], x[G][V];
-        load_pm<C, V>(node, cat, lane, Pm, pt);
-#pragma unroll
-        for (int q = 0; q < G; ++q)
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = (mk[q] >> (4 * t + g)) & 1u ? 1.0 : 0.0;
-        mfma_products<V, G>(pt, x, r);
-    } else if constexpr (K == SRC_CLV) {
-        double x[G][V];
-#pragma unroll
-        for (int q = 0; q < G; ++q)
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = to_d(xr[q][t]);
-        mfma_products<V, G>(pf, x, r);
-    } else if constexpr (K == SRC_CARRY_A) {
-        mfma_products<V, G>(pf, cA, r);
-    } else {
-        double x[G][V];
-#pragma unroll
-        for (int q = 0; q < G; ++q)
-#pragma unroll
-            for (int t = 0; t < V; ++t) x[q][t] = cB[(q * V + t) * 64];
-        mfma_products<V, G>(pf, x, r);
-    }
-}
-
-// An op of child shape (LK, RK) (kind order, RK != SRC_NONE): the tip masks
-// are read first, then every load of the op (P operands, stored partials and
-// their scalers, tip columns) is issued before the first product, so the two
-// children's memory latencies overlap.  val = left factor x right factor and
-// sc = the children's scalers, as the generic op computes them.
-template <int LK, int RK, typename T, int C, int V, int G, bool TL>
-__device__ __forceinline__ void mfma_shape(const Op& op, int cat, const int (&s)[G], int sg0, int n_sg, int lane,
-                                           int g, int m_pad, int S, uint32_t full, const uint32_t* __restrict__ tips,
-                                           const uint32_t* tl, const T* clv, size_t slot_stride, const int* scl,
-                                           const double* __restrict__ Pm, const double* __restrict__ PTm,
-                                           const double (&cA)[G][V], const int (&sA)[G], const double* cB,
-                                           const int (&sB)[G], double (&val)[G][V], int (&sc)[G]) {
-    constexpr int TNV = (V > 4 ? 2 : 1) * V;
-    uint32_t mkL[G], mkR[G];
-    bool colL = false, colR = false;
-    if constexpr (LK == SRC_TIP) colL = tip_masks<G, TL>(op.l_idx, s, lane, m_pad, full, tips, tl, mkL);
-    if constexpr (RK == SRC_TIP) colR = tip_masks<G, TL>(op.r_idx, s, lane, m_pad, full, tips, tl, mkR);
-    double pL[TNV], pR[TNV];
-    if constexpr (LK != SRC_TIP) load_pm<C, V>(op.l_node, cat, lane, Pm, pL);
-    T xL[G][V], xR[G][V];
-    const auto load_stored = [&](int idx, T (&xr)[G][V]) {
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const T* src = clv + (size_t)idx * slot_stride + ((size_t)cat * n_sg + sg0 + q) * V * 64 + lane;
-#pragma unroll
-            for (int t = 0; t < V; ++t) xr[q][t] = src[t * 64];
-            sc[q] += scl[((size_t)idx * C + cat) * m_pad + s[q]];
-        }
-    };
-    if constexpr (LK == SRC_CLV) load_stored(op.l_idx, xL);
-    if constexpr (RK == SRC_CLV) load_stored(op.r_idx, xR);
-    double gL[G][V], gR[G][V];
-    const auto tip_columns = [&](int node, const uint32_t (&mk)[G], double (&cols)[G][V]) {
-        const double* base = PTm + ((size_t)node * C + cat) * (S + 1) * (4 * V) + g;
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            const int col = mk[q] == full ? S : __ffs(mk[q]) - 1;
-            const double* pt = base + (size_t)col * (4 * V);
-#pragma unroll
-            for (int t = 0; t < V; ++t) cols[q][t] = pt[4 * t];
-        }
-    };
-    if constexpr (LK == SRC_TIP)
-        if (colL) tip_columns(op.l_node, mkL, gL);
-    if constexpr (RK == SRC_TIP)
-        if (colR) tip_columns(op.r_node, mkR, gR);
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        if constexpr (LK == SRC_CARRY_A || RK == SRC_CARRY_A) sc[q] += sA[q];
-        if constexpr (LK == SRC_CARRY_B || RK == SRC_CARRY_B) sc[q] += sB[q];
-    }
-    mfma_factor<LK, T, C, V, G>(colL, gL, mkL, op.l_node, cat, lane, g, Pm, pL, xL, cA, cB, val);
-    if constexpr (RK != SRC_TIP) load_pm<C, V>(op.r_node, cat, lane, Pm, pR);
-    double r[G][V];
-    mfma_factor<RK, T, C, V, G>(colR, gR, mkR, op.r_node, cat, lane, g, Pm, pR, xR, cA, cB, r);
-#pragma unroll
-    for (int q = 0; q < G; ++q)
-#pragma unroll
-        for (int t = 0; t < V; ++t) val[q][t] *= r[q][t];
-}
-
-// grid = (m_pad / (16 G), n_programs), block = 64 * C: wave c computes
-// category c of the G 16-site groups starting at group G * x of site block
-// x (blockIdx.x in a plain launch; the tail-split mapping of prune4_kernel
-// otherwise).
-// Taxa whose tip masks a wide-state workgroup stages in LDS.
-constexpr int kMfmaTipLdsTaxa = 128;
-
-// TL (n_taxa <= kMfmaTipLdsTaxa): the workgroup first copies the tip masks of
-// its 16 G sites into LDS (tl[16 G t + site]).
-// MP: the program-major launch of prune4_kernel (n_main site blocks, n_tail
-// programs, blk0 of them a workgroup, grouped by XCD), one program after
-// another in the workgroup.
-template <typename T, int C, int V, int G, bool TL, bool MP>
-__device__ __forceinline__ void prune_mfma_walk(
-    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
-    int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
-    const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
-    int S, uint32_t full, int n_taxa, int n_main, int prog_main, int blk0, int prog_piece, int tail0, int n_tail,
-    unsigned* fold_counter, double* fold_out) {
-    __shared__ int xsc[C][16 * G];
-    __shared__ double xroot[C][16 * G];
-    __shared__ uint32_t tl[TL ? kMfmaTipLdsTaxa * 16 * G : 1];
-    __shared__ double xb[C][G * V * 64];    // each wave's carry B (LDS keeps the registers for the products)
-    // work mapping as in prune4_kernel (plain or tail-split launch)
-    const int y = blockIdx.y;
-    int bx = blockIdx.x, prog = y;
-    bool has_root = true;
-    if (prog_main >= 0) {
-        if ((int)blockIdx.x < n_main) {
-            bx = blk0 + (int)blockIdx.x;
-            prog = prog_main;
-        } else {
-            const int r = (int)blockIdx.x - n_main;
-            bx = tail0 + r % n_tail;
-            prog = prog_piece + r / n_tail;
-            has_root = false;
-        }
-    } else if (MP) {
-        const int slot = (int)blockIdx.x >> 3, n_pg = (n_tail + blk0 - 1) / blk0;
-        prog = slot % n_pg * blk0;
-        bx = slot / n_pg * 8 + ((int)blockIdx.x & 7);
-        if (bx >= n_main) return;        // the last group's padding (uniform per workgroup)
-    }
-    if (TL) {
-        const uint32_t* blk = tips + (size_t)bx * 16 * G;
-        for (int i = threadIdx.x; i < n_taxa * 16 * G; i += 64 * C)
-            tl[i] = blk[(size_t)(i / (16 * G)) * m_pad + i % (16 * G)];
-        __syncthreads();
-    }
-    const int lane = threadIdx.x & 63;
-    const int g = lane >> 4, j = lane & 15;
-    const int cat = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int sg0 = bx * G, n_sg = m_pad >> 4;
-    int s[G];
-#pragma unroll
-    for (int q = 0; q < G; ++q) s[q] = (sg0 + q) * 16 + j;
-    const int p_end = MP ? min(prog + blk0, n_tail) : prog + 1;
-    int p = prog;
-    do {    // MP: the workgroup's programs in turn; otherwise once
-    const int k0 = prog_begin[p], k1 = prog_begin[p + 1];
-    const size_t slot_stride = (size_t)C * m_pad * 4 * V;
-    // carried results stay in FP64 and are rescaled lazily, as in the DNA
-    // walker; only stored partials are rounded to T
-    double cA[G][V];
-    int sA[G], sB[G];
-    double* const cB = &xb[cat][lane];      // carry B: (group q, slot t) at cB[64 (q V + t)]
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-#pragma unroll
-        for (int t = 0; t < V; ++t) { cA[q][t] = 0.0; cB[(q * V + t) * 64] = 0.0; }
-        sA[q] = 0;
-        sB[q] = 0;
-    }
-    double lnl[G];
-#pragma unroll
-    for (int q = 0; q < G; ++q) lnl[q] = 0.0;
-    Op nxt = ops[k0];
-    for (int k = k0; k < k1; ++k) {
-        const Op op = nxt;
-        nxt = ops[k + 1];     // in flight during this op (an op buffer ends with one pad op)
-        int sc[G];
-#pragma unroll
-        for (int q = 0; q < G; ++q) sc[q] = 0;
-        double val[G][V];
-#define PHYLO_MFMA_SHAPE(LK, RK)                                                                                     \
-    mfma_shape<LK, RK, T, C, V, G, TL>(op, cat, s, sg0, n_sg, lane, g, m_pad, S, full, tips, tl, clv, slot_stride, \
-                                       scl, Pm, PTm, cA, sA, cB, sB, val, sc)
-        if (op.flags & OP_SH_AT) PHYLO_MFMA_SHAPE(SRC_CARRY_A, SRC_TIP);
-        else if (op.flags & OP_SH_TT) PHYLO_MFMA_SHAPE(SRC_TIP, SRC_TIP);
-        else if (op.flags & OP_SH_AB) PHYLO_MFMA_SHAPE(SRC_CARRY_A, SRC_CARRY_B);
-        else if (op.flags & OP_SH_AC) PHYLO_MFMA_SHAPE(SRC_CARRY_A, SRC_CLV);
-        else {
-#undef PHYLO_MFMA_SHAPE
-            // the other shapes: one child at a time, kinds read at run time
-            mfma_d4 acc[G][2];
-            mfma_child<T, C, V, G, TL>(op.l_kind, op.l_idx, op.l_node, cat, s, sg0, n_sg, lane, g, m_pad, S, full,
-                                       tips, tl, clv, slot_stride, scl, Pm, PTm, cA, sA, cB, sB, acc, sc);
-#pragma unroll
-            for (int q = 0; q < G; ++q)
-#pragma unroll
-                for (int t = 0; t < V; ++t) val[q][t] = acc[q][t / 4][t % 4];
-            if (op.r_kind != SRC_NONE) {
-                mfma_child<T, C, V, G, TL>(op.r_kind, op.r_idx, op.r_node, cat, s, sg0, n_sg, lane, g, m_pad, S,
-                                           full, tips, tl, clv, slot_stride, scl, Pm, PTm, cA, sA, cB, sB, acc, sc);
-#pragma unroll
-                for (int q = 0; q < G; ++q)
-#pragma unroll
-                    for (int t = 0; t < V; ++t) val[q][t] *= acc[q][t / 4][t % 4];
-            }
-        }
-        // Lazy rescale: only when a site's largest state falls below 2^-256
-        // (a site's states are spread over the lane groups, so its maximum
-        // takes two cross-lane steps; every lane holding part of such a site
-        // has its own largest state below the threshold, so those steps run
-        // only when some lane of the wave has).
-        bool low = false;
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            int h = __double2hiint(val[q][0]);     // the lane's largest state of the site, as a high word
-#pragma unroll
-            for (int t = 1; t < V; ++t) h = max(h, __double2hiint(val[q][t]));
-            low |= h < kLazyRescaleHi;
-        }
-        if (__builtin_amdgcn_ballot_w64(low) != 0) {
-#pragma unroll
-            for (int q = 0; q < G; ++q) {
-                const int e = site_exponent<V>(val[q]);
-                const double mx = site_max<V>(val[q]);
-                if (mx < 0x1p-256) {
-                    sc[q] += e;
-#pragma unroll
-                    for (int t = 0; t < V; ++t) val[q][t] = ldexp(val[q][t], -e);
-                }
-            }
-        }
-#pragma unroll
-        for (int q = 0; q < G; ++q) {
-            if (op.out_slot >= 0) {
-                // stored: brought to [0.5, 1) with its own scaler, then rounded
-                // to T with per-state random bits
-                const int e = site_exponent<V>(val[q]);
-                const uint32_t key = round_key(s[q], op, cat) + 0x9e3779b9u * (8u * (uint32_t)g);
-                T* dst = clv + (size_t)op.out_slot * slot_stride + ((size_t)cat * n_sg + sg0 + q) * V * 64 + lane;
-#pragma unroll
-                for (int t = 0; t < V; ++t)
-                    dst[t * 64] = (T)round_cut(ldexp(val[q][t], -e), key + 0x9e3779b9u * t, T());
-                if (g == 0) scl[((size_t)op.out_slot * C + cat) * m_pad + s[q]] = sc[q] + e;
-            }
-            if (op.flags & OP_TO_B) {
-#pragma unroll
-                for (int t = 0; t < V; ++t) cB[(q * V + t) * 64] = val[q][t];
-                sB[q] = sc[q];
-            } else {
-#pragma unroll
-                for (int t = 0; t < V; ++t) cA[q][t] = val[q][t];
-                sA[q] = sc[q];
-            }
-        }
-        if (op.flags & OP_ROOT) {
-            double lc[G];
-#pragma unroll
-            for (int q = 0; q < G; ++q) {
-                // the root partial brought to [0.5, 1) first (as in walk4)
-                const int e = site_exponent<V>(val[q]);
-                sc[q] += e;
-#pragma unroll
-                for (int t = 0; t < V; ++t) val[q][t] = ldexp(val[q][t], -e);
-                lc[q] = 0.0;
-#pragma unroll
-                for (int t = 0; t < V; ++t) lc[q] = fma(roots[4 * t + g], val[q][t], lc[q]);
-                lc[q] += __shfl_xor(lc[q], 16, 64);
-                lc[q] += __shfl_xor(lc[q], 32, 64);
-                lc[q] *= roots[kRootCatOff + cat];
-            }
-            if (C > 1) {
-                // the categories' sums at their largest exponent
-                if (g == 0) {
-#pragma unroll
-                    for (int q = 0; q < G; ++q) {
-                        xroot[cat][16 * q + j] = lc[q];
-                        xsc[cat][16 * q + j] = sc[q];
-                    }
-                }
-                __syncthreads();
-#pragma unroll
-                for (int q = 0; q < G; ++q) {
-                    int M = xsc[0][16 * q + j];
-#pragma unroll
-                    for (int c = 1; c < C; ++c) M = max(M, xsc[c][16 * q + j]);
-                    lc[q] = 0.0;
-#pragma unroll
-                    for (int c = 0; c < C; ++c) lc[q] += ldexp(xroot[c][16 * q + j], xsc[c][16 * q + j] - M);
-                    sc[q] = M;
-                }
-                __syncthreads();
-            }
-#pragma unroll
-            for (int q = 0; q < G; ++q) lnl[q] = log(lc[q]) + sc[q] * kLn2;
-        }
-    }
-    if (!has_root) return;    // a piece: its stores are its result (uniform per workgroup)
-    double sum = 0.0;
-#pragma unroll
-    for (int q = 0; q < G; ++q) {
-        const bool live = s[q] < m && cat == 0 && g == 0;
-        if (live && site_lnl) site_lnl[(size_t)(MP ? p : y) * m + s[q]] = lnl[q];
-        if (live) sum += (site_w ? site_w[s[q]] : 1.0) * lnl[q];
-    }
-    if constexpr (MP) {
-        // only the category-0 wave holds site values: its sum is the block's
-        if (cat == 0) {
-            const double v = wave_sum(sum);
-            if (lane == 0) partial[(size_t)p * n_main + bx] = v;
-        }
-    } else {
-        block_sum_store(sum, partial + (prog_main >= 0 ? (size_t)bx : (size_t)y * gridDim.x + blockIdx.x));
-        if (64 * C == kSumThreads && fold_counter) fold_total(partial, blk0 + n_main, fold_counter, fold_out);
-    }
-    } while (MP && ++p < p_end);
-}
-
-template <typename T, int C, int V, int G, bool TL>
-__global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_kernel(
-    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
-    int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
-    const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
-    int S, uint32_t full, int n_taxa, int n_main, int prog_main, int blk0, int prog_piece, int tail0, int n_tail,
-    unsigned* fold_counter, double* fold_out) {
-    prune_mfma_walk<T, C, V, G, TL, false>(ops, prog_begin, tips, clv, scl, Pm, PTm, roots, site_w, site_lnl, partial, m, m_pad, S, full,
-                                          n_taxa, n_main, prog_main, blk0, prog_piece, tail0, n_tail, fold_counter,
-                                          fold_out);
-}
-
-// An NNI neighbourhood's programs, program-major and grouped by XCD
-// (prune_mfma_walk's MP launch).
-template <typename T, int C, int V, int G>
-__global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_nni_kernel(
-    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
-    int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
-    const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
-    int S, uint32_t full, int n_taxa, int n_main, int prog_main, int blk0, int prog_piece, int tail0, int n_tail,
-    unsigned* fold_counter, double* fold_out) {
-    prune_mfma_walk<T, C, V, G, false, true>(ops, prog_begin, tips, clv, scl, Pm, PTm, roots, site_w, site_lnl, partial, m, m_pad, S, full,
-                                          n_taxa, n_main, prog_main, blk0, prog_piece, tail0, n_tail, fold_counter,
-                                          fold_out);
 }
 
 // Compensated fixed-order sum of the per-workgroup partials of each program
@@ -1505,8 +640,18 @@ struct phylo_ctx {
     double* d_P = nullptr; size_t P_bytes = 0;
     Op* d_ops = nullptr; size_t ops_bytes = 0;
     int* d_prog = nullptr; size_t prog_bytes = 0;
-    Op* d_nni_ops = nullptr; size_t nni_ops_bytes = 0;   // NNI partial-recompute programs
+    Op* d_nni_ops = nullptr; size_t nni_ops_bytes = 0;   // NNI partial-recompute programs (wide alphabets)
     int* d_nni_prog = nullptr; size_t nni_prog_bytes = 0;
+    // NNI walks of the current topology (nni_program.h), rebuilt when it changes
+    struct NniWalks {
+        int mode = -1;                                    // -1: none built
+        std::vector<int> node, side, which;               // variants; variant of each output
+        int n_prog = 0;
+        long path_ops = 0;
+        NniOp* d_ops = nullptr; size_t ops_bytes = 0;
+        int* d_prog = nullptr; size_t prog_bytes = 0;
+        double2* d_part = nullptr; size_t part_bytes = 0;
+    } walks;
     const Op* run_ops = nullptr;                          // program set of the launch in flight
     const int* run_prog = nullptr;
     bool run_whole_tree = false;                          // the launch in flight walks every internal node
@@ -1874,37 +1019,20 @@ int resident_dna(const phylo_ctx* c) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prune4_kernel<T, C, true>, 64 * C,
                                                         tip_lds_bytes(c->n_taxa)) == hipSuccess ? n : 0;
 }
-template <typename T, int C, int V>
-int resident_wide(const phylo_ctx*) {
-    int n = 0;
-    return hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, prune_mfma_kernel<T, C, V, kMfmaGroups, true>, 64 * C, 0) ==
-                   hipSuccess ? n : 0;
-}
-template <typename T, int C>
-int resident_wide_v(const phylo_ctx* c) {
-    switch (mfma_slots(c->S)) {
-    case 2: return resident_wide<T, C, 2>(c);
-    case 3: return resident_wide<T, C, 3>(c);
-    case 4: return resident_wide<T, C, 4>(c);
-    case 5: return resident_wide<T, C, 5>(c);
-    case 6: return resident_wide<T, C, 6>(c);
-    case 7: return resident_wide<T, C, 7>(c);
-    default: return resident_wide<T, C, 8>(c);
-    }
-}
 template <typename T>
-int resident_per_cu_t(const phylo_ctx* c) {
-    const bool wide = c->S > 4;
+int resident_dna_c(const phylo_ctx* c) {
     switch (c->C) {
-    case 1: return wide ? resident_wide_v<T, 1>(c) : resident_dna<T, 1>(c);
-    case 2: return wide ? resident_wide_v<T, 2>(c) : resident_dna<T, 2>(c);
-    case 4: return wide ? resident_wide_v<T, 4>(c) : resident_dna<T, 4>(c);
-    case 8: return wide ? resident_wide_v<T, 8>(c) : resident_dna<T, 8>(c);
+    case 1: return resident_dna<T, 1>(c);
+    case 2: return resident_dna<T, 2>(c);
+    case 4: return resident_dna<T, 4>(c);
+    case 8: return resident_dna<T, 8>(c);
     default: return 0;
     }
 }
 int resident_per_cu(const phylo_ctx* c) {
-    return c->prec == PHYLO_PREC_FP64 ? resident_per_cu_t<double>(c) : resident_per_cu_t<float>(c);
+    const bool f64 = c->prec == PHYLO_PREC_FP64;
+    if (uses_mfma(c)) return mfma_resident(f64, c->C, c->S);
+    return f64 ? resident_dna_c<double>(c) : resident_dna_c<float>(c);
 }
 
 int compile_full_program(phylo_ctx* c) {
@@ -1992,16 +1120,10 @@ int upload_pmatrices(phylo_ctx* c) {
     }
     if (Sp > 4) {
         const int V = mfma_slots(c->S_model), TN = V > 4 ? 2 : 1;
-        const long nPm = (long)c->n_nodes * c->C * TN * V * 64;
-        HIPCHK(c, ensure(c->d_Pm, c->Pm_bytes, (size_t)nPm * sizeof(double)));
-        hipLaunchKernelGGL(pmfma_kernel, dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, c->stream, c->d_P,
-                           c->S_model, Sp, c->C, c->n_nodes, V, TN, c->d_Pm);
-        HIPCHK(c, hipGetLastError());
-        const long nPT = (long)c->n_nodes * c->C * (c->S_model + 1) * 4 * V;
-        HIPCHK(c, ensure(c->d_PTm, c->PTm_bytes, (size_t)nPT * sizeof(double)));
-        hipLaunchKernelGGL(ptm_kernel, dim3((unsigned)((nPT + 255) / 256)), dim3(256), 0, c->stream, c->d_P,
-                           c->S_model, Sp, c->C, c->n_nodes, 4 * V, c->d_PTm);
-        HIPCHK(c, hipGetLastError());
+        const size_t nPm = (size_t)c->n_nodes * c->C * TN * V * 64, nPT = (size_t)c->n_nodes * c->C * (c->S_model + 1) * 4 * V;
+        HIPCHK(c, ensure(c->d_Pm, c->Pm_bytes, nPm * sizeof(double)));
+        HIPCHK(c, ensure(c->d_PTm, c->PTm_bytes, nPT * sizeof(double)));
+        HIPCHK(c, mfma_operands(c->d_P, c->S_model, Sp, c->C, c->n_nodes, c->d_Pm, c->d_PTm, c->stream));
     }
     c->dirty_P = false;
     return PHYLO_OK;
@@ -2053,6 +1175,7 @@ int prepare(phylo_ctx* c) {
         HIPCHK(c, hipMemcpyAsync(c->d_prog, c->prog_begin.data(), c->prog_begin.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));
         c->dirty_topo = false;
+        c->walks.mode = -1;
     }
     const size_t elt = c->prec == PHYLO_PREC_FP64 ? sizeof(double) : sizeof(float);
     HIPCHK(c, ensure(c->d_clv, c->clv_bytes,
@@ -2093,8 +1216,6 @@ void launch_prune4(phylo_ctx* c, dim3 grid, double* site_lnl) {
     const auto* tips = reinterpret_cast<const uint8_t*>(c->d_tips);
     T* clv = reinterpret_cast<T*>(c->d_clv);
     const double* sw = c->have_site_w ? c->d_sitew : nullptr;
-    // staging every tip pays off for whole-tree walks, not for the short
-    // path-to-root programs of an NNI neighbourhood
     if (c->run_whole_tree && c->n_taxa <= kTipLdsTaxa) {
         const int nblk = (int)grid.x;
         const int main_b = split_main_blocks(c, nblk), tail = nblk - main_b;
@@ -2118,17 +1239,6 @@ void launch_prune4(phylo_ctx* c, dim3 grid, double* site_lnl) {
                                tips, clv, c->d_scl, c->d_P, c->d_roots, sw, site_lnl, c->d_partial, c->m, c->m_pad,
                                c->n_taxa, (int)grid.x, -1, 0, 0, 0, 1, nullptr, nullptr);
         }
-    } else if (grid.y > 1) {
-        // many programs (an NNI neighbourhood): program-major, grouped by
-        // XCD, four programs a workgroup while that leaves 8 workgroups per CU
-        const int nblk = (int)grid.x, n_prog = (int)grid.y, nb8 = (nblk + 7) / 8 * 8;
-        const long fill = 8L * (c->n_cu > 0 ? c->n_cu : 256);
-        int ppw = 4;
-        while (ppw > 1 && (long)nb8 * ((n_prog + ppw - 1) / ppw) < fill) ppw /= 2;
-        const int n_pg = (n_prog + ppw - 1) / ppw;
-        hipLaunchKernelGGL((prune4_kernel<T, C, false>), dim3(nb8 * n_pg), dim3(64 * C), 0,
-                           c->stream, c->run_ops, c->run_prog, tips, clv, c->d_scl, c->d_P, c->d_roots, sw, site_lnl,
-                           c->d_partial, c->m, c->m_pad, c->n_taxa, nblk, -2, ppw, 0, 0, n_prog, nullptr, nullptr);
     } else {
         hipLaunchKernelGGL((prune4_kernel<T, C, false>), grid, dim3(64 * C), 0, c->stream, c->run_ops, c->run_prog,
                            tips, clv, c->d_scl, c->d_P, c->d_roots, sw, site_lnl, c->d_partial, c->m, c->m_pad,
@@ -2149,78 +1259,77 @@ int dispatch_prune4(phylo_ctx* c, dim3 grid, double* site_lnl) {
 }
 
 
-template <typename T, int C, int V>
-void launch_mfma(phylo_ctx* c, dim3 grid, double* site_lnl) {
-    const auto* tips = reinterpret_cast<const uint32_t*>(c->d_tips);
-    T* clv = reinterpret_cast<T*>(c->d_clv);
-    const double* sw = c->have_site_w ? c->d_sitew : nullptr;
-    const uint32_t full = c->S == 32 ? 0xFFFFFFFFu : ((1u << c->S) - 1u);
+int dispatch_mfma(phylo_ctx* c, dim3 grid, double* site_lnl) {
+    if (c->C != 1 && c->C != 2 && c->C != 4 && c->C != 8)
+        return fail(c, PHYLO_ERR_UNSUPPORTED, "number of rate categories must be 1, 2, 4 or 8");
+    MfmaArgs a;
+    a.f64 = c->prec == PHYLO_PREC_FP64;
+    a.C = c->C;
+    a.S = c->S;
+    a.ops = c->run_ops;
+    a.prog = c->run_prog;
+    a.tips = static_cast<const uint32_t*>(c->d_tips);
+    a.clv = c->d_clv;
+    a.scl = c->d_scl;
+    a.Pm = c->d_Pm;
+    a.PTm = c->d_PTm;
+    a.roots = c->d_roots;
+    a.site_w = c->have_site_w ? c->d_sitew : nullptr;
+    a.site_lnl = site_lnl;
+    a.partial = c->d_partial;
+    a.m = c->m;
+    a.m_pad = c->m_pad;
+    a.n_taxa = c->n_taxa;
+    a.grid = grid;
+    a.n_main = (int)grid.x;
+    const int nblk = (int)grid.x;
     if (c->run_whole_tree && c->n_taxa <= kMfmaTipLdsTaxa) {
-        const int nblk = (int)grid.x;
         const int main_b = split_main_blocks(c, nblk), tail = nblk - main_b;
+        a.tip_lds = true;
         if (c->tail_split && c->split_K > 0 && grid.y == 1 && tail > 0) {
-            // the main blocks and the tail's pieces, then the tail's top program
+            // the main blocks and the tail's pieces, then the tail's top
+            // program (which reads a few tips: no LDS staging)
             const int base = c->split_base[c->run_full ? 0 : 1], K = c->split_K;
-            hipLaunchKernelGGL((prune_mfma_kernel<T, C, V, kMfmaGroups, true>), dim3(main_b + K * tail), dim3(64 * C),
-                               0, c->stream, c->run_ops, c->d_prog, tips, clv, c->d_scl, c->d_Pm, c->d_PTm,
-                               c->d_roots, sw, site_lnl, c->d_partial, c->m, c->m_pad, c->S, full, c->n_taxa, main_b,
-                               c->run_full ? 0 : 1, 0, base, main_b, tail, nullptr, nullptr);
-            // (the top program reads a few tips: no LDS staging)
-            unsigned* fold = 64 * C == kSumThreads ? c->d_fold : nullptr;
-            hipLaunchKernelGGL((prune_mfma_kernel<T, C, V, kMfmaGroups, false>), dim3(tail), dim3(64 * C), 0,
-                               c->stream, c->run_ops, c->d_prog, tips, clv, c->d_scl, c->d_Pm, c->d_PTm, c->d_roots,
-                               sw, site_lnl, c->d_partial, c->m, c->m_pad, c->S, full, c->n_taxa, tail, base + K,
-                               main_b, 0, 0, 1, fold, c->h_total_dev);
-            c->folded = fold != nullptr;
-        } else {
-            hipLaunchKernelGGL((prune_mfma_kernel<T, C, V, kMfmaGroups, true>), grid, dim3(64 * C), 0, c->stream,
-                               c->run_ops, c->run_prog, tips, clv, c->d_scl, c->d_Pm, c->d_PTm, c->d_roots, sw,
-                               site_lnl, c->d_partial, c->m, c->m_pad, c->S, full, c->n_taxa, (int)grid.x, -1, 0, 0, 0,
-                               1, nullptr, nullptr);
+            a.prog = c->d_prog;
+            a.grid = dim3(main_b + K * tail);
+            a.n_main = main_b;
+            a.prog_main = c->run_full ? 0 : 1;
+            a.prog_piece = base;
+            a.tail0 = main_b;
+            a.n_tail = tail;
+            HIPCHK(c, mfma_launch(a, c->stream));
+            a.tip_lds = false;
+            a.grid = dim3(tail);
+            a.n_main = tail;
+            a.prog_main = base + K;
+            a.blk0 = main_b;
+            a.prog_piece = a.tail0 = 0;
+            a.n_tail = 1;
+            a.fold = 64 * c->C == kSumThreads ? c->d_fold : nullptr;
+            a.fold_out = c->h_total_dev;
+            c->folded = a.fold != nullptr;
         }
     } else if (grid.y > 1) {
-        // many programs (an NNI neighbourhood): program-major, grouped by XCD,
-        // as in launch_prune4, but one program a workgroup: these ops are
-        // long enough that fewer, longer workgroups do not pay (one, two,
-        // four programs: 2.976, 2.997, 3.014 ms for a 122-variant
-        // neighbourhood of 64 taxa x 20,000 sites)
-        const int nblk = (int)grid.x, n_prog = (int)grid.y, nb8 = (nblk + 7) / 8 * 8;
-        const int ppw = 1, n_pg = n_prog;
-        hipLaunchKernelGGL((prune_mfma_nni_kernel<T, C, V, kMfmaGroups>), dim3(nb8 * n_pg), dim3(64 * C), 0,
-                           c->stream, c->run_ops, c->run_prog, tips, clv, c->d_scl, c->d_Pm, c->d_PTm, c->d_roots, sw,
-                           site_lnl, c->d_partial, c->m, c->m_pad, c->S, full, c->n_taxa, nblk, -2, ppw, 0, 0, n_prog,
-                           nullptr, nullptr);
-    } else {
-        hipLaunchKernelGGL((prune_mfma_kernel<T, C, V, kMfmaGroups, false>), grid, dim3(64 * C), 0, c->stream,
-                           c->run_ops, c->run_prog, tips, clv, c->d_scl, c->d_Pm, c->d_PTm, c->d_roots, sw, site_lnl,
-                           c->d_partial, c->m, c->m_pad, c->S, full, c->n_taxa, (int)grid.x, -1, 0, 0, 0, 1, nullptr,
-                           nullptr);
+        // an NNI neighbourhood: program-major, grouped by XCD (1-D grid)
+        a.prog_main = -2;
+        a.n_tail = (int)grid.y;
+        a.blk0 = 1;
+        a.grid = dim3((nblk + 7) / 8 * 8 * grid.y);
     }
-}
-
-template <typename T, int C>
-int dispatch_mfma_v(phylo_ctx* c, dim3 grid, double* site_lnl) {
-    switch (mfma_slots(c->S)) {
-    case 2: launch_mfma<T, C, 2>(c, grid, site_lnl); break;
-    case 3: launch_mfma<T, C, 3>(c, grid, site_lnl); break;
-    case 4: launch_mfma<T, C, 4>(c, grid, site_lnl); break;
-    case 5: launch_mfma<T, C, 5>(c, grid, site_lnl); break;
-    case 6: launch_mfma<T, C, 6>(c, grid, site_lnl); break;
-    case 7: launch_mfma<T, C, 7>(c, grid, site_lnl); break;
-    default: launch_mfma<T, C, 8>(c, grid, site_lnl); break;
-    }
+    HIPCHK(c, mfma_launch(a, c->stream));
     return PHYLO_OK;
 }
 
-template <typename T>
-int dispatch_mfma(phylo_ctx* c, dim3 grid, double* site_lnl) {
-    switch (c->C) {
-    case 1: return dispatch_mfma_v<T, 1>(c, grid, site_lnl);
-    case 2: return dispatch_mfma_v<T, 2>(c, grid, site_lnl);
-    case 4: return dispatch_mfma_v<T, 4>(c, grid, site_lnl);
-    case 8: return dispatch_mfma_v<T, 8>(c, grid, site_lnl);
-    default: return fail(c, PHYLO_ERR_UNSUPPORTED, "number of rate categories must be 1, 2, 4 or 8");
-    }
+// Mapped pinned memory for n totals.
+int ensure_totals(phylo_ctx* c, size_t n) {
+    if (c->h_total_bytes >= n * sizeof(double)) return PHYLO_OK;
+    if (c->h_total) HIPCHK(c, hipHostFree(c->h_total));
+    c->h_total = nullptr;
+    c->h_total_bytes = 0;
+    HIPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_total), n * sizeof(double), hipHostMallocMapped));
+    HIPCHK(c, hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_total_dev), c->h_total, 0));
+    c->h_total_bytes = n * sizeof(double);
+    return PHYLO_OK;
 }
 
 // Launches the program set currently in c->ops / c->prog_begin and returns
@@ -2233,14 +1342,7 @@ int run_programs(phylo_ctx* c, const Op* d_ops, const int* d_prog, int n_prog, d
     const int nblk = c->m_pad / (mfma ? 16 * kMfmaGroups : 64);
     HIPCHK(c, ensure(c->d_partial, c->partial_bytes, (size_t)n_prog * nblk * sizeof(double)));
     if (site_lnl_host) HIPCHK(c, ensure(c->d_sitelnl, c->sitelnl_bytes, (size_t)n_prog * c->m * sizeof(double)));
-    if (c->h_total_bytes < (size_t)n_prog * sizeof(double)) {
-        if (c->h_total) HIPCHK(c, hipHostFree(c->h_total));
-        c->h_total = nullptr;
-        HIPCHK(c, hipHostMalloc(reinterpret_cast<void**>(&c->h_total), (size_t)n_prog * sizeof(double),
-                                hipHostMallocMapped));
-        HIPCHK(c, hipHostGetDevicePointer(reinterpret_cast<void**>(&c->h_total_dev), c->h_total, 0));
-        c->h_total_bytes = (size_t)n_prog * sizeof(double);
-    }
+    if (int rc = ensure_totals(c, n_prog)) return rc;
     dim3 grid(nblk, n_prog);
     double* dsite = site_lnl_host ? c->d_sitelnl : nullptr;
     if (!c->d_fold) {
@@ -2256,7 +1358,7 @@ int run_programs(phylo_ctx* c, const Op* d_ops, const int* d_prog, int n_prog, d
     if (c->S <= 4)
         rc = c->prec == PHYLO_PREC_FP64 ? dispatch_prune4<double>(c, grid, dsite) : dispatch_prune4<float>(c, grid, dsite);
     else
-        rc = c->prec == PHYLO_PREC_FP64 ? dispatch_mfma<double>(c, grid, dsite) : dispatch_mfma<float>(c, grid, dsite);
+        rc = dispatch_mfma(c, grid, dsite);
     if (rc) return rc;
     HIPCHK(c, hipGetLastError());
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
@@ -2410,6 +1512,48 @@ bool append_nni_program(const TV* c, const std::vector<int>& par, int v, int sid
     return true;
 }
 
+// The node an interchange at v moves out of v's surroundings: v's sibling or,
+// at a child of the root, the sibling's left child; -1 where there is none
+// (the variant is the tree itself).
+template <class TV>
+int nni_partner(const TV* c, const std::vector<int>& par, int v) {
+    if (v < 0 || v == c->root || c->left[v] < 0) return -1;
+    const int p = par[v], sib = c->left[p] == v ? c->right[p] : c->left[p];
+    if (p != c->root) return sib;
+    return sib >= 0 ? c->left[sib] : -1;
+}
+
+// Ops a program that recomputes one variant's path to the root would run
+// (the update count reported for a neighbourhood).
+template <class TV>
+long nni_path_ops(const TV* c, const std::vector<int>& par, int v) {
+    if (par[v] == c->root) return 3;
+    long n = 2;
+    for (int u = par[v]; u != c->root; u = par[u]) ++n;
+    return n;
+}
+
+// Enumerates a neighbourhood and builds its walks (nni_program.h): node / side of
+// every variant in `node` / `side`, the variant of each scored output in
+// `which` (both sides of an edge are scored or neither is).
+template <class TV>
+void build_nni(const TV* c, int mode, int max_edges, std::vector<int>& node, std::vector<int>& side,
+               std::vector<int>& which, long& path_ops, std::vector<NniOp>& ops, std::vector<int>& begin) {
+    enumerate_nni(c, mode, node, side);
+    const std::vector<int> par = parents_of(c);
+    std::vector<int> pair_of(c->n_nodes, -1);
+    which.clear();
+    path_ops = 0;
+    for (size_t k = 0; k + 1 < node.size(); k += 2) {
+        if (nni_partner(c, par, node[k]) < 0) continue;
+        pair_of[node[k]] = (int)which.size();
+        which.push_back((int)k);
+        which.push_back((int)k + 1);
+        path_ops += 2 * nni_path_ops(c, par, node[k]);
+    }
+    if (!which.empty()) build_nni_walks(c, pair_of, max_edges, ops, begin);
+}
+
 // Checks a rooted topology over n_taxa tips (nodes 0..n_taxa-1, no children)
 // and internal nodes n_taxa..n_nodes-1: one or two valid children each, every
 // node but the root with exactly one parent.  Returns the reason, or nullptr.
@@ -2467,7 +1611,7 @@ void phylo_destroy(phylo_ctx* c) {
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     void* bufs[] = {c->d_tips, c->d_Pm, c->d_PTm, c->d_clv, c->d_scl, c->d_P, c->d_ops, c->d_prog, c->d_nni_ops, c->d_nni_prog,
                     c->d_roots, c->d_sitew,
-                    c->d_sitelnl, c->d_partial, c->d_eig, c->d_fold};
+                    c->d_sitelnl, c->d_partial, c->d_eig, c->d_fold, c->walks.d_ops, c->walks.d_prog, c->walks.d_part};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_total) (void)hipHostFree(c->h_total);
@@ -2724,6 +1868,78 @@ int phylo_get_pmatrix(phylo_ctx* c, int node, double* P) {
     return PHYLO_OK;
 }
 
+namespace {
+
+// The DNA neighbourhood: every variant by the outer-partial walks, against
+// the stored partials of an evaluation that kept them all.
+int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* lnl, int32_t* node, int32_t* side,
+                int* n_variants, double* base_lnl) {
+    auto& w = c->walks;
+    const int nblk = c->m_pad / 64;
+    if (w.mode != mode) {
+        w.mode = -1;
+        std::vector<NniOp> ops;
+        std::vector<int> begin{0};
+        build_nni(c, mode, nni_segment_edges((double)(c->n_nodes - c->n_taxa) * nblk, c->n_cu), w.node, w.side, w.which,
+                  w.path_ops, ops, begin);
+        w.n_prog = (int)begin.size() - 1;
+        if (w.n_prog > 0) {
+            ops.push_back(NniOp{});     // the walks read the op after the one they run
+            HIPCHK(c, ensure(w.d_ops, w.ops_bytes, ops.size() * sizeof(NniOp)));
+            HIPCHK(c, hipMemcpyAsync(w.d_ops, ops.data(), ops.size() * sizeof(NniOp), hipMemcpyHostToDevice, c->stream));
+            HIPCHK(c, ensure(w.d_prog, w.prog_bytes, begin.size() * sizeof(int)));
+            HIPCHK(c, hipMemcpyAsync(w.d_prog, begin.data(), begin.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+        }
+        w.mode = mode;
+    }
+    const int nv = (int)w.node.size(), n_out = (int)w.which.size();
+    *n_variants = nv;
+    if (base_lnl) *base_lnl = base;
+    if (nv == 0 || !lnl) return PHYLO_OK;   // count query
+    if (max_variants < nv) return fail(c, PHYLO_ERR_ARG, "nni_score: output arrays too small");
+    for (int k = 0; k < nv; ++k) {
+        lnl[k] = base;   // no-op interchanges keep the base tree
+        if (node) node[k] = w.node[k];
+        if (side) side[k] = w.side[k];
+    }
+    if (n_out == 0) return PHYLO_OK;
+    HIPCHK(c, ensure(w.d_part, w.part_bytes, (size_t)nblk * n_out * sizeof(double2)));
+    if (int rc = ensure_totals(c, n_out)) return rc;
+    NniArgs a;
+    a.f64 = c->prec == PHYLO_PREC_FP64;
+    a.C = c->C;
+    a.ops = w.d_ops;
+    a.prog = w.d_prog;
+    a.tips = static_cast<const uint8_t*>(c->d_tips);
+    a.clv = c->d_clv;
+    a.scl = c->d_scl;
+    a.P = c->d_P;
+    a.roots = c->d_roots;
+    a.site_w = c->have_site_w ? c->d_sitew : nullptr;
+    a.part = w.d_part;
+    a.one.m = c->m;
+    a.one.m_pad = c->m_pad;
+    a.one.n_taxa = a.max_taxa = c->n_taxa;
+    a.one.n_var = n_out;
+    a.one.nblk = nblk;
+    a.n_prog = w.n_prog;
+    HIPCHK(c, hipEventRecord(c->ev0, c->stream));
+    HIPCHK(c, nni4_launch(a, c->stream));
+    HIPCHK(c, hipEventRecord(c->ev1, c->stream));
+    HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr,
+                             (n_out + kNniSumVars - 1) / kNniSumVars, c->h_total_dev, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    float ms = 0.f;
+    HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
+    c->last_ms = ms;
+    for (int q = 0; q < n_out; ++q) lnl[w.which[q]] = c->h_total[q];
+    c->nni_ops_last = w.path_ops;
+    return PHYLO_OK;
+}
+
+}  // namespace
+
 int phylo_nni_score(phylo_ctx* c, int mode, int max_variants, double* lnl, int32_t* node, int32_t* side,
                     int* n_variants, double* base_lnl) {
     if (!c || !n_variants) return PHYLO_ERR_ARG;
@@ -2736,6 +1952,7 @@ int phylo_nni_score(phylo_ctx* c, int mode, int max_variants, double* lnl, int32
         if (rc) return rc;
     }
     base = c->base_total;
+    if (!uses_mfma(c)) return score_walks(c, mode, max_variants, base, lnl, node, side, n_variants, base_lnl);
     std::vector<int> nodes, sides;
     enumerate_nni(c, mode, nodes, sides);
     const int nv = (int)nodes.size();

@@ -1,0 +1,44 @@
+// prune_mfma.h -- launches of the matrix-core pruning walker (4 < S <= 32).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+#include <type_traits>
+
+#include "prune_device.h"
+
+// Operand slots that cover S states, four a slot.
+__host__ __device__ constexpr int mfma_slots(int S) { return (S + 3) / 4; }
+
+// Taxa whose tip masks a wide-state workgroup stages in LDS.
+constexpr int kMfmaTipLdsTaxa = 128;
+
+struct MfmaArgs {
+    bool f64 = false;
+    int C = 1, S = 0;
+    const Op* ops = nullptr;
+    const int* prog = nullptr;
+    const uint32_t* tips = nullptr;
+    void* clv = nullptr;
+    int* scl = nullptr;
+    const double* Pm = nullptr;
+    const double* PTm = nullptr;
+    const double* roots = nullptr;
+    const double* site_w = nullptr;
+    double* site_lnl = nullptr;
+    double* partial = nullptr;
+    int m = 0, m_pad = 0, n_taxa = 0;
+    bool tip_lds = false;              // stage the tips (n_taxa <= kMfmaTipLdsTaxa)
+    dim3 grid;
+    // work mapping (prune_mfma_kernel)
+    int n_main = 0, prog_main = -1, blk0 = 0, prog_piece = 0, tail0 = 0, n_tail = 1;
+    unsigned* fold = nullptr;
+    double* fold_out = nullptr;
+};
+
+hipError_t mfma_launch(const MfmaArgs& a, hipStream_t st);
+// Workgroups of the staging walker that one CU holds at once, 0 if unknown.
+int mfma_resident(bool f64, int C, int S);
+// The walker's P operands and tip columns from P (pmfma_kernel, ptm_kernel).
+hipError_t mfma_operands(const double* P, int S, int Sp, int C, int n_nodes, double* Pm, double* PTm, hipStream_t st);
