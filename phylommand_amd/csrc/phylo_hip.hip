@@ -34,7 +34,6 @@
 #include <cstring>
 #include <mutex>
 #include <string>
-#include <unordered_map>
 #include <vector>
 
 #include "../../include/phylo_hip.h"
@@ -239,7 +238,7 @@ __device__ __forceinline__ void walk4_op(const Op op, const uint8_t* __restrict_
     sB = to_b ? sc : sB;
 }
 
-// PAIRS: two ops per loop turn (the whole-tree and NNI launches); without
+// PAIRS: two ops per loop turn (the whole-tree launches); without
 // it one op per turn, the result copied into carry A (the batch kernel,
 // where the second copy of the op body would cost it a resident wave).  The
 // values are the same either way.
@@ -408,7 +407,7 @@ __global__ __launch_bounds__(64 * C) void prune4_kernel(
     }
 }
 
-// Batched scoring: many independent problems (and their NNI programs) in one
+// Batched scoring: the whole trees of many independent problems in one
 // persistent launch.  Workgroup g takes work items (instance, program, block
 // of 64 sites) g, g + grid, g + 2*grid, ... of a list sorted by decreasing
 // cost; the loop counter is uniform, so every wave runs the same barriers and
@@ -432,7 +431,7 @@ struct WorkItem {
 // Category tiling CW: CW = C puts the C categories on the C waves of a
 // workgroup (they meet in LDS at the root); CW = 1 has one wave walk the
 // program once per category and combine the root sums in registers, with no
-// barrier at all (a better fit for short programs such as NNI variants).
+// barrier at all.
 template <typename T, int C, int CW>
 __global__ __launch_bounds__(64 * CW) void batch4_kernel(const WorkItem* __restrict__ items, int n_items,
                                                          const BatchInst* __restrict__ inst,
@@ -484,20 +483,15 @@ __global__ __launch_bounds__(64 * CW) void batch4_kernel(const WorkItem* __restr
     }
 }
 
-// Segmented compensated sums: out[k] = sum partial[seg[k] .. seg[k+1]).
-__global__ __launch_bounds__(64) void segment_sum_kernel(const double* __restrict__ partial,
-                                                        const int* __restrict__ seg, int n_seg,
-                                                        double* __restrict__ out) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n_seg) return;
-    double s = 0.0, comp = 0.0;
-    for (int i = seg[k]; i < seg[k + 1]; ++i) {
-        const double x = partial[i] - comp;
-        const double t = s + x;
-        comp = (t - s) - x;
-        s = t;
-    }
-    out[k] = s;
+// Segmented compensated sums: out[k] = sum partial[seg[k] .. seg[k+1]), one
+// workgroup a segment (one thread a segment took 20 us for 24 alignments, its
+// loads one after another).
+__global__ __launch_bounds__(kSumThreads) void segment_sum_kernel(const double* __restrict__ partial,
+                                                                 const int* __restrict__ seg,
+                                                                 double* __restrict__ out) {
+    const int k = blockIdx.x;
+    const double t = block_total(partial + seg[k], seg[k + 1] - seg[k]);
+    if (threadIdx.x == 0) out[k] = t;
 }
 
 // Compensated fixed-order sum of the per-workgroup partials of each program
@@ -2296,7 +2290,8 @@ struct phylo_batch {
         long tips_off = 0, clv_off = 0, scl_off = 0, P_off = 0;
         int roots_off = 0;
         int full_prog = -1;
-        std::vector<int> nni_prog, nni_node, nni_side;   // nni_prog[k] = -1: no-op variant
+        std::vector<int> nni_node, nni_side, nni_which;  // variants; those scored (the others keep the tree)
+        std::vector<int> walk;                           // its NNI walks
         long full_ops = 0, nni_ops = 0;
     };
     int device = 0;
@@ -2309,7 +2304,7 @@ struct phylo_batch {
     int cat_waves = 4;                // category tiling: C waves per workgroup, or 1
     int per_cu_cap = 0;               // resident workgroups per CU of the persistent grid (0: all that fit)
     int max_per_cu = 1;               // all that fit, for the current tiling
-    int blocks_per_item = 2, grid = 0, n_items1 = 0, n_items2 = 0, n_seg1 = 0, n_seg2 = 0, n_var = 0;
+    int blocks_per_item = 2, grid = 0, n_items1 = 0, n_seg1 = 0, n_var = 0;
     double updates1 = 0, updates2 = 0, last_ms = 0;
     std::vector<int> var_offsets;     // per instance into the flat variant list
     // device
@@ -2322,18 +2317,24 @@ struct phylo_batch {
     int* d_prog = nullptr;
     BatchInst* d_inst = nullptr;
     WorkItem* d_items1 = nullptr;
-    WorkItem* d_items2 = nullptr;
     double* d_partial = nullptr;
     int* d_seg1 = nullptr;
-    int* d_seg2 = nullptr;
+    // the NNI phase: walks, their (instance, block) items, sums
+    NniArgs nni;
+    NniOp* d_walk_ops = nullptr;
+    int* d_walk_prog = nullptr;
+    NniInst* d_walk_inst = nullptr;
+    NniItem* d_walk_items = nullptr;
+    NniSum* d_sums = nullptr;
+    double2* d_nni_part = nullptr;
+    int n_sums = 0, n_scored = 0;
     double* d_out = nullptr;
     double* h_out = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     // host copies used to build work lists
-    std::vector<WorkItem> items1, items2;
-    std::vector<int> seg1, seg2;
-    std::vector<int> var_prog_of;     // flat variant -> program (-1 = no-op)
+    std::vector<WorkItem> items1;
+    std::vector<int> seg1;
 };
 
 namespace {
@@ -2379,10 +2380,9 @@ int batch_grid(phylo_batch* b) {
     return PHYLO_OK;
 }
 
-int enqueue_batch_phase(phylo_batch* b, int phase, int bpi) {
-    const WorkItem* items = phase == 1 ? b->d_items1 : b->d_items2;
-    const int n = phase == 1 ? b->n_items1 : b->n_items2;
-    if (n == 0) return PHYLO_OK;
+int enqueue_batch_trees(phylo_batch* b, int bpi) {
+    const WorkItem* items = b->d_items1;
+    const int n = b->n_items1;
     const bool f64 = b->prec == PHYLO_PREC_FP64;
     switch (b->C) {
     case 1: f64 ? launch_batch<double, 1>(b, items, n, bpi) : launch_batch<float, 1>(b, items, n, bpi); break;
@@ -2399,9 +2399,8 @@ int enqueue_batch_phase(phylo_batch* b, int phase, int bpi) {
 // placed by segment.
 void build_work_lists(phylo_batch* b, int bpi, const std::vector<int>& prog_len) {
     struct Cand { long cost; WorkItem w; };
-    std::vector<Cand> c1, c2;
+    std::vector<Cand> c1;
     b->seg1.assign(1, 0);
-    b->seg2.assign(1, 0);
     int out = 0;
     for (size_t i = 0; i < b->inst.size(); ++i) {
         const auto& I = b->inst[i];
@@ -2412,66 +2411,45 @@ void build_work_lists(phylo_batch* b, int bpi, const std::vector<int>& prog_len)
         }
         b->seg1.push_back(out);
     }
-    const int base2 = out;
-    // a variant's blocks keep consecutive partial slots (its segment), but
-    // the list runs block by block over the variants, so that items of equal
-    // cost that run side by side are variants of one site block and share
-    // its stored partials in L2
+    std::stable_sort(c1.begin(), c1.end(), [](const Cand& x, const Cand& y) { return x.cost > y.cost; });
+    b->items1.clear();
+    for (auto& x : c1) b->items1.push_back(x.w);
+}
+
+// Items of the NNI phase: every walk over every site block of its instance,
+// in order of decreasing length.  Workgroup g runs on XCD g mod 8
+// (workgroups are dealt to the XCDs in turn); the walks of one (instance,
+// site block) are dealt to one XCD, in cost order there, so those running
+// side by side share the block's stored partials in that XCD's L2.
+std::vector<NniItem> build_walk_items(const phylo_batch* b, const std::vector<int>& begin) {
+    struct Cand { long cost; NniItem w; int xcd; };
+    std::vector<Cand> c;
+    int n_blk = 0;
     for (size_t i = 0; i < b->inst.size(); ++i) {
         const auto& I = b->inst[i];
-        const int nb = I.m_pad / 64, n_items = (nb + bpi - 1) / bpi;
-        std::vector<int> first;
-        for (int pg : I.nni_prog) {
-            if (pg < 0) continue;
-            first.push_back(out);
-            out += n_items;
-            b->seg2.push_back(out - base2);
-        }
-        for (int blk = 0, q = 0; blk < nb; blk += bpi, ++q) {
-            const int sites = std::min(bpi, nb - blk) * 64;
-            size_t v = 0;
-            for (int pg : I.nni_prog) {
-                if (pg < 0) continue;
-                c2.push_back({(long)prog_len[pg] * sites, {(int)i, pg, blk, first[v++] + q}});
-            }
-        }
+        if (I.walk.empty()) continue;
+        for (int blk = 0; blk < I.m_pad / 64; ++blk, ++n_blk)
+            for (int w : I.walk) c.push_back({begin[w + 1] - begin[w], {(int)i, w, blk, 0}, n_blk % 8});
     }
-    auto by_cost = [](const Cand& x, const Cand& y) { return x.cost > y.cost; };
-    std::stable_sort(c1.begin(), c1.end(), by_cost);
-    std::stable_sort(c2.begin(), c2.end(), by_cost);
-    b->items1.clear();
-    b->items2.clear();
-    for (auto& x : c1) b->items1.push_back(x.w);
-    // Workgroup g runs on XCD g mod 8 (workgroups are dealt to the XCDs in
-    // turn) and the grid is a multiple of 8, so item j runs on XCD j mod 8.
-    // The variants of one (alignment, site block) are dealt to one XCD, in
-    // cost order there, so those running side by side share the block's
-    // stored partials in that XCD's L2.
-    std::vector<std::vector<WorkItem>> q(8);
-    std::unordered_map<long, int> xcd_of;
-    for (const auto& x : c2) {
-        const long key = (long)x.w.inst << 32 | (unsigned)x.w.block;
-        const auto it = xcd_of.emplace(key, (int)(xcd_of.size() % 8)).first;
-        q[it->second].push_back(x.w);
-    }
+    std::stable_sort(c.begin(), c.end(), [](const Cand& x, const Cand& y) { return x.cost > y.cost; });
+    std::vector<std::vector<NniItem>> q(8);
+    for (const auto& x : c) q[x.xcd].push_back(x.w);
     size_t next[8] = {};
-    for (size_t j = 0; j < c2.size(); ++j) {
+    std::vector<NniItem> items;
+    for (size_t j = 0; j < c.size(); ++j) {
         int x = (int)(j % 8);
         if (next[x] == q[x].size()) {    // this XCD's share is done: take from the longest remaining
             for (int k = 0; k < 8; ++k)
                 if (q[k].size() - next[k] > q[x].size() - next[x]) x = k;
         }
-        b->items2.push_back(q[x][next[x]++]);
+        items.push_back(q[x][next[x]++]);
     }
-    for (auto& s : b->seg2) s += base2;
-    b->seg2.front() = base2;
+    return items;
 }
 
 int upload_work_lists(phylo_batch* b) {
     b->n_items1 = (int)b->items1.size();
-    b->n_items2 = (int)b->items2.size();
     b->n_seg1 = (int)b->seg1.size() - 1;
-    b->n_seg2 = (int)b->seg2.size() - 1;
     auto up = [&](auto*& dptr, const auto& vec) -> hipError_t {
         if (dptr) { hipError_t e = hipFree(dptr); if (e != hipSuccess) return e; dptr = nullptr; }
         hipError_t e = hipMalloc(reinterpret_cast<void**>(&dptr), std::max<size_t>(vec.size(), 1) * sizeof(vec[0]));
@@ -2480,29 +2458,26 @@ int upload_work_lists(phylo_batch* b) {
         return hipMemcpy(dptr, vec.data(), vec.size() * sizeof(vec[0]), hipMemcpyHostToDevice);
     };
     HIPCHK(b, up(b->d_items1, b->items1));
-    HIPCHK(b, up(b->d_items2, b->items2));
     HIPCHK(b, up(b->d_seg1, b->seg1));
-    HIPCHK(b, up(b->d_seg2, b->seg2));
     if (b->d_partial) HIPCHK(b, hipFree(b->d_partial));
     b->d_partial = nullptr;
-    HIPCHK(b, hipMalloc(&b->d_partial, std::max<size_t>(b->n_items1 + b->n_items2, 1) * sizeof(double)));
+    HIPCHK(b, hipMalloc(&b->d_partial, std::max<size_t>(b->n_items1, 1) * sizeof(double)));
     return PHYLO_OK;
 }
 
-// Enqueues one full batch run (both phases and the segment sums) on the stream.
+// Enqueues one full batch run (both phases and their sums) on the stream.
 int enqueue_batch_run(phylo_batch* b) {
-    int rc = enqueue_batch_phase(b, 1, b->blocks_per_item);
+    int rc = enqueue_batch_trees(b, b->blocks_per_item);
     if (rc) return rc;
-    rc = enqueue_batch_phase(b, 2, b->blocks_per_item);
-    if (rc) return rc;
-    if (b->n_seg1)
-        hipLaunchKernelGGL(segment_sum_kernel, dim3((b->n_seg1 + 63) / 64), dim3(64), 0, b->stream, b->d_partial,
-                           b->d_seg1, b->n_seg1, b->d_out);
-    if (b->n_seg2)
-        hipLaunchKernelGGL(segment_sum_kernel, dim3((b->n_seg2 + 63) / 64), dim3(64), 0, b->stream, b->d_partial,
-                           b->d_seg2, b->n_seg2, b->d_out + b->n_seg1);
+    if (b->n_sums) {
+        HIPCHK(b, nni4_launch(b->nni, b->stream));
+        HIPCHK(b, nni_sum_launch(b->d_nni_part, false, b->d_walk_inst, b->nni.one, b->d_sums, b->n_sums, b->d_out,
+                                 b->stream));
+    }
+    hipLaunchKernelGGL(segment_sum_kernel, dim3(b->n_seg1), dim3(kSumThreads), 0, b->stream, b->d_partial, b->d_seg1,
+                       b->d_out);
     HIPCHK(b, hipGetLastError());
-    HIPCHK(b, hipMemcpyAsync(b->h_out, b->d_out, (size_t)(b->n_seg1 + b->n_seg2) * sizeof(double),
+    HIPCHK(b, hipMemcpyAsync(b->h_out, b->d_out, (size_t)(b->n_seg1 + b->n_scored) * sizeof(double),
                              hipMemcpyDeviceToHost, b->stream));
     return PHYLO_OK;
 }
@@ -2612,7 +2587,19 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
     int roots_elems = 0;
     b->updates1 = b->updates2 = 0;
     b->var_offsets.assign(1, 0);
-    b->var_prog_of.clear();
+    double edge_blocks = 0.0;
+    for (const auto& I : b->inst)
+        if (I.nni_mode >= 0) edge_blocks += (double)(I.n_nodes - I.n_taxa) * (I.m_pad / 64);
+    hipDeviceProp_t prop;
+    HIPCHK(b, hipGetDeviceProperties(&prop, b->device));
+    const int max_edges = nni_segment_edges(edge_blocks, prop.multiProcessorCount);
+    std::vector<NniOp> walk_ops;
+    std::vector<int> walk_begin{0};
+    std::vector<NniInst> walk_inst;
+    std::vector<NniSum> sums;
+    long part_elems = 0;
+    b->n_scored = 0;
+    b->nni.max_taxa = 0;
     for (auto& I : b->inst) {
         I.tips_off = tips_bytes;
         tips_bytes += (long)I.n_taxa * I.m_pad;
@@ -2632,26 +2619,35 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
         prog_len.push_back((int)(ops.size() - before));
         I.full_ops = (long)(ops.size() - before);
         b->updates1 += (double)I.full_ops * I.m * b->C;
-        I.nni_prog.clear();
         I.nni_node.clear();
         I.nni_side.clear();
+        I.nni_which.clear();
+        I.walk.clear();
         I.nni_ops = 0;
+        NniInst w{};
+        w.tips_off = I.tips_off;
+        w.clv_off = I.clv_off;
+        w.scl_off = I.scl_off;
+        w.P_off = I.P_off;
+        w.roots_off = I.roots_off;
+        w.m = I.m;
+        w.m_pad = I.m_pad;
+        w.n_taxa = I.n_taxa;
+        w.nblk = I.m_pad / 64;
+        w.part_off = part_elems;
         if (I.nni_mode >= 0) {
-            const std::vector<int> par = parents_of(&I);
-            enumerate_nni(&I, I.nni_mode, I.nni_node, I.nni_side);
-            for (size_t k = 0; k < I.nni_node.size(); ++k) {
-                const size_t b0 = ops.size();
-                if (append_nni_program(&I, par, I.nni_node[k], I.nni_side[k], ops)) {
-                    I.nni_prog.push_back((int)prog_begin.size() - 1);
-                    prog_begin.push_back((int)ops.size());
-                    prog_len.push_back((int)(ops.size() - b0));
-                    I.nni_ops += (long)(ops.size() - b0);
-                } else {
-                    I.nni_prog.push_back(-1);
-                }
-            }
+            const int first = (int)walk_begin.size() - 1;
+            build_nni(&I, I.nni_mode, max_edges, I.nni_node, I.nni_side, I.nni_which, I.nni_ops, walk_ops, walk_begin);
+            for (int p = first; p + 1 < (int)walk_begin.size(); ++p) I.walk.push_back(p);
             b->updates2 += (double)I.nni_ops * I.m * b->C;
+            w.n_var = (int)I.nni_which.size();
+            for (int v = 0; v < w.n_var; v += kNniSumVars)
+                sums.push_back({(int)walk_inst.size(), v, (int)b->inst.size() + b->n_scored + v, 0});
+            b->n_scored += w.n_var;
+            part_elems += (long)w.n_var * w.nblk;
+            if (w.n_var) b->nni.max_taxa = std::max(b->nni.max_taxa, I.n_taxa);
         }
+        walk_inst.push_back(w);
         b->var_offsets.push_back(b->var_offsets.back() + (int)I.nni_node.size());
     }
     b->n_var = b->var_offsets.back();
@@ -2691,6 +2687,35 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
     order_children(ops);
     HIPCHK(b, hipMemcpy(b->d_ops, ops.data(), ops.size() * sizeof(Op), hipMemcpyHostToDevice));
     HIPCHK(b, hipMemcpy(b->d_prog, prog_begin.data(), prog_begin.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (!sums.empty()) {
+        walk_ops.push_back(NniOp{});     // the walks read the op after the one they run
+        const std::vector<NniItem> items = build_walk_items(b, walk_begin);
+        const auto up = [&](auto*& d, const auto& v) -> hipError_t {
+            hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), v.size() * sizeof(v[0]));
+            return e == hipSuccess ? hipMemcpy(d, v.data(), v.size() * sizeof(v[0]), hipMemcpyHostToDevice) : e;
+        };
+        HIPCHK(b, up(b->d_walk_ops, walk_ops));
+        HIPCHK(b, up(b->d_walk_prog, walk_begin));
+        HIPCHK(b, up(b->d_walk_inst, walk_inst));
+        HIPCHK(b, up(b->d_walk_items, items));
+        HIPCHK(b, up(b->d_sums, sums));
+        HIPCHK(b, hipMalloc(&b->d_nni_part, (size_t)part_elems * sizeof(double2)));
+        NniArgs& a = b->nni;
+        a.f64 = b->prec == PHYLO_PREC_FP64;
+        a.C = b->C;
+        a.ops = b->d_walk_ops;
+        a.prog = b->d_walk_prog;
+        a.tips = b->d_tips;
+        a.clv = b->d_clv;
+        a.scl = b->d_scl;
+        a.P = b->d_P;
+        a.roots = b->d_roots;
+        a.part = b->d_nni_part;
+        a.insts = b->d_walk_inst;
+        a.items = b->d_walk_items;
+        a.n_items = (int)items.size();
+        b->n_sums = (int)sums.size();
+    }
     const int n_out = (int)b->inst.size() + b->n_var;
     HIPCHK(b, hipMalloc(&b->d_out, std::max(n_out, 1) * sizeof(double)));
     HIPCHK(b, hipHostMalloc(reinterpret_cast<void**>(&b->h_out), std::max(n_out, 1) * sizeof(double)));
@@ -2717,8 +2742,9 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
         b->blocks_per_item = cfg.bpi;
         float ms = 0.f;
         for (int rep = 0; rep < (autotune ? 2 : 0); ++rep) {
+            // (the tiling is that of the whole-tree phase; the NNI walks have none)
             HIPCHK(b, hipEventRecord(b->ev0, b->stream));
-            rc = enqueue_batch_run(b);
+            rc = enqueue_batch_trees(b, cfg.bpi);
             if (rc) return rc;
             HIPCHK(b, hipEventRecord(b->ev1, b->stream));
             HIPCHK(b, hipStreamSynchronize(b->stream));
@@ -2739,8 +2765,8 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
         }
     }
     if (autotune) {
-        // fewer resident workgroups per CU: the NNI programs mostly read
-        // stored partials, and more waves in flight can thrash the caches
+        // fewer resident workgroups per CU: more waves in flight can thrash
+        // the caches with stored partials
         b->cat_waves = best_cfg.cw;
         int rc = batch_grid(b);
         if (rc) return rc;
@@ -2791,11 +2817,9 @@ int phylo_batch_run(phylo_batch* b, double* totals, double* nni_lnl) {
         int seg = 0;
         for (int i = 0; i < ni; ++i) {
             const auto& I = b->inst[i];
-            for (size_t k = 0; k < I.nni_prog.size(); ++k) {
-                double v = b->h_out[i];                  // no-op variants keep the base tree
-                if (I.nni_prog[k] >= 0) v = b->h_out[ni + seg++];
-                nni_lnl[b->var_offsets[i] + k] = v;
-            }
+            double* dst = nni_lnl + b->var_offsets[i];
+            std::fill(dst, dst + I.nni_node.size(), b->h_out[i]);     // no-op variants keep the base tree
+            for (int k : I.nni_which) dst[k] = b->h_out[ni + seg++];
         }
     }
     return PHYLO_OK;
@@ -2852,7 +2876,8 @@ void phylo_batch_destroy(phylo_batch* b) {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
     void* bufs[] = {b->d_tips, b->d_clv, b->d_scl, b->d_P, b->d_roots, b->d_ops, b->d_prog, b->d_inst,
-                    b->d_items1, b->d_items2, b->d_partial, b->d_seg1, b->d_seg2, b->d_out};
+                    b->d_items1, b->d_partial, b->d_seg1, b->d_out, b->d_walk_ops, b->d_walk_prog, b->d_walk_inst,
+                    b->d_walk_items, b->d_sums, b->d_nni_part};
     for (void* p : bufs)
         if (p) (void)hipFree(p);
     if (b->h_out) (void)hipHostFree(b->h_out);
