@@ -50,7 +50,8 @@ struct NniArgs {
 // Edges a walk should hold so that the launch has some 12 workgroups per CU
 // (site blocks x walks; 5 are resident): each segment repeats the walk from
 // the root to its start, so few segments move less memory (128 taxa x 100,000
-// sites: 64 edges a walk 0.538 ms, 32 0.585, 16 0.599), but a launch of few
+// sites: 64 edges a walk 0.538 ms, 32 0.585, 16 0.599; 6 to 18 workgroups
+// within 2 %), but a launch of few
 // site blocks needs the segments to fill the CUs.
 inline int nni_segment_edges(double edge_blocks, int n_cu) {
     const double per = edge_blocks / (12.0 * std::max(1, n_cu));

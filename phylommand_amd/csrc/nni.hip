@@ -2,6 +2,7 @@
 // (nni_program.h).
 #include "nni.h"
 
+#include "nni_device.h"
 #include "prune_device.h"
 
 namespace {
@@ -26,32 +27,6 @@ __device__ __forceinline__ void matvec4t(const double* __restrict__ P, const dou
     }
 }
 
-// Product over the wave of doubles in [0.5, 1) or 1 (or 0, NaN), in lane 63,
-// by DPP row shifts and row broadcasts (lanes without a source multiply by 1);
-// the same for sums of integers.
-template <int CTRL, int ROWS>
-__device__ __forceinline__ double dpp_mul(double v) {
-    const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL, ROWS, 0xf, false);
-    const int hi = __builtin_amdgcn_update_dpp(0x3ff00000, __double2hiint(v), CTRL, ROWS, 0xf, false);
-    return v * __hiloint2double(hi, lo);
-}
-__device__ __forceinline__ double wave_product(double v) {
-    v = dpp_mul<0x111, 0xf>(v);   // row_shr 1, 2, 4, 8
-    v = dpp_mul<0x112, 0xf>(v);
-    v = dpp_mul<0x114, 0xf>(v);
-    v = dpp_mul<0x118, 0xf>(v);
-    v = dpp_mul<0x142, 0xa>(v);   // row_bcast 15, 31
-    return dpp_mul<0x143, 0xc>(v);
-}
-__device__ __forceinline__ int wave_add(int v) {
-    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
-    return v + __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
-}
-
 // One workgroup walks one program over 64 sites, wave c computing rate
 // category c (P is wave-uniform: scalar loads).  The variants' category sums
 // meet in LDS, EV variants at a time, and wave w finishes variant w of them.
@@ -67,8 +42,9 @@ __device__ __forceinline__ int wave_add(int v) {
 // An edge issues about 220 vector instructions, 108 of them the FP64 products,
 // and reads two stored partials; issue (58 % busy) and the reads (1.0 GB of
 // partials, re-read once for the siblings) bind together, so five waves a
-// SIMD are asked for at the cost of a few spills.  250 variants of 128 taxa x
-// 100,000 sites: 0.538 ms, 2.206 ms as one path-to-root program a variant.
+// SIMD are asked for (80 registers; four 0.69, five 0.52 ms).  250 variants
+// of 128 taxa x 100,000 sites: 0.52 ms, 2.206 ms as one path-to-root program
+// a variant.
 template <typename T, int C, bool TL, bool BATCH, bool WEIGHTED>
 __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
     const NniOp* __restrict__ ops, const int* __restrict__ prog_begin, const NniInst* __restrict__ insts, NniInst one,
@@ -154,25 +130,12 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
         }
     };
     const bool live = s < I.m;
+    // edges held and their output index (an NNI_ROOT op has one variant)
     int n_held = 0, held_var[EP] = {};
     // site values of one variant from the categories' sums, to out[var]
     const auto finish = [&](double lc, int sc, int var) {
-        if constexpr (WEIGHTED) {
-            const double v = wave_sum(live ? site_w[s] * (log(lc) + sc * kLn2) : 0.0);
-            if (lane == 63) out[var] = make_double2(v, 0.0);
-        } else {
-            int e = 0;
-            double mant = 1.0;
-            if (live) {
-                mant = frexp(lc, &e);
-                e += sc;
-                // a negative sum has no logarithm: its sign must not cancel in the product
-                if (!(lc >= 0.0)) mant = __builtin_nan("");
-            }
-            mant = wave_product(mant);
-            e = wave_add(e);
-            if (lane == 63) out[var] = make_double2(mant, (double)e);
-        }
+        const double2 r = WEIGHTED ? nni_weighted(lc, sc, live ? site_w[s] : 0.0, live) : nni_product(lc, sc, live);
+        if (lane == 63) out[var] = r;
     };
     const auto flush = [&]() {
         if constexpr (C > 1) {
@@ -188,7 +151,8 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
                 double lc = 0.0;
 #pragma unroll
                 for (int c = 0; c < C; ++c) lc += ldexp(xr[cat][c][lane], xs[p][c][lane] - M);
-                finish(lc, M, var + (cat & 1));
+                if (!(var & kNniSingle)) finish(lc, M, var + (cat & 1));
+                else if (!(cat & 1)) finish(lc, M, var & ~kNniSingle);
             }
             __syncthreads();
             n_held = 0;
@@ -198,14 +162,14 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
         const int q = op.flags & NNI_XY ? 1 : 0;
         if constexpr (C == 1) {
             finish(l0, sc, op.var + q);
-            finish(l1, sc, op.var + 1 - q);
+            if (!(op.flags & NNI_ROOT)) finish(l1, sc, op.var + 1 - q);
         } else {
             xr[2 * n_held + q][cat][lane] = l0;
             xr[2 * n_held + 1 - q][cat][lane] = l1;
             xs[n_held][cat][lane] = sc;
 #pragma unroll
             for (int p = 0; p < EP; ++p)
-                if (n_held == p) held_var[p] = op.var;
+                if (n_held == p) held_var[p] = op.var | (op.flags & NNI_ROOT ? kNniSingle : 0);
             ++n_held;
         }
     };
@@ -257,8 +221,23 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
             sv[l][cat][1][lane] = make_double2(O[2], O[3]);
             svs[l][cat][lane] = sO;
         }
+        int sc = sO + sX + sY;
+        if (op.flags & NNI_ROOT) {
+            // in the pair's terms below: S = the factor of c, X = P_s (X x D)
+            T z[4] = {};
+            double f[4];
+            int sD;
+            fetch(op.d, z, sD);
+            factor(op.d, z, f);
+            sc += sD;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) f[i] *= X[i];
+            matvec4(P_of(op.s), f, X);
+            fetch(op.c, z, sB);
+            factor(op.c, z, B);
+        }
         const double* Pv = P_of(op.v);
-        if (op.flags & NNI_PAIR) {
+        if (op.flags & (NNI_PAIR | NNI_ROOT)) {
             double x[4], u[4], l0 = 0.0, l1 = 0.0;
 #pragma unroll
             for (int i = 0; i < 4; ++i) x[i] = B[i] * Y[i];
@@ -270,33 +249,7 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
             matvec4(Pv, x, u);
 #pragma unroll
             for (int i = 0; i < 4; ++i) l1 = fma(O[i] * Y[i], u[i], l1);
-            hold(l0, l1, sO + sB + sX + sY, op);
-        } else if (op.flags & NNI_ROOT_PAIR) {
-            // v's child and the sibling's left child change places: the
-            // root sees (P_v (C x Y)) and (P_s (X x D)), or with x, y
-            // exchanged (once a tree: a loop keeps its registers few)
-            double l0 = 0.0, l1 = 0.0;
-            int sC = 0, sD = 0;
-#pragma unroll 1
-            for (int q = 0; q < 2; ++q) {
-                T z[4] = {};
-                double f[4], u[4], w[4], l = 0.0;
-                fetch(op.c, z, sC);
-                factor(op.c, z, f);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) f[i] *= q ? X[i] : Y[i];
-                matvec4(Pv, f, u);
-                fetch(op.d, z, sD);
-                factor(op.d, z, f);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) f[i] *= q ? Y[i] : X[i];
-                matvec4(P_of(op.s), f, w);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) l = fma(O[i] * u[i], w[i], l);
-                if (q) l1 = l;
-                else l0 = l;
-            }
-            hold(l0, l1, sO + sX + sY + sC + sD, op);
+            hold(l0, l1, sc + sB, op);
         }
         if (op.flags & NNI_DESC) {
             double x[4];

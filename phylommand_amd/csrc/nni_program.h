@@ -28,8 +28,9 @@ enum NniFlags : int {
     NNI_SAVE = 8,       // O kept in a save slot for the sibling edge
     NNI_DESC = 16,      // v becomes the current node: O = P_v^T (O x S), B = factor of y
     NNI_PAIR = 32,      // score the edge's two variants into var, var + 1
-    NNI_ROOT_PAIR = 64, // the same for a child v of the root: its partner is the
-                        // sibling's left child c (d: the sibling's right child)
+    NNI_ROOT = 64,      // score one variant at a child v of the root into var: v's child
+                        // x changes places with the sibling's left child c (d: its
+                        // right child); the root sees P_v (C x Y) and P_s (X x D)
     NNI_XY = 128        // x is v's right child (the child entered first is always x)
 };
 
@@ -39,7 +40,7 @@ struct alignas(16) NniOp {
     int s;           // v's sibling, -1 for none
     int flags;       // NniFlags | save slot to read << 8 | save slot to write << 12
     int var;         // output index of the edge's first variant
-    int c, d;        // NNI_ROOT_PAIR: the sibling's children
+    int c, d;        // NNI_ROOT: the sibling's children
 };
 constexpr int nni_pop_slot(int flags) { return flags >> 8 & 15; }
 constexpr int nni_save_slot(int flags) { return flags >> 12 & 15; }
@@ -152,17 +153,16 @@ void build_nni_walks(const TV* c, const std::vector<int>& pair_of, int max_edges
                 pop = false;
             }
             if (!path.empty() || !pop) cur = u;
+            if (u == root && pair_of[v] >= 0) {
+                const int sib = sibling(v), l = c->left[v], r = c->right[v];
+                for (int side = 0; side < 2; ++side)
+                    ops.push_back({v, side ? r : l, side ? l : r, sib, NNI_ROOT | (pop ? NNI_POP | slot[u] << 8 : 0),
+                                   pair_of[v] + side, c->left[sib], c->right[sib]});
+            }
             NniOp o = edge_op(v, pop);
-            if (pair_of[v] >= 0) {
-                const int sib = sibling(v);
+            if (pair_of[v] >= 0 && u != root) {
                 o.var = pair_of[v];
-                if (u != root) {
-                    o.flags |= NNI_PAIR;
-                } else {
-                    o.flags |= NNI_ROOT_PAIR;
-                    o.c = c->left[sib];
-                    o.d = c->right[sib];
-                }
+                o.flags |= NNI_PAIR;
             }
             --later[u];
             if (later[u] == 0 && slot[u] >= 0) {     // u's last edge: its slot is free

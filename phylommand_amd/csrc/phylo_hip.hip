@@ -634,8 +634,8 @@ struct phylo_ctx {
     double* d_P = nullptr; size_t P_bytes = 0;
     Op* d_ops = nullptr; size_t ops_bytes = 0;
     int* d_prog = nullptr; size_t prog_bytes = 0;
-    Op* d_nni_ops = nullptr; size_t nni_ops_bytes = 0;   // NNI partial-recompute programs (wide alphabets)
-    int* d_nni_prog = nullptr; size_t nni_prog_bytes = 0;
+    double* d_PmT = nullptr; size_t PmT_bytes = 0;       // P transposed in MFMA operand order (NNI walks)
+    bool have_PmT = false;                                // d_PmT matches d_P
     // NNI walks of the current topology (nni_program.h), rebuilt when it changes
     struct NniWalks {
         int mode = -1;                                    // -1: none built
@@ -1120,6 +1120,7 @@ int upload_pmatrices(phylo_ctx* c) {
         HIPCHK(c, mfma_operands(c->d_P, c->S_model, Sp, c->C, c->n_nodes, c->d_Pm, c->d_PTm, c->stream));
     }
     c->dirty_P = false;
+    c->have_PmT = false;
     return PHYLO_OK;
 }
 
@@ -1303,12 +1304,6 @@ int dispatch_mfma(phylo_ctx* c, dim3 grid, double* site_lnl) {
             a.fold_out = c->h_total_dev;
             c->folded = a.fold != nullptr;
         }
-    } else if (grid.y > 1) {
-        // an NNI neighbourhood: program-major, grouped by XCD (1-D grid)
-        a.prog_main = -2;
-        a.n_tail = (int)grid.y;
-        a.blk0 = 1;
-        a.grid = dim3((nblk + 7) / 8 * 8 * grid.y);
     }
     HIPCHK(c, mfma_launch(a, c->stream));
     return PHYLO_OK;
@@ -1435,77 +1430,6 @@ void enumerate_nni(const TV* c, int mode, std::vector<int>& nodes, std::vector<i
     }
 }
 
-// Appends the partial-recompute program of tree::interchange(v, side == 0)
-// (tree.cpp:2480-2518): the two nodes whose children change, then the path to
-// the root, each child coming from a stored partial, a tip or a register
-// carry.  Returns false when the interchange is a no-op (no swap partner).
-template <class TV>
-bool append_nni_program(const TV* c, const std::vector<int>& par, int v, int side, std::vector<Op>& ops) {
-    if (v < 0 || v == c->root || c->left[v] < 0) return false;
-    const int p = par[v], r = c->root;
-    const auto mem = [&](int x, int& kind, int& idx) {
-        if (x < c->n_taxa) { kind = SRC_TIP; idx = x; }
-        else { kind = SRC_CLV; idx = x - c->n_taxa; }
-    };
-    const int sib = c->left[p] == v ? c->right[p] : c->left[p];
-    int partner = -1;
-    if (p != r) partner = sib;
-    else if (sib >= 0 && c->left[sib] >= 0) partner = c->left[sib];
-    if (partner < 0) return false;
-    const int tmp = side == 0 ? c->left[v] : c->right[v];
-    // v with `partner` in place of `tmp`
-    Op o1{};
-    const int vl = side == 0 ? partner : c->left[v], vr = side == 0 ? c->right[v] : partner;
-    o1.l_node = vl; o1.r_node = vr;
-    mem(vl, o1.l_kind, o1.l_idx);
-    mem(vr, o1.r_kind, o1.r_idx);
-    o1.out_slot = -1;
-    o1.flags = 0;
-    ops.push_back(o1);
-    const int pp = p != r ? p : sib;            // partner's old parent
-    // pp with `tmp` in place of `partner` (and v carried when pp == p)
-    Op o2{};
-    const int ql = c->left[pp] == partner ? tmp : c->left[pp];
-    const int qr = c->right[pp] == partner ? tmp : c->right[pp];
-    o2.l_node = ql; o2.r_node = qr;
-    if (ql == v) { o2.l_kind = SRC_CARRY_A; o2.l_idx = 0; } else mem(ql, o2.l_kind, o2.l_idx);
-    if (qr == v) { o2.r_kind = SRC_CARRY_A; o2.r_idx = 0; } else mem(qr, o2.r_kind, o2.r_idx);
-    o2.out_slot = -1;
-    if (p != r) {
-        o2.flags = 0;
-        ops.push_back(o2);
-        int cur = p;
-        while (cur != r) {
-            const int up = par[cur];
-            Op o{};
-            o.l_node = c->left[up];
-            o.r_node = c->right[up];
-            if (c->left[up] == cur) { o.l_kind = SRC_CARRY_A; o.l_idx = 0; mem(c->right[up], o.r_kind, o.r_idx); }
-            else { o.r_kind = SRC_CARRY_A; o.r_idx = 0; mem(c->left[up], o.l_kind, o.l_idx); }
-            o.out_slot = -1;
-            o.flags = up == r ? OP_ROOT : 0;
-            ops.push_back(o);
-            cur = up;
-        }
-    } else {
-        // at the root: v waits in B (o2 does not read it), its sibling comes
-        // in A, then the root
-        ops[ops.size() - 1].flags |= OP_TO_B;
-        o2.flags = 0;
-        ops.push_back(o2);
-        Op o3{};
-        o3.l_node = c->left[r];
-        o3.r_node = c->right[r];
-        o3.l_kind = c->left[r] == v ? SRC_CARRY_B : SRC_CARRY_A;
-        o3.r_kind = c->right[r] == v ? SRC_CARRY_B : SRC_CARRY_A;
-        o3.l_idx = o3.r_idx = 0;
-        o3.out_slot = -1;
-        o3.flags = OP_ROOT;
-        ops.push_back(o3);
-    }
-    return true;
-}
-
 // The node an interchange at v moves out of v's surroundings: v's sibling or,
 // at a child of the root, the sibling's left child; -1 where there is none
 // (the variant is the tree itself).
@@ -1603,7 +1527,7 @@ void phylo_destroy(phylo_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void* bufs[] = {c->d_tips, c->d_Pm, c->d_PTm, c->d_clv, c->d_scl, c->d_P, c->d_ops, c->d_prog, c->d_nni_ops, c->d_nni_prog,
+    void* bufs[] = {c->d_tips, c->d_Pm, c->d_PTm, c->d_clv, c->d_scl, c->d_P, c->d_ops, c->d_prog, c->d_PmT,
                     c->d_roots, c->d_sitew,
                     c->d_sitelnl, c->d_partial, c->d_eig, c->d_fold, c->walks.d_ops, c->walks.d_prog, c->walks.d_part};
     for (void* b : bufs)
@@ -1864,12 +1788,13 @@ int phylo_get_pmatrix(phylo_ctx* c, int node, double* P) {
 
 namespace {
 
-// The DNA neighbourhood: every variant by the outer-partial walks, against
-// the stored partials of an evaluation that kept them all.
+// A neighbourhood: every variant by the outer-partial walks, against the
+// stored partials of an evaluation that kept them all.
 int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* lnl, int32_t* node, int32_t* side,
                 int* n_variants, double* base_lnl) {
     auto& w = c->walks;
-    const int nblk = c->m_pad / 64;
+    const bool mfma = uses_mfma(c);
+    const int nblk = c->m_pad / (mfma ? 16 * kNniGroups : 64);
     if (w.mode != mode) {
         w.mode = -1;
         std::vector<NniOp> ops;
@@ -1918,8 +1843,15 @@ int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* l
     a.one.n_var = n_out;
     a.one.nblk = nblk;
     a.n_prog = w.n_prog;
+    if (mfma && !c->have_PmT) {
+        const int S = c->S_model, V = mfma_slots(S), TN = V > 4 ? 2 : 1;
+        HIPCHK(c, ensure(c->d_PmT, c->PmT_bytes, (size_t)c->n_nodes * c->C * TN * V * 64 * sizeof(double)));
+        HIPCHK(c, mfma_transposed(c->d_P, S, padded_states(S), c->C, c->n_nodes, c->d_PmT, c->stream));
+        c->have_PmT = true;
+    }
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    HIPCHK(c, nni4_launch(a, c->stream));
+    if (mfma) HIPCHK(c, nni_mfma_launch(a, c->S, static_cast<const uint32_t*>(c->d_tips), c->d_Pm, c->d_PmT, c->d_PTm, c->stream));
+    else HIPCHK(c, nni4_launch(a, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr,
                              (n_out + kNniSumVars - 1) / kNniSumVars, c->h_total_dev, c->stream));
@@ -1946,38 +1878,7 @@ int phylo_nni_score(phylo_ctx* c, int mode, int max_variants, double* lnl, int32
         if (rc) return rc;
     }
     base = c->base_total;
-    if (!uses_mfma(c)) return score_walks(c, mode, max_variants, base, lnl, node, side, n_variants, base_lnl);
-    std::vector<int> nodes, sides;
-    enumerate_nni(c, mode, nodes, sides);
-    const int nv = (int)nodes.size();
-    *n_variants = nv;
-    if (base_lnl) *base_lnl = base;
-    if (nv == 0 || !lnl) return PHYLO_OK;   // count query
-    if (max_variants < nv) return fail(c, PHYLO_ERR_ARG, "nni_score: output arrays too small");
-    const std::vector<int> par = parents_of(c);
-    std::vector<Op> ops;
-    std::vector<int> begin{0}, which;
-    for (int k = 0; k < nv; ++k) {
-        if (append_nni_program(c, par, nodes[k], sides[k], ops)) {
-            begin.push_back((int)ops.size());
-            which.push_back(k);
-        }
-        lnl[k] = base;   // no-op interchanges keep the base tree
-        if (node) node[k] = nodes[k];
-        if (side) side[k] = sides[k];
-    }
-    const int n_prog = (int)which.size();
-    if (n_prog == 0) return PHYLO_OK;
-    if (!root_ops_last(ops, begin)) return fail(c, PHYLO_ERR_STATE, "internal: root op not last");
-    HIPCHK(c, upload_ops(c->d_nni_ops, c->nni_ops_bytes, ops, c->stream));
-    HIPCHK(c, ensure(c->d_nni_prog, c->nni_prog_bytes, begin.size() * sizeof(int)));
-    HIPCHK(c, hipMemcpyAsync(c->d_nni_prog, begin.data(), begin.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-    std::vector<double> tot(n_prog);
-    rc = run_programs(c, c->d_nni_ops, c->d_nni_prog, n_prog, tot.data(), nullptr);
-    if (rc) return rc;
-    for (int q = 0; q < n_prog; ++q) lnl[which[q]] = tot[q];
-    c->nni_ops_last = (long)ops.size();
-    return PHYLO_OK;
+    return score_walks(c, mode, max_variants, base, lnl, node, side, n_variants, base_lnl);
 }
 
 int phylo_simulate(phylo_ctx* c, int n_sites, const double* root_freq, uint64_t seed, uint8_t* states) {

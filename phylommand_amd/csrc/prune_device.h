@@ -47,6 +47,9 @@ constexpr int kSplitAllBelowPerCu = 4;
 // wave share each P operand load and overlap their memory latency.
 constexpr int kMfmaGroups = 2;
 
+// Site groups per wave of the matrix-core NNI walk.
+constexpr int kNniGroups = 1;
+
 // ---------------------------------------------------------------------------
 // Device helpers
 // ---------------------------------------------------------------------------

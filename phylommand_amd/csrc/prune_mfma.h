@@ -6,6 +6,7 @@
 #include <cstdint>
 #include <type_traits>
 
+#include "nni.h"
 #include "prune_device.h"
 
 // Operand slots that cover S states, four a slot.
@@ -42,3 +43,9 @@ hipError_t mfma_launch(const MfmaArgs& a, hipStream_t st);
 int mfma_resident(bool f64, int C, int S);
 // The walker's P operands and tip columns from P (pmfma_kernel, ptm_kernel).
 hipError_t mfma_operands(const double* P, int S, int Sp, int C, int n_nodes, double* Pm, double* PTm, hipStream_t st);
+
+// The same operands of every P's transpose (the NNI walks' way down).
+hipError_t mfma_transposed(const double* P, int S, int Sp, int C, int n_nodes, double* PmT, hipStream_t st);
+// NNI walks (nni.h; a.tips, a.P and the batch members unused).
+hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const double* Pm, const double* PmT,
+                           const double* PTm, hipStream_t st);

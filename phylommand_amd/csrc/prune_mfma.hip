@@ -2,6 +2,8 @@
 // (prune_mfma.h).
 #include "prune_mfma.h"
 
+#include "nni.h"
+#include "nni_device.h"
 #include "prune_device.h"
 
 namespace {
@@ -37,6 +39,8 @@ typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 // = 4b + 16k + i holds P[16 + i][4t + k] for every block b.  That product
 // lands as D[lane j + 16 i] = row 16 + i of site j, the operand slot of
 // states 16..19, with no padded rows.
+// TR: of the transpose.
+template <bool TR>
 __global__ void pmfma_kernel(const double* __restrict__ P, int S, int Sp, int C, int n_nodes, int V, int TN,
                              double* __restrict__ Pm) {
     const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -48,7 +52,7 @@ __global__ void pmfma_kernel(const double* __restrict__ P, int S, int Sp, int C,
     const long mat = gid / (64L * V * TN);          // node * C + cat
     const bool short_tile = V == 5 && T == 1;
     const int row = 16 * T + (short_tile ? l % 4 : l % 16), col = 4 * t + l / 16;
-    Pm[gid] = (row < S && col < S) ? P[(mat * Sp + row) * Sp + col] : 0.0;
+    Pm[gid] = (row < S && col < S) ? P[TR ? (mat * Sp + col) * Sp + row : (mat * Sp + row) * Sp + col] : 0.0;
 }
 
 // PTm[node][cat][k][i] = P[i][k] for k < S, PTm[..][S][i] = sum_q P[i][q]
@@ -355,11 +359,8 @@ __device__ __forceinline__ void mfma_shape(const Op& op, int cat, const int (&s)
 // otherwise).
 // TL (n_taxa <= kMfmaTipLdsTaxa): the workgroup first copies the tip masks of
 // its 16 G sites into LDS (tl[16 G t + site]).
-// MP: the program-major launch of prune4_kernel (n_main site blocks, n_tail
-// programs, blk0 of them a workgroup, grouped by XCD), one program after
-// another in the workgroup.
-template <typename T, int C, int V, int G, bool TL, bool MP>
-__device__ __forceinline__ void prune_mfma_walk(
+template <typename T, int C, int V, int G, bool TL>
+__global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_kernel(
     const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
     int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
     const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
@@ -383,11 +384,6 @@ __device__ __forceinline__ void prune_mfma_walk(
             prog = prog_piece + r / n_tail;
             has_root = false;
         }
-    } else if (MP) {
-        const int slot = (int)blockIdx.x >> 3, n_pg = (n_tail + blk0 - 1) / blk0;
-        prog = slot % n_pg * blk0;
-        bx = slot / n_pg * 8 + ((int)blockIdx.x & 7);
-        if (bx >= n_main) return;        // the last group's padding (uniform per workgroup)
     }
     if (TL) {
         const uint32_t* blk = tips + (size_t)bx * 16 * G;
@@ -402,10 +398,7 @@ __device__ __forceinline__ void prune_mfma_walk(
     int s[G];
 #pragma unroll
     for (int q = 0; q < G; ++q) s[q] = (sg0 + q) * 16 + j;
-    const int p_end = MP ? min(prog + blk0, n_tail) : prog + 1;
-    int p = prog;
-    do {    // MP: the workgroup's programs in turn; otherwise once
-    const int k0 = prog_begin[p], k1 = prog_begin[p + 1];
+    const int k0 = prog_begin[prog], k1 = prog_begin[prog + 1];
     const size_t slot_stride = (size_t)C * m_pad * 4 * V;
     // carried results stay in FP64 and are rescaled lazily, as in the DNA
     // walker; only stored partials are rounded to T
@@ -551,46 +544,306 @@ __device__ __forceinline__ void prune_mfma_walk(
 #pragma unroll
     for (int q = 0; q < G; ++q) {
         const bool live = s[q] < m && cat == 0 && g == 0;
-        if (live && site_lnl) site_lnl[(size_t)(MP ? p : y) * m + s[q]] = lnl[q];
+        if (live && site_lnl) site_lnl[(size_t)y * m + s[q]] = lnl[q];
         if (live) sum += (site_w ? site_w[s[q]] : 1.0) * lnl[q];
     }
-    if constexpr (MP) {
-        // only the category-0 wave holds site values: its sum is the block's
-        if (cat == 0) {
-            const double v = wave_sum(sum);
-            if (lane == 0) partial[(size_t)p * n_main + bx] = v;
-        }
-    } else {
-        block_sum_store(sum, partial + (prog_main >= 0 ? (size_t)bx : (size_t)y * gridDim.x + blockIdx.x));
-        if (64 * C == kSumThreads && fold_counter) fold_total(partial, blk0 + n_main, fold_counter, fold_out);
-    }
-    } while (MP && ++p < p_end);
+    block_sum_store(sum, partial + (prog_main >= 0 ? (size_t)bx : (size_t)y * gridDim.x + blockIdx.x));
+    if (64 * C == kSumThreads && fold_counter) fold_total(partial, blk0 + n_main, fold_counter, fold_out);
 }
 
-template <typename T, int C, int V, int G, bool TL>
-__global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_kernel(
-    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
-    int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
-    const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
-    int S, uint32_t full, int n_taxa, int n_main, int prog_main, int blk0, int prog_piece, int tail0, int n_tail,
-    unsigned* fold_counter, double* fold_out) {
-    prune_mfma_walk<T, C, V, G, TL, false>(ops, prog_begin, tips, clv, scl, Pm, PTm, roots, site_w, site_lnl, partial, m, m_pad, S, full,
-                                          n_taxa, n_main, prog_main, blk0, prog_piece, tail0, n_tail, fold_counter,
-                                          fold_out);
-}
-
-// An NNI neighbourhood's programs, program-major and grouped by XCD
-// (prune_mfma_walk's MP launch).
+// One workgroup walks one NNI program (nni_program.h) over 16 G sites, wave c
+// computing rate category c: the DNA walk of nni.hip with the products on
+// the matrix cores.  P_v serves both variants from one load; its transpose
+// (PmT, the same operand order) carries the outer partial down.  The outer
+// partial and one child factor stay in registers between edges.  One site
+// group a wave: two need 168 registers and spill 188 in the loop, one fits 128
+// (20 states), four waves a SIMD to hide the chain of dependent products that
+// binds it.  74 variants of 40 taxa x 5,000 sites, 20 states: 0.176 ms, 0.44 ms
+// as one path-to-root program a variant.
 template <typename T, int C, int V, int G>
-__global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_nni_kernel(
-    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint32_t* __restrict__ tips, T* clv,
-    int* scl, const double* __restrict__ Pm, const double* __restrict__ PTm, const double* __restrict__ roots,
-    const double* __restrict__ site_w, double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad,
-    int S, uint32_t full, int n_taxa, int n_main, int prog_main, int blk0, int prog_piece, int tail0, int n_tail,
-    unsigned* fold_counter, double* fold_out) {
-    prune_mfma_walk<T, C, V, G, false, true>(ops, prog_begin, tips, clv, scl, Pm, PTm, roots, site_w, site_lnl, partial, m, m_pad, S, full,
-                                          n_taxa, n_main, prog_main, blk0, prog_piece, tail0, n_tail, fold_counter,
-                                          fold_out);
+__global__ __launch_bounds__(64 * C, (V <= 5 ? 4 : 3)) void nni_mfma_kernel(
+    const NniOp* __restrict__ ops, const int* __restrict__ prog_begin, int n_prog, const uint32_t* __restrict__ tips,
+    const T* __restrict__ clv, const int* __restrict__ scl, const double* __restrict__ Pm,
+    const double* __restrict__ PmT, const double* __restrict__ PTm, const double* __restrict__ roots,
+    const double* __restrict__ site_w, double2* __restrict__ part, int m, int m_pad, int S, uint32_t full, int n_taxa,
+    int nblk, int n_var, int tip_lds) {
+    constexpr int EV = C == 1 ? 2 : C < 4 ? C : 4, EP = EV / 2, TNV = (V > 4 ? 2 : 1) * V;
+    __shared__ double xr[EV][C][16 * G];
+    __shared__ int xs[EP][C][16 * G];
+    static_assert(kNniSaves == 1, "one save slot");
+    __shared__ double sv[C][G * V * 64];
+    __shared__ int svs[C][G][64];
+    extern __shared__ uint32_t tl[];        // n_taxa x 16 G masks (tip_lds)
+    const int slot = (int)blockIdx.x >> 3;
+    const int prog = slot % n_prog, bx = slot / n_prog * 8 + ((int)blockIdx.x & 7);
+    if (bx >= nblk) return;
+    if (tip_lds) {
+        const uint32_t* blk = tips + (size_t)bx * 16 * G;
+        for (int i = threadIdx.x; i < n_taxa * 16 * G; i += 64 * C)
+            tl[i] = blk[(size_t)(i / (16 * G)) * m_pad + i % (16 * G)];
+        __syncthreads();
+    }
+    const int lane = threadIdx.x & 63, g = lane >> 4, j = lane & 15;
+    const int cat = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int sg0 = bx * G, n_sg = m_pad >> 4;
+    const size_t slot_stride = (size_t)C * m_pad * 4 * V;
+    double2* const out = part + (size_t)bx * n_var;
+
+    // a node's own partial: tip masks (col: all single states or gaps) or a stored partial
+    const auto fetch = [&](int node, T (&x)[G][V], uint32_t (&mk)[G], bool& col, int (&sc)[G]) {
+#pragma unroll
+        for (int q = 0; q < G; ++q) sc[q] = 0;
+        col = false;
+        if (node >= n_taxa) {
+            const size_t idx = node - n_taxa;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const T* src = clv + idx * slot_stride + ((size_t)cat * n_sg + sg0 + q) * V * 64 + lane;
+#pragma unroll
+                for (int t = 0; t < V; ++t) x[q][t] = src[t * 64];
+                sc[q] = scl[(idx * C + cat) * m_pad + (sg0 + q) * 16 + j];
+            }
+        } else if (node >= 0) {
+            bool simple = true;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                mk[q] = tip_lds ? tl[node * 16 * G + 16 * q + j] : tips[(size_t)node * m_pad + (sg0 + q) * 16 + j];
+                simple = simple && (mk[q] == full || __popc(mk[q]) == 1);
+            }
+            col = __all(simple);
+        }
+    };
+    // its factor P x (ones for a missing child)
+    const auto factor = [&](int node, const T (&x)[G][V], const uint32_t (&mk)[G], bool col, double (&f)[G][V]) {
+        if (node < 0) {
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int t = 0; t < V; ++t) f[q][t] = 1.0;
+        } else if (col) {
+            const double* base = PTm + ((size_t)node * C + cat) * (S + 1) * (4 * V) + g;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                const int c = mk[q] == full ? S : __ffs(mk[q]) - 1;
+                const double* pt = base + (size_t)c * (4 * V);
+#pragma unroll
+                for (int t = 0; t < V; ++t) f[q][t] = pt[4 * t];
+            }
+        } else {
+            double p[TNV], v[G][V];
+            load_pm<C, V>(node, cat, lane, Pm, p);
+            const bool tip = node < n_taxa;
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int t = 0; t < V; ++t)
+                    v[q][t] = tip ? ((mk[q] >> (4 * t + g)) & 1u ? 1.0 : 0.0) : to_d(x[q][t]);
+            mfma_products<V, G>(p, v, f);
+        }
+    };
+    int n_held = 0, held_var[EP] = {};
+    const auto flush = [&]() {
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < (EV + C - 1) / C; ++r) {
+            const int w = cat + r * C;
+            if (w >= 2 * n_held) continue;
+            const int p = w >> 1, i = lane % (16 * G);
+            int var = held_var[0];
+#pragma unroll
+            for (int q = 1; q < EP; ++q) var = p == q ? held_var[q] : var;
+            int M = xs[p][0][i];
+#pragma unroll
+            for (int c = 1; c < C; ++c) M = max(M, xs[p][c][i]);
+            double lc = 0.0;
+#pragma unroll
+            for (int c = 0; c < C; ++c) lc += ldexp(xr[w][c][i], xs[p][c][i] - M);
+            const int s = sg0 * 16 + lane;
+            const bool live = lane < 16 * G && s < m;
+            const double2 res = site_w ? nni_weighted(lc, M, live ? site_w[s] : 0.0, live) : nni_product(lc, M, live);
+            if (lane == 63) {
+                if (!(var & kNniSingle)) out[var + (w & 1)] = res;
+                else if (!(w & 1)) out[var & ~kNniSingle] = res;
+            }
+        }
+        __syncthreads();
+        n_held = 0;
+    };
+    // l[q]: a site's sum over its states, still spread over the lane groups
+    const auto hold = [&](const double (&l0)[G], const double (&l1)[G], const int (&sc)[G], const NniOp& op) {
+        const int k = 2 * n_held + (op.flags & NNI_XY ? 1 : 0);
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            double a = l0[q], b = l1[q];
+            a += __shfl_xor(a, 16, 64);
+            b += __shfl_xor(b, 16, 64);
+            a += __shfl_xor(a, 32, 64);
+            b += __shfl_xor(b, 32, 64);
+            if (g == 0) {
+                xr[k][cat][16 * q + j] = a;
+                xr[k ^ 1][cat][16 * q + j] = b;
+                xs[n_held][cat][16 * q + j] = sc[q];
+            }
+        }
+#pragma unroll
+        for (int p = 0; p < EP; ++p)
+            if (n_held == p) held_var[p] = op.var | (op.flags & NNI_ROOT ? kNniSingle : 0);
+        ++n_held;
+    };
+
+    double O[G][V] = {}, B[G][V] = {};
+    int sO[G] = {}, sB[G] = {};
+    const int k0 = prog_begin[prog], k1 = prog_begin[prog + 1];
+    NniOp nx = ops[k0];
+    for (int k = k0; k < k1; ++k) {
+        const NniOp op = nx;
+        nx = ops[k + 1];
+        double X[G][V], Y[G][V];
+        int sX[G], sY[G];
+        {
+            T rx[G][V] = {}, ry[G][V] = {};
+            uint32_t mx[G] = {}, my[G] = {};
+            bool cx, cy;
+            fetch(op.x, rx, mx, cx, sX);
+            fetch(op.y, ry, my, cy, sY);
+            factor(op.x, rx, mx, cx, X);
+            factor(op.y, ry, my, cy, Y);
+        }
+        if (op.flags & NNI_INIT) {
+            const double w = roots[kRootCatOff + cat];
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) {
+                    O[q][t] = roots[4 * t + g] * w;
+                    B[q][t] = Y[q][t];
+                }
+                sO[q] = 0;
+                sB[q] = sY[q];
+            }
+            continue;
+        }
+        if (op.flags & NNI_POP) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) O[q][t] = sv[cat][(q * V + t) * 64 + lane];
+                sO[q] = svs[cat][q][lane];
+            }
+        }
+        if (op.flags & NNI_FETCH_S) {
+            T r[G][V] = {};
+            uint32_t mk[G] = {};
+            bool col;
+            fetch(op.s, r, mk, col, sB);
+            factor(op.s, r, mk, col, B);
+        }
+        if (op.flags & NNI_SAVE) {
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) sv[cat][(q * V + t) * 64 + lane] = O[q][t];
+                svs[cat][q][lane] = sO[q];
+            }
+        }
+        if (op.flags & NNI_ROOT) {
+            // in the pair's terms below: S = the factor of c, X = P_s (X x D)
+            T r[G][V] = {};
+            uint32_t mk[G] = {};
+            bool col;
+            int sD[G];
+            double f[G][V], p[TNV];
+            fetch(op.d, r, mk, col, sD);
+            factor(op.d, r, mk, col, f);
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                sX[q] += sD[q];
+#pragma unroll
+                for (int t = 0; t < V; ++t) f[q][t] *= X[q][t];
+            }
+            load_pm<C, V>(op.s, cat, lane, Pm, p);
+            mfma_products<V, G>(p, f, X);
+            fetch(op.c, r, mk, col, sB);
+            factor(op.c, r, mk, col, B);
+        }
+        if (op.flags & (NNI_PAIR | NNI_ROOT)) {
+            double p[TNV], v[G][V], u[G][V], l0[G], l1[G];
+            int sc[G];
+            load_pm<C, V>(op.v, cat, lane, Pm, p);
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int t = 0; t < V; ++t) v[q][t] = B[q][t] * Y[q][t];
+            mfma_products<V, G>(p, v, u);
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                l0[q] = 0.0;
+#pragma unroll
+                for (int t = 0; t < V; ++t) l0[q] = fma(O[q][t] * X[q][t], u[q][t], l0[q]);
+#pragma unroll
+                for (int t = 0; t < V; ++t) v[q][t] = B[q][t] * X[q][t];
+            }
+            mfma_products<V, G>(p, v, u);
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                l1[q] = 0.0;
+#pragma unroll
+                for (int t = 0; t < V; ++t) l1[q] = fma(O[q][t] * Y[q][t], u[q][t], l1[q]);
+                sc[q] = sO[q] + sB[q] + sX[q] + sY[q];
+            }
+            hold(l0, l1, sc, op);
+        }
+        if (op.flags & NNI_DESC) {
+            double p[TNV], v[G][V];
+            load_pm<C, V>(op.v, cat, lane, PmT, p);
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+#pragma unroll
+                for (int t = 0; t < V; ++t) v[q][t] = O[q][t] * B[q][t];
+            mfma_products<V, G>(p, v, O);
+            // lazy rescale, as in the pruning walker
+            bool low = false;
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+                sO[q] += sB[q];
+                int h = __double2hiint(O[q][0]);
+#pragma unroll
+                for (int t = 1; t < V; ++t) h = max(h, __double2hiint(O[q][t]));
+                low |= h < kLazyRescaleHi;
+            }
+            if (__builtin_amdgcn_ballot_w64(low) != 0) {
+#pragma unroll
+                for (int q = 0; q < G; ++q) {
+                    const int e = site_exponent<V>(O[q]);
+                    const double mx = site_max<V>(O[q]);
+                    if (mx < 0x1p-256) {
+                        sO[q] += e;
+#pragma unroll
+                        for (int t = 0; t < V; ++t) O[q][t] = ldexp(O[q][t], -e);
+                    }
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < G; ++q) {
+#pragma unroll
+                for (int t = 0; t < V; ++t) B[q][t] = Y[q][t];
+                sB[q] = sY[q];
+            }
+        }
+        if (n_held == EP) flush();
+    }
+    if (n_held) flush();    // (uniform per workgroup)
+}
+
+template <typename T, int C, int V>
+void launch_nni_v(const NniArgs& a, int S, const uint32_t* tips, const double* Pm, const double* PmT, const double* PTm,
+                  hipStream_t st) {
+    const uint32_t full = S == 32 ? 0xFFFFFFFFu : ((1u << S) - 1u);
+    const bool tl = a.max_taxa <= kMfmaTipLdsTaxa;
+    hipLaunchKernelGGL((nni_mfma_kernel<T, C, V, kNniGroups>), dim3((a.one.nblk + 7) / 8 * 8 * a.n_prog), dim3(64 * C),
+                       tl ? (size_t)a.max_taxa * 16 * kNniGroups * sizeof(uint32_t) : 0, st, a.ops, a.prog, a.n_prog,
+                       tips, static_cast<const T*>(a.clv), a.scl, Pm, PmT, PTm, a.roots, a.site_w, a.part, a.one.m,
+                       a.one.m_pad, S, full, a.one.n_taxa, a.one.nblk, a.one.n_var, tl ? 1 : 0);
 }
 
 template <typename T, int C, int V>
@@ -601,8 +854,7 @@ void launch_v(const MfmaArgs& a, hipStream_t st) {
     hipLaunchKernelGGL(K, a.grid, dim3(64 * C), 0, st, a.ops, a.prog, a.tips, clv, a.scl, a.Pm, a.PTm, a.roots, a.site_w, \
                        a.site_lnl, a.partial, a.m, a.m_pad, a.S, full, a.n_taxa, a.n_main, a.prog_main, a.blk0,        \
                        a.prog_piece, a.tail0, a.n_tail, a.fold, a.fold_out)
-    if (a.prog_main == -2) PHYLO_MFMA_LAUNCH((prune_mfma_nni_kernel<T, C, V, kMfmaGroups>));
-    else if (a.tip_lds) PHYLO_MFMA_LAUNCH((prune_mfma_kernel<T, C, V, kMfmaGroups, true>));
+    if (a.tip_lds) PHYLO_MFMA_LAUNCH((prune_mfma_kernel<T, C, V, kMfmaGroups, true>));
     else PHYLO_MFMA_LAUNCH((prune_mfma_kernel<T, C, V, kMfmaGroups, false>));
 #undef PHYLO_MFMA_LAUNCH
 }
@@ -656,10 +908,26 @@ int mfma_resident(bool f64, int C, int S) {
     return n;
 }
 
+hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const double* Pm, const double* PmT,
+                           const double* PTm, hipStream_t st) {
+    with_kernel(a.f64, a.C, S, [&](auto t, auto c, auto v) {
+        launch_nni_v<decltype(t), c(), v()>(a, S, tips, Pm, PmT, PTm, st);
+    });
+    return hipGetLastError();
+}
+
+hipError_t mfma_transposed(const double* P, int S, int Sp, int C, int n_nodes, double* PmT, hipStream_t st) {
+    const int V = mfma_slots(S), TN = V > 4 ? 2 : 1;
+    const long nPm = (long)n_nodes * C * TN * V * 64;
+    hipLaunchKernelGGL((pmfma_kernel<true>), dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, V,
+                       TN, PmT);
+    return hipGetLastError();
+}
+
 hipError_t mfma_operands(const double* P, int S, int Sp, int C, int n_nodes, double* Pm, double* PTm, hipStream_t st) {
     const int V = mfma_slots(S), TN = V > 4 ? 2 : 1;
     const long nPm = (long)n_nodes * C * TN * V * 64, nPT = (long)n_nodes * C * (S + 1) * 4 * V;
-    hipLaunchKernelGGL(pmfma_kernel, dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, V, TN,
+    hipLaunchKernelGGL((pmfma_kernel<false>), dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, V, TN,
                        Pm);
     hipLaunchKernelGGL(ptm_kernel, dim3((unsigned)((nPT + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, 4 * V,
                        PTm);

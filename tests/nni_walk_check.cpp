@@ -131,19 +131,22 @@ int main() {
                         if (nni_pop_slot(o.flags) >= kNniSaves) { printf("slot out of range\n"); return 1; }
                         O = save[nni_pop_slot(o.flags)];
                     }
-                    const V4 S = o.flags & NNI_FETCH_S ? factor(o.s) : B;
+                    const V4 S = o.flags & (NNI_FETCH_S | NNI_ROOT) ? factor(o.s) : B;
                     if (O.empty() || S.empty()) { printf("state not loaded\n"); return 1; }
                     double l[2] = {0, 0};
                     if (o.flags & NNI_PAIR) {
                         const V4 a = mul(mul(O, X), mv(o.v, mul(S, Y))), b = mul(mul(O, Y), mv(o.v, mul(S, X)));
                         for (int i = 0; i < 4; ++i) { l[0] += a[i]; l[1] += b[i]; }
-                    } else if (o.flags & NNI_ROOT_PAIR) {
-                        const V4 C = factor(o.c), D = factor(o.d);
-                        const V4 a = mul(O, mul(mv(o.v, mul(C, Y)), mv(o.s, mul(X, D))));
-                        const V4 b = mul(O, mul(mv(o.v, mul(X, C)), mv(o.s, mul(Y, D))));
-                        for (int i = 0; i < 4; ++i) { l[0] += a[i]; l[1] += b[i]; }
+                    } else if (o.flags & NNI_ROOT) {
+                        const V4 a = mul(O, mul(mv(o.v, mul(factor(o.c), Y)), mv(o.s, mul(X, factor(o.d)))));
+                        double l0 = 0.0;
+                        for (double z : a) l0 += z;
+                        if (o.var < 0 || o.var >= n_out || got[o.var] >= 0) { printf("output index\n"); return 1; }
+                        got[o.var] = l0;
+                        B.clear();
+                        continue;
                     }
-                    if (o.flags & (NNI_PAIR | NNI_ROOT_PAIR)) {
+                    if (o.flags & NNI_PAIR) {
                         if (o.var < 0 || o.var + 1 >= n_out || got[o.var] >= 0) { printf("output index\n"); return 1; }
                         const int q = o.flags & NNI_XY ? 1 : 0;
                         got[o.var + q] = l[0];
