@@ -228,121 +228,309 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
 
 // ---------------------------------------------------------------------------
 // MLP kernels (FP32)
+//
+// A training step is six launches: two hidden layers forward (bias and ReLU
+// in the product's epilogue, the minibatch's rows gathered as they are read),
+// the output layer with the loss and its gradient, the gradients of the second
+// and the first layer's pre-activations, and all weight and bias
+// gradients with their Adam updates.  Every sum runs over k in ascending order
+// by fused multiply-adds, one accumulator an output: Adam divides a gradient
+// by its own magnitude, so another order (split sums, the matrix cores) moves
+// a few weights by whole steps, although its gradients are as accurate.
+// The products are a few tens of MFLOP, too few waves to hide a load behind
+// another wave's work, so what binds is the chain of loads and dependent
+// multiply-adds.  A workgroup of two waves owns a 16 x 32 tile (256 of them for
+// 256 x 512 outputs, 2 x 2 a thread) and stages 64 k of both operands in LDS
+// while the next two pieces are on their way into registers (what a launch reads
+// was written by the launch before, on other XCDs, so it comes from beyond L2).  (Rows by scalar loads
+// and columns from L1 waited in every 16-long piece: 18 us for 256 x 512 x 512.)
 // ---------------------------------------------------------------------------
 
-constexpr int kTile = 64;
+constexpr int kTileM = 16, kTileN = 32, kTileK = 64, kTileThreads = 128;
 
-// C[M x N] (+)= op(A) op(B); op(A) is M x K (A stored K x M when ta), op(B)
-// is K x N (B stored N x K when tb).  64 x 64 tiles through LDS, 256 threads,
-// 4 x 4 outputs per thread.
-__global__ __launch_bounds__(256) void gemm_kernel(int M, int N, int K, const float* __restrict__ A, int lda,
-                                                   const float* __restrict__ B, int ldb, float* __restrict__ C,
-                                                   int ldc, int ta, int tb, int accumulate) {
-    __shared__ float As[16][kTile + 4];
-    __shared__ float Bs[16][kTile + 4];
-    const int tx = threadIdx.x % 16, ty = threadIdx.x / 16;
-    const int row0 = blockIdx.y * kTile, col0 = blockIdx.x * kTile;
-    float acc[4][4] = {};
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        for (int e = threadIdx.x; e < 16 * kTile; e += 256) {
-            const int kk = e / kTile, mm = e % kTile;
-            const int r = row0 + mm, k = k0 + kk;
-            float va = 0.f;
-            if (r < M && k < K) va = ta ? A[(size_t)k * lda + r] : A[(size_t)r * lda + k];
-            As[kk][mm] = va;
-            const int c = col0 + mm;
-            float vb = 0.f;
-            if (c < N && k < K) vb = tb ? B[(size_t)c * ldb + k] : B[(size_t)k * ldb + c];
-            Bs[kk][mm] = vb;
+struct TileLds {
+    float a[kTileK][kTileM + 2];
+    float b[kTileK][kTileN];
+};
+
+// The thread's four sums over k (ascending) of A(row, k) B(k, col) for rows
+// row0 + 2 p, + 1 and columns col0 + 2 q, + 1 (p = thread / 16, q = thread % 16).
+// A is row-major (K_MINOR: element (row, k) at A[row * lda + k], storage row
+// rows[row] where set) or its transpose (A[k * lda + row], storage row rows[k]).
+// B(k, col) is B[k * ldb + col].  Rows past M and columns past N repeat the last.
+template <bool K_MINOR>
+__device__ __forceinline__ void tile_products(TileLds& t, const float* __restrict__ A, int lda,
+                                              const int* __restrict__ rows, int row0, int M, int K,
+                                              const float* __restrict__ B, int ldb, int col0, int N,
+                                              float (&acc)[2][2]) {
+    constexpr int NA = kTileM * kTileK / kTileThreads, NB = kTileN * kTileK / kTileThreads;
+    const int tid = threadIdx.x;
+    // staging: A by k runs of 64 (K_MINOR) or rows of 16, B by rows of 32.  A
+    // load is a uniform base and the thread's own 32-bit offset, so that a
+    // piece's 24 addresses cost the vector unit nothing.
+    const int ak = K_MINOR ? tid & 63 : tid >> 4, ar = K_MINOR ? tid >> 6 : tid & 15;
+    const int bk = tid >> 5, bc = min(col0 + (tid & 31), N - 1);
+    uint32_t aoff[K_MINOR ? NA : 1];
+    if constexpr (K_MINOR) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int r = min(row0 + ar + 2 * i, M - 1);
+            aoff[i] = (uint32_t)(rows ? rows[r] - rows[0] : r) * (uint32_t)lda + (uint32_t)ak;
         }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
-        }
-        __syncthreads();
+    } else {
+        aoff[0] = (uint32_t)ak * (uint32_t)lda + (uint32_t)min(row0 + ar, M - 1);
     }
+    const float* a0 = K_MINOR && rows ? A + (size_t)rows[0] * lda : A;
+    const uint32_t boff = (uint32_t)bk * (uint32_t)ldb + (uint32_t)bc;
+    float ra[2][NA], rb[2][NB];
+    const auto load = [&](int k0, int h) {
+        if (k0 + kTileK <= K) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int r = row0 + ty * 4 + i, c = col0 + tx * 4 + j;
-            if (r < M && c < N) {
-                float* dst = C + (size_t)r * ldc + c;
-                *dst = accumulate ? *dst + acc[i][j] : acc[i][j];
+            for (int i = 0; i < NA; ++i) {
+                if constexpr (K_MINOR) ra[h][i] = (a0 + k0)[(int)aoff[i]];
+                else if (rows) ra[h][i] = A[(size_t)rows[k0 + ak + 8 * i] * lda + min(row0 + ar, M - 1)];
+                else ra[h][i] = (A + (size_t)(k0 + 8 * i) * lda)[aoff[0]];
             }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) rb[h][i] = (B + (size_t)(k0 + 4 * i) * ldb)[boff];
+        } else {
+#pragma unroll
+            for (int i = 0; i < NA; ++i) {
+                if constexpr (K_MINOR) {
+                    ra[h][i] = (a0 + (min(k0 + ak, K - 1) - ak))[(int)aoff[i]];
+                } else {
+                    const int k = min(k0 + ak + 8 * i, K - 1);
+                    ra[h][i] = A[(size_t)(rows ? rows[k] : k) * lda + min(row0 + ar, M - 1)];
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < NB; ++i) rb[h][i] = B[(size_t)min(k0 + bk + 4 * i, K - 1) * ldb + bc];
+        }
+    };
+    const int p = tid >> 4, q = tid & 15;
+    acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = 0.f;
+    const auto piece = [&](int k0, int h) {
+        if (k0) __syncthreads();
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            if constexpr (K_MINOR) t.a[ak][ar + 2 * i] = ra[h][i];
+            else t.a[ak + 8 * i][ar] = ra[h][i];
+        }
+#pragma unroll
+        for (int i = 0; i < NB; ++i) t.b[bk + 4 * i][tid & 31] = rb[h][i];
+        __syncthreads();
+        if (k0 + 2 * kTileK < K) load(k0 + 2 * kTileK, h);
+        const int n = min(kTileK, K - k0);
+        const auto step = [&](int k) {
+            const float2 x = *reinterpret_cast<const float2*>(&t.a[k][2 * p]);
+            const float2 y = *reinterpret_cast<const float2*>(&t.b[k][2 * q]);
+            acc[0][0] = fmaf(x.x, y.x, acc[0][0]);
+            acc[0][1] = fmaf(x.x, y.y, acc[0][1]);
+            acc[1][0] = fmaf(x.y, y.x, acc[1][0]);
+            acc[1][1] = fmaf(x.y, y.y, acc[1][1]);
+        };
+        if (n == kTileK) {
+            // 16 k read ahead of their sums (one wave a SIMD: each read waited
+            // for by itself costs the LDS latency, 3.3 us a piece of 64)
+            constexpr int U = 16;
+            float2 x[2][U], y[2][U];
+            const auto read = [&](int k, int h) {
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    x[h][u] = *reinterpret_cast<const float2*>(&t.a[k + u][2 * p]);
+                    y[h][u] = *reinterpret_cast<const float2*>(&t.b[k + u][2 * q]);
+                }
+            };
+            read(0, 0);
+#pragma unroll
+            for (int k = 0; k < kTileK; k += U) {
+                const int h = k / U % 2;
+                if (k + U < kTileK) read(k + U, 1 - h);
+                __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    acc[0][0] = fmaf(x[h][u].x, y[h][u].x, acc[0][0]);
+                    acc[0][1] = fmaf(x[h][u].x, y[h][u].y, acc[0][1]);
+                    acc[1][0] = fmaf(x[h][u].y, y[h][u].x, acc[1][0]);
+                    acc[1][1] = fmaf(x[h][u].y, y[h][u].y, acc[1][1]);
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        } else {
+            for (int k = 0; k < n; ++k) step(k);
+        }
+    };
+    load(0, 0);
+    if (kTileK < K) load(kTileK, 1);
+    for (int k0 = 0; k0 < K; k0 += 2 * kTileK) {
+        piece(k0, 0);
+        if (k0 + kTileK < K) piece(k0 + kTileK, 1);
+    }
+}
+
+// epi(row, col, value) for the thread's elements inside M x N
+template <class Epi>
+__device__ __forceinline__ void tile_out(const float (&acc)[2][2], int row0, int M, int col0, int N, Epi&& epi) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int r = row0 + 2 * (threadIdx.x >> 4) + i, c = col0 + 2 * (threadIdx.x & 15) + j;
+            if (r < M && c < N) epi(r, c, acc[i][j]);
         }
 }
 
-// Y = X + bias (per column), optionally ReLU.
-__global__ void bias_act_kernel(int M, int N, float* __restrict__ Y, const float* __restrict__ b, int relu) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)M * N) return;
-    float v = Y[i] + b[i % N];
-    Y[i] = relu ? fmaxf(v, 0.f) : v;
+// H = relu(X W + b), X's rows through `rows` where set.
+__global__ __launch_bounds__(kTileThreads) void layer_kernel(int M, int N, int K, const float* __restrict__ X,
+                                                             const int* __restrict__ rows, const float* __restrict__ W,
+                                                             const float* __restrict__ b, float* __restrict__ H) {
+    __shared__ TileLds t;
+    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
+    float acc[2][2];
+    tile_products<true>(t, X, K, rows, row0, M, K, W, N, col0, N, acc);
+    tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) { H[(size_t)r * N + c] = fmaxf(v + b[c], 0.f); });
 }
 
-// dY = 2 (Y - T) / (M N); loss partial sums per block.
-__global__ void mse_grad_kernel(int M, int N, const float* __restrict__ Y, const float* __restrict__ T,
-                                float* __restrict__ dY, float* __restrict__ loss_part) {
-    __shared__ float red[256];
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    float l = 0.f;
-    if (i < (long)M * N) {
-        const float d = Y[i] - T[i];
-        dY[i] = 2.f * d / ((float)M * N);
-        l = d * d / ((float)M * N);
-    }
-    red[threadIdx.x] = l;
+// dZ = (dY W^T) x (H > 0), from the transposed weights WT: the gradient
+// through a layer and its input's ReLU.
+__global__ __launch_bounds__(kTileThreads) void back_kernel(int M, int N, int K, const float* __restrict__ dY,
+                                                            const float* __restrict__ WT, const float* __restrict__ H,
+                                                            float* __restrict__ dZ) {
+    __shared__ TileLds t;
+    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
+    float acc[2][2];
+    tile_products<true>(t, dY, K, nullptr, row0, M, K, WT, N, col0, N, acc);
+    tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) {
+        const size_t i = (size_t)r * N + c;
+        dZ[i] = H[i] > 0.f ? v : 0.f;
+    });
+}
+
+// The output layer: Y = H W + b; with targets also dY = 2 (Y - T) / (M N) and
+// the workgroup's share of the loss.
+__global__ __launch_bounds__(kTileThreads) void output_kernel(int M, int N, int K, const float* __restrict__ H,
+                                                              const float* __restrict__ W, const float* __restrict__ b,
+                                                              const float* __restrict__ T, const int* __restrict__ rows,
+                                                              float* __restrict__ Y, float* __restrict__ dY,
+                                                              float* __restrict__ loss_part) {
+    __shared__ TileLds t;
+    __shared__ float wave_loss[2];
+    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
+    float acc[2][2], loss = 0.f;
+    tile_products<true>(t, H, K, nullptr, row0, M, K, W, N, col0, N, acc);
+    tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) {
+        const float y = v + b[c];
+        Y[(size_t)r * N + c] = y;
+        if (T) {
+            const float d = y - T[(size_t)(rows ? rows[r] : r) * N + c];
+            dY[(size_t)r * N + c] = 2.f * d / ((float)M * N);
+            loss += d * d / ((float)M * N);
+        }
+    });
+    if (!T) return;
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) loss += __shfl_xor(loss, d, 64);
+    if ((threadIdx.x & 63) == 0) wave_loss[threadIdx.x >> 6] = loss;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-        __syncthreads();
+    if (threadIdx.x == 0) loss_part[blockIdx.x] = wave_loss[0] + wave_loss[1];
+}
+
+// dZ = (dY W^T) x (H > 0) for the few outputs of the last layer (M x n_out by
+// n_out x N, W stored N x n_out): eight rows and 64 units a wave, dY uniform.
+__global__ __launch_bounds__(64) void output_back_kernel(int M, int N, int n_out, const float* __restrict__ dY,
+                                                         const float* __restrict__ W, const float* __restrict__ H,
+                                                         float* __restrict__ dZ) {
+    constexpr int R = 8;
+    const int nx = (N + 63) / 64, row0 = blockIdx.x / nx * R, c = blockIdx.x % nx * 64 + threadIdx.x;
+    if (c >= N) return;
+    float z[R] = {};
+#pragma unroll 4
+    for (int o = 0; o < n_out; ++o) {
+        const float w = W[(size_t)c * n_out + o];
+#pragma unroll
+        for (int r = 0; r < R; ++r) z[r] = fmaf(dY[(size_t)min(row0 + r, M - 1) * n_out + o], w, z[r]);
     }
-    if (threadIdx.x == 0) loss_part[blockIdx.x] = red[0];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+        if (row0 + r < M) {
+            const size_t i = (size_t)(row0 + r) * N + c;
+            dZ[i] = H[i] > 0.f ? z[r] : 0.f;
+        }
 }
 
-// dZ *= (H > 0): the ReLU gradient through the stored activation.
-__global__ void relu_grad_kernel(long n, const float* __restrict__ H, float* __restrict__ dZ) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !(H[i] > 0.f)) dZ[i] = 0.f;
+// WT = W^T (n x n)
+__global__ __launch_bounds__(256) void transpose_kernel(int n, const float* __restrict__ W, float* __restrict__ WT) {
+    __shared__ float t[32][33];
+    const int nb = (n + 31) / 32, r0 = blockIdx.x / nb * 32, c0 = blockIdx.x % nb * 32;
+    const int x = threadIdx.x & 31, y = threadIdx.x >> 5;
+    for (int i = y; i < 32; i += 8)
+        if (r0 + i < n && c0 + x < n) t[i][x] = W[(size_t)(r0 + i) * n + c0 + x];
+    __syncthreads();
+    for (int i = y; i < 32; i += 8)
+        if (c0 + i < n && r0 + x < n) WT[(size_t)(c0 + i) * n + r0 + x] = t[x][i];
 }
 
-// db[j] = sum_i dZ[i][j]
-__global__ void col_sum_kernel(int M, int N, const float* __restrict__ dZ, float* __restrict__ db) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    if (j >= N) return;
+struct Adam {
+    float lr, b1, b2, eps, c1, c2;
+    float *w, *m, *v;      // null w: gradients only
+};
+__device__ __forceinline__ void put_gradient(const Adam& a, float* __restrict__ g, size_t i, float gi) {
+    if (!a.w) {
+        g[i] = gi;
+        return;
+    }
+    const float mi = a.b1 * a.m[i] + (1.f - a.b1) * gi;
+    const float vi = a.b2 * a.v[i] + (1.f - a.b2) * gi * gi;
+    a.m[i] = mi;
+    a.v[i] = vi;
+    a.w[i] -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+}
+
+// Every weight gradient A^T dZ and bias gradient (column sums of dZ) of the
+// step, and the Adam updates (and W2's transpose kept up with them).
+// Workgroups: the layers' tiles in turn, then kTileThreads bias columns each.
+struct GradArgs {
+    int n_in, n_hid, n_out, M;
+    int tile[3], bias[3];              // first workgroup of each layer's tiles, of its biases
+    size_t w_off[3], b_off[3];
+};
+__global__ __launch_bounds__(kTileThreads) void gradient_kernel(
+    GradArgs a, const float* __restrict__ X, const int* __restrict__ rows, const float* __restrict__ H1,
+    const float* __restrict__ H2, const float* __restrict__ dZ1, const float* __restrict__ dZ2,
+    const float* __restrict__ dY, Adam adam, float* __restrict__ g, float* __restrict__ W2T) {
+    __shared__ TileLds t;
+    const int blk = blockIdx.x;
+    if (blk < a.bias[0]) {
+        const int l = blk >= a.tile[2] ? 2 : blk >= a.tile[1] ? 1 : 0;
+        const float* A = l == 0 ? X : l == 1 ? H1 : H2;
+        const float* D = l == 0 ? dZ1 : l == 1 ? dZ2 : dY;
+        const int n_a = l == 0 ? a.n_in : a.n_hid, n_d = l == 2 ? a.n_out : a.n_hid;
+        const int nx = (n_d + kTileN - 1) / kTileN, tile = blk - a.tile[l];
+        const int row0 = tile / nx * kTileM, col0 = tile % nx * kTileN;
+        float acc[2][2];
+        tile_products<false>(t, A, n_a, l == 0 ? rows : nullptr, row0, n_a, a.M, D, n_d, col0, n_d, acc);
+        tile_out(acc, row0, n_a, col0, n_d, [&](int r, int c, float v) {
+            const size_t i = a.w_off[l] + (size_t)r * n_d + c;
+            put_gradient(adam, g, i, v);
+            if (l == 1 && adam.w) W2T[(size_t)c * n_d + r] = adam.w[i];
+        });
+        return;
+    }
+    const int l = blk >= a.bias[2] ? 2 : blk >= a.bias[1] ? 1 : 0;
+    const float* D = l == 0 ? dZ1 : l == 1 ? dZ2 : dY;
+    const int n_d = l == 2 ? a.n_out : a.n_hid, j = (blk - a.bias[l]) * kTileThreads + threadIdx.x;
+    if (j >= n_d) return;
     float s = 0.f;
-    for (int i = 0; i < M; ++i) s += dZ[(size_t)i * N + j];
-    db[j] = s;
-}
-
-__global__ void adam_kernel(long n, float* __restrict__ w, const float* __restrict__ g, float* __restrict__ m,
-                            float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
-    const float mi = b1 * m[i] + (1.f - b1) * gi;
-    const float vi = b2 * v[i] + (1.f - b2) * gi * gi;
-    m[i] = mi;
-    v[i] = vi;
-    w[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-}
-
-__global__ void gather_rows_kernel(int rows, int cols, const int* __restrict__ idx, const float* __restrict__ src,
-                                   float* __restrict__ dst) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long)rows * cols) return;
-    const int r = i / cols, c = i % cols;
-    dst[i] = src[(size_t)idx[r] * cols + c];
+    int i = 0;
+    for (; i + 32 <= a.M; i += 32) {
+        float x[32];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) x[u] = D[(size_t)(i + u) * n_d + j];
+#pragma unroll
+        for (int u = 0; u < 32; ++u) s += x[u];
+    }
+    for (; i < a.M; ++i) s += D[(size_t)i * n_d + j];
+    put_gradient(adam, g, a.b_off[l] + j, s);
 }
 
 }  // namespace
@@ -370,9 +558,11 @@ struct phylo_mlp {
     float* d_dh2 = nullptr;
     float* d_dy = nullptr;
     float* d_loss = nullptr;
+    float* d_w2t = nullptr;     // W2 transposed
     int* d_idx = nullptr;
     float* d_data_x = nullptr;  // training set
     float* d_data_t = nullptr;
+    size_t data_x_cap = 0, data_t_cap = 0, loss_cap = 0, idx_cap = 0;
     int n_data = 0;
     long step = 0;
 };
@@ -389,14 +579,6 @@ int mfail(phylo_mlp* p, int code, const std::string& m) {
         if (e_ != hipSuccess) return mfail((p), PHYLO_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
 
-void gemm(phylo_mlp* p, int M, int N, int K, const float* A, int lda, const float* B, int ldb, float* C, int ldc,
-          int ta, int tb, int acc) {
-    dim3 grid((N + kTile - 1) / kTile, (M + kTile - 1) / kTile);
-    hipLaunchKernelGGL(gemm_kernel, grid, dim3(256), 0, p->stream, M, N, K, A, lda, B, ldb, C, ldc, ta, tb, acc);
-}
-
-inline unsigned nblk(long n, int t = 256) { return (unsigned)((n + t - 1) / t); }
-
 // Parameter views inside the flat buffer.
 struct Views {
     float *W1, *b1, *W2, *b2, *W3, *b3;
@@ -412,46 +594,69 @@ Views views(phylo_mlp* p, float* base) {
     return v;
 }
 
-void forward(phylo_mlp* p, int B, const float* X) {
-    Views w = views(p, p->d_w);
-    gemm(p, B, p->n_hid, p->n_in, X, p->n_in, w.W1, p->n_hid, p->d_h1, p->n_hid, 0, 0, 0);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((long)B * p->n_hid)), dim3(256), 0, p->stream, B, p->n_hid, p->d_h1, w.b1, 1);
-    gemm(p, B, p->n_hid, p->n_hid, p->d_h1, p->n_hid, w.W2, p->n_hid, p->d_h2, p->n_hid, 0, 0, 0);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((long)B * p->n_hid)), dim3(256), 0, p->stream, B, p->n_hid, p->d_h2, w.b2, 1);
-    gemm(p, B, p->n_out, p->n_hid, p->d_h2, p->n_hid, w.W3, p->n_out, p->d_y, p->n_out, 0, 0, 0);
-    hipLaunchKernelGGL(bias_act_kernel, dim3(nblk((long)B * p->n_out)), dim3(256), 0, p->stream, B, p->n_out, p->d_y, w.b3, 0);
+unsigned tiles(int n, int t) { return (unsigned)((n + t - 1) / t); }
+
+// Workgroups of the output layer, each with a part of the loss.
+unsigned loss_parts(const phylo_mlp* p, int B) { return tiles(B, kTileM) * tiles(p->n_out, kTileN); }
+
+// One pass over B rows of X (through `rows` where set): the forward layers
+// and the output; with targets also the loss parts and the gradients of the
+// pre-activations (d_dy, d_dh2, d_dh1; d_w2t holds W2's transpose).
+void pass(phylo_mlp* p, int B, const float* X, const int* rows, const float* T, float* loss) {
+    const Views w = views(p, p->d_w);
+    const int H = p->n_hid;
+    const dim3 grid(tiles(H, kTileN) * tiles(B, kTileM)), block(kTileThreads);
+    hipLaunchKernelGGL(layer_kernel, grid, block, 0, p->stream, B, H, p->n_in, X, rows, w.W1, w.b1, p->d_h1);
+    hipLaunchKernelGGL(layer_kernel, grid, block, 0, p->stream, B, H, H, p->d_h1, nullptr, w.W2, w.b2, p->d_h2);
+    hipLaunchKernelGGL(output_kernel, dim3(loss_parts(p, B)), block, 0, p->stream, B, p->n_out, H, p->d_h2, w.W3, w.b3, T,
+                       rows, p->d_y, p->d_dy, loss);
+    if (!T) return;
+    hipLaunchKernelGGL(output_back_kernel, dim3(tiles(H, 64) * tiles(B, 8)), dim3(64), 0, p->stream, B, H, p->n_out, p->d_dy,
+                       w.W3, p->d_h2, p->d_dh2);
+    hipLaunchKernelGGL(back_kernel, grid, block, 0, p->stream, B, H, H, p->d_dh2, p->d_w2t, p->d_h1, p->d_dh1);
 }
 
-// Gradient of the mean squared error into d_g; loss partials in d_loss.
-void backward(phylo_mlp* p, int B, const float* X, const float* T) {
-    Views w = views(p, p->d_w), g = views(p, p->d_g);
-    const long ny = (long)B * p->n_out;
-    hipLaunchKernelGGL(mse_grad_kernel, dim3(nblk(ny)), dim3(256), 0, p->stream, B, p->n_out, p->d_y, T, p->d_dy, p->d_loss);
-    // layer 3
-    gemm(p, p->n_hid, p->n_out, B, p->d_h2, p->n_hid, p->d_dy, p->n_out, g.W3, p->n_out, 1, 0, 0);
-    hipLaunchKernelGGL(col_sum_kernel, dim3(nblk(p->n_out)), dim3(256), 0, p->stream, B, p->n_out, p->d_dy, g.b3);
-    gemm(p, B, p->n_hid, p->n_out, p->d_dy, p->n_out, w.W3, p->n_out, p->d_dh2, p->n_hid, 0, 1, 0);
-    hipLaunchKernelGGL(relu_grad_kernel, dim3(nblk((long)B * p->n_hid)), dim3(256), 0, p->stream, (long)B * p->n_hid, p->d_h2, p->d_dh2);
-    // layer 2
-    gemm(p, p->n_hid, p->n_hid, B, p->d_h1, p->n_hid, p->d_dh2, p->n_hid, g.W2, p->n_hid, 1, 0, 0);
-    hipLaunchKernelGGL(col_sum_kernel, dim3(nblk(p->n_hid)), dim3(256), 0, p->stream, B, p->n_hid, p->d_dh2, g.b2);
-    gemm(p, B, p->n_hid, p->n_hid, p->d_dh2, p->n_hid, w.W2, p->n_hid, p->d_dh1, p->n_hid, 0, 1, 0);
-    hipLaunchKernelGGL(relu_grad_kernel, dim3(nblk((long)B * p->n_hid)), dim3(256), 0, p->stream, (long)B * p->n_hid, p->d_h1, p->d_dh1);
-    // layer 1
-    gemm(p, p->n_in, p->n_hid, B, X, p->n_in, p->d_dh1, p->n_hid, g.W1, p->n_hid, 1, 0, 0);
-    hipLaunchKernelGGL(col_sum_kernel, dim3(nblk(p->n_hid)), dim3(256), 0, p->stream, B, p->n_hid, p->d_dh1, g.b1);
+void transpose_w2(phylo_mlp* p) {
+    hipLaunchKernelGGL(transpose_kernel, dim3(tiles(p->n_hid, 32) * tiles(p->n_hid, 32)), dim3(256), 0, p->stream, p->n_hid,
+                       views(p, p->d_w).W2, p->d_w2t);
 }
 
-float read_loss(phylo_mlp* p, int B) {
-    const long ny = (long)B * p->n_out;
-    std::vector<float> part(nblk(ny));
-    if (hipMemcpyAsync(part.data(), p->d_loss, part.size() * sizeof(float), hipMemcpyDeviceToHost, p->stream) !=
-            hipSuccess ||
-        hipStreamSynchronize(p->stream) != hipSuccess)
-        return NAN;
+// The step's gradients: into d_g (adam.w null) or straight into the weights.
+void gradients(phylo_mlp* p, int B, const float* X, const int* rows, const Adam& adam) {
+    const Views o = views(p, p->d_w);
+    const auto off = [&](const float* q) { return (size_t)(q - p->d_w); };
+    GradArgs a{p->n_in, p->n_hid, p->n_out, B, {}, {}, {off(o.W1), off(o.W2), off(o.W3)}, {off(o.b1), off(o.b2), off(o.b3)}};
+    const int n_a[3] = {p->n_in, p->n_hid, p->n_hid}, n_d[3] = {p->n_hid, p->n_hid, p->n_out};
+    int n = 0;
+    for (int l = 0; l < 3; ++l) {
+        a.tile[l] = n;
+        n += tiles(n_a[l], kTileM) * tiles(n_d[l], kTileN);
+    }
+    for (int l = 0; l < 3; ++l) {
+        a.bias[l] = n;
+        n += tiles(n_d[l], kTileThreads);
+    }
+    hipLaunchKernelGGL(gradient_kernel, dim3(n), dim3(kTileThreads), 0, p->stream, a, X, rows, p->d_h1, p->d_h2, p->d_dh1, p->d_dh2,
+                       p->d_dy, adam, p->d_g, p->d_w2t);
+}
+
+// The loss of a step from its parts.
+float sum_loss(const float* part, unsigned n) {
     double s = 0.0;
-    for (float x : part) s += x;
+    for (unsigned i = 0; i < n; ++i) s += part[i];
     return (float)s;
+}
+
+// Grows a device buffer to n elements.
+template <typename T>
+hipError_t grow(T*& d, size_t& have, size_t n) {
+    if (n <= have) return hipSuccess;
+    if (d) (void)hipFree(d);
+    d = nullptr;
+    have = 0;
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), n * sizeof(T));
+    if (e == hipSuccess) have = n;
+    return e;
 }
 
 }  // namespace
@@ -552,7 +757,7 @@ int phylo_mlp_create(int device, int n_in, int n_hidden, int n_out, int max_batc
         !alloc(p->d_v, p->n_params) || !alloc(p->d_x, B * n_in) || !alloc(p->d_t, B * n_out) ||
         !alloc(p->d_h1, B * n_hidden) || !alloc(p->d_h2, B * n_hidden) || !alloc(p->d_y, B * n_out) ||
         !alloc(p->d_dh1, B * n_hidden) || !alloc(p->d_dh2, B * n_hidden) || !alloc(p->d_dy, B * n_out) ||
-        !alloc(p->d_loss, nblk((long)B * n_out)) || !alloc(p->d_idx, B)) {
+        !alloc(p->d_w2t, (size_t)n_hidden * n_hidden) || grow(p->d_loss, p->loss_cap, loss_parts(p, max_batch)) != hipSuccess) {
         phylo_mlp_destroy(p);
         return PHYLO_ERR_HIP;
     }
@@ -600,7 +805,7 @@ int phylo_mlp_forward(phylo_mlp* p, int batch, const float* x, float* y) {
         const int B = std::min(p->max_batch, batch - b0);
         MCHK(p, hipMemcpyAsync(p->d_x, x + (size_t)b0 * p->n_in, (size_t)B * p->n_in * sizeof(float),
                                hipMemcpyHostToDevice, p->stream));
-        forward(p, B, p->d_x);
+        pass(p, B, p->d_x, nullptr, nullptr, nullptr);
         MCHK(p, hipGetLastError());
         MCHK(p, hipMemcpyAsync(y + (size_t)b0 * p->n_out, p->d_y, (size_t)B * p->n_out * sizeof(float),
                                hipMemcpyDeviceToHost, p->stream));
@@ -614,24 +819,24 @@ int phylo_mlp_grad(phylo_mlp* p, int batch, const float* x, const float* t, floa
     MCHK(p, hipSetDevice(p->device));
     MCHK(p, hipMemcpyAsync(p->d_x, x, (size_t)batch * p->n_in * sizeof(float), hipMemcpyHostToDevice, p->stream));
     MCHK(p, hipMemcpyAsync(p->d_t, t, (size_t)batch * p->n_out * sizeof(float), hipMemcpyHostToDevice, p->stream));
-    forward(p, batch, p->d_x);
-    backward(p, batch, p->d_x, p->d_t);
+    transpose_w2(p);
+    pass(p, batch, p->d_x, nullptr, p->d_t, p->d_loss);
+    gradients(p, batch, p->d_x, nullptr, Adam{});
     MCHK(p, hipGetLastError());
+    std::vector<float> part(loss_parts(p, batch));
+    if (loss) MCHK(p, hipMemcpyAsync(part.data(), p->d_loss, part.size() * sizeof(float), hipMemcpyDeviceToHost, p->stream));
     if (grad) MCHK(p, hipMemcpyAsync(grad, p->d_g, p->n_params * sizeof(float), hipMemcpyDeviceToHost, p->stream));
     MCHK(p, hipStreamSynchronize(p->stream));
-    if (loss) *loss = read_loss(p, batch);
+    if (loss) *loss = sum_loss(part.data(), (unsigned)part.size());
     return PHYLO_OK;
 }
 
 int phylo_mlp_set_data(phylo_mlp* p, int n, const float* x, const float* t) {
     if (!p || n < 1 || !x || !t) return PHYLO_ERR_ARG;
     MCHK(p, hipSetDevice(p->device));
-    if (p->d_data_x) (void)hipFree(p->d_data_x);
-    if (p->d_data_t) (void)hipFree(p->d_data_t);
-    p->d_data_x = nullptr;
-    p->d_data_t = nullptr;
-    MCHK(p, hipMalloc(reinterpret_cast<void**>(&p->d_data_x), (size_t)n * p->n_in * sizeof(float)));
-    MCHK(p, hipMalloc(reinterpret_cast<void**>(&p->d_data_t), (size_t)n * p->n_out * sizeof(float)));
+    p->n_data = 0;
+    MCHK(p, grow(p->d_data_x, p->data_x_cap, (size_t)n * p->n_in));
+    MCHK(p, grow(p->d_data_t, p->data_t_cap, (size_t)n * p->n_out));
     MCHK(p, hipMemcpy(p->d_data_x, x, (size_t)n * p->n_in * sizeof(float), hipMemcpyHostToDevice));
     MCHK(p, hipMemcpy(p->d_data_t, t, (size_t)n * p->n_out * sizeof(float), hipMemcpyHostToDevice));
     p->n_data = n;
@@ -640,33 +845,38 @@ int phylo_mlp_set_data(phylo_mlp* p, int n, const float* x, const float* t) {
 
 // Epochs of minibatch Adam over the stored training set (shuffled per epoch).
 int phylo_mlp_train(phylo_mlp* p, int epochs, int batch, float lr, uint64_t seed, float* loss_per_epoch) {
-    if (!p || epochs < 1 || batch < 1 || batch > p->max_batch || !p->d_data_x) return PHYLO_ERR_ARG;
+    if (!p || epochs < 1 || batch < 1 || batch > p->max_batch || !p->d_data_x || p->n_data < 1)
+        return PHYLO_ERR_ARG;
     MCHK(p, hipSetDevice(p->device));
     std::mt19937_64 rng(seed);
     std::vector<int> perm(p->n_data);
     const float b1 = 0.9f, b2 = 0.999f;
+    // an epoch is enqueued whole: the shuffled order goes over once, the steps'
+    // loss parts come back together
+    const unsigned n_part = loss_parts(p, batch);
+    const int steps = p->n_data / batch;
+    MCHK(p, grow(p->d_idx, p->idx_cap, (size_t)p->n_data));
+    MCHK(p, grow(p->d_loss, p->loss_cap, (size_t)std::max(1, steps) * n_part));
+    std::vector<float> part((size_t)steps * n_part);
+    transpose_w2(p);      // (kept up by the steps)
     for (int ep = 0; ep < epochs; ++ep) {
         for (int i = 0; i < p->n_data; ++i) perm[i] = i;
         std::shuffle(perm.begin(), perm.end(), rng);
-        double lsum = 0.0;
-        int nb = 0;
-        for (int b0 = 0; b0 + batch <= p->n_data; b0 += batch) {
-            MCHK(p, hipMemcpyAsync(p->d_idx, perm.data() + b0, batch * sizeof(int), hipMemcpyHostToDevice, p->stream));
-            hipLaunchKernelGGL(gather_rows_kernel, dim3(nblk((long)batch * p->n_in)), dim3(256), 0, p->stream, batch,
-                               p->n_in, p->d_idx, p->d_data_x, p->d_x);
-            hipLaunchKernelGGL(gather_rows_kernel, dim3(nblk((long)batch * p->n_out)), dim3(256), 0, p->stream, batch,
-                               p->n_out, p->d_idx, p->d_data_t, p->d_t);
-            forward(p, batch, p->d_x);
-            backward(p, batch, p->d_x, p->d_t);
+        MCHK(p, hipMemcpyAsync(p->d_idx, perm.data(), perm.size() * sizeof(int), hipMemcpyHostToDevice, p->stream));
+        for (int k = 0; k < steps; ++k) {
+            const int* rows = p->d_idx + (size_t)k * batch;
+            pass(p, batch, p->d_data_x, rows, p->d_data_t, p->d_loss + (size_t)k * n_part);
             ++p->step;
             const float c1 = 1.f - std::pow(b1, (float)p->step), c2 = 1.f - std::pow(b2, (float)p->step);
-            hipLaunchKernelGGL(adam_kernel, dim3(nblk(p->n_params)), dim3(256), 0, p->stream, p->n_params, p->d_w,
-                               p->d_g, p->d_m, p->d_v, lr, b1, b2, 1e-8f, c1, c2);
+            gradients(p, batch, p->d_data_x, rows, Adam{lr, b1, b2, 1e-8f, c1, c2, p->d_w, p->d_m, p->d_v});
             MCHK(p, hipGetLastError());
-            lsum += read_loss(p, batch);   // synchronises the stream (perm buffer reuse is safe)
-            ++nb;
         }
-        if (loss_per_epoch) loss_per_epoch[ep] = nb ? (float)(lsum / nb) : NAN;
+        if (steps)
+            MCHK(p, hipMemcpyAsync(part.data(), p->d_loss, part.size() * sizeof(float), hipMemcpyDeviceToHost, p->stream));
+        MCHK(p, hipStreamSynchronize(p->stream));
+        double lsum = 0.0;
+        for (int k = 0; k < steps; ++k) lsum += sum_loss(part.data() + (size_t)k * n_part, n_part);
+        if (loss_per_epoch) loss_per_epoch[ep] = steps ? (float)(lsum / steps) : NAN;
     }
     return PHYLO_OK;
 }
@@ -676,7 +886,7 @@ void phylo_mlp_destroy(phylo_mlp* p) {
     (void)hipSetDevice(p->device);
     if (p->stream) (void)hipStreamSynchronize(p->stream);
     void* bufs[] = {p->d_w, p->d_g, p->d_m, p->d_v, p->d_x, p->d_t, p->d_h1, p->d_h2, p->d_y,
-                    p->d_dh1, p->d_dh2, p->d_dy, p->d_loss, p->d_idx, p->d_data_x, p->d_data_t};
+                    p->d_dh1, p->d_dh2, p->d_dy, p->d_loss, p->d_w2t, p->d_idx, p->d_data_x, p->d_data_t};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (p->stream) (void)hipStreamDestroy(p->stream);
