@@ -10,6 +10,7 @@
 #include <cmath>
 #include <cstdint>
 #include <cstring>
+#include <memory>
 #include <random>
 #include <string>
 #include <vector>
@@ -24,7 +25,6 @@ constexpr int kMaxSimTaxa = 32;
 constexpr int kMaxSimNodes = 2 * kMaxSimTaxa - 1;
 constexpr int kMaxSimCat = 8;
 constexpr int kFeat = 256;
-constexpr unsigned char kGap = 255;
 
 __device__ inline uint64_t mix64(uint64_t z) {
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
@@ -39,72 +39,68 @@ __device__ inline float urand(uint64_t seed, uint64_t a, uint64_t b, uint64_t c)
 
 // One workgroup per alignment.  Per-alignment inputs (eig = V[16], Vinv[16],
 // lam[4]; pi[4]; cat_rates[C]) give P(t) = V exp(lam r t) Vinv in LDS as
-// cumulative rows; each thread simulates one site of a 256-site chunk down
-// the tree in preorder, then the chunk's tip states update the features.
+// cumulative rows; walk holds the nodes in preorder as node | parent << 8.
+// Each thread simulates one site of a 256-site chunk down the tree; a tip's
+// states leave as four ballot words a wave (one bit a site and state), so the
+// joint state counts of a pair of taxa are 16 popcounts of ANDed words per 64
+// sites.  (A byte a site, counted site by site into an array indexed at run
+// time, which lies in scratch memory, took 1.42 ms for 512 alignments of 32
+// taxa x 2,000 sites.)  What is left is the generator: three 64-bit mixes a
+// draw, 94 draws a site.
 __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
-    int n_taxa, int n_sites, int n_cat, const int* __restrict__ left, const int* __restrict__ right,
-    const int* __restrict__ roots, const double* __restrict__ blen, const double* __restrict__ eig,
-    const double* __restrict__ pi_all, const double* __restrict__ cat_all, float gap_frac, uint64_t seed,
-    float* __restrict__ feat, uint32_t* __restrict__ masks_out) {
+    int n_taxa, int n_sites, int n_cat, const int* __restrict__ walk, const double* __restrict__ blen,
+    const double* __restrict__ eig, const double* __restrict__ pi_all, const double* __restrict__ cat_all,
+    float gap_frac, uint64_t seed, float* __restrict__ feat, uint32_t* __restrict__ masks_out) {
     const int a = blockIdx.x;
-    const int tid = threadIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int n_nodes = 2 * n_taxa - 1;
-    __shared__ float cumP[kMaxSimNodes][kMaxSimCat][16];
-    __shared__ unsigned char st[kMaxSimNodes][kSimThreads];
-    __shared__ int pre[kMaxSimNodes];
-    __shared__ int par[kMaxSimNodes];
+    extern __shared__ __align__(16) float cumP[];       // [n_nodes][n_cat][4][4]
+    __shared__ unsigned char st[kMaxSimNodes - kMaxSimTaxa][kSimThreads];   // inner nodes' states
+    __shared__ __align__(16) uint64_t tip[kMaxSimTaxa][kSimThreads / 64][4];    // [taxon][wave][state]
     __shared__ float cum_pi[4];
     __shared__ int h_site[4 + 32 + 32];
     __shared__ float h_pair[16 + 32 + 32 + 32 + 8];
     __shared__ int base[4];
-    __shared__ int gaps_total;
     __shared__ int invariant;
-    const int* L = left + (size_t)a * n_nodes;
-    const int* R = right + (size_t)a * n_nodes;
     const double* bl = blen + (size_t)a * n_nodes;
     const double* V = eig + (size_t)a * 36;
     const double* Vi = V + 16;
     const double* lam = V + 32;
+    walk += (size_t)a * n_nodes;
     for (int i = tid; i < 4 + 32 + 32; i += kSimThreads) h_site[i] = 0;
     for (int i = tid; i < 16 + 32 + 32 + 32 + 8; i += kSimThreads) h_pair[i] = 0.f;
     if (tid < 4) base[tid] = 0;
     if (tid == 0) {
-        gaps_total = 0;
         invariant = 0;
-        // preorder by an explicit stack, parents recorded
-        int stack[kMaxSimNodes];
-        int sp = 0, k = 0;
-        stack[sp++] = roots[a];
-        par[roots[a]] = -1;
-        while (sp) {
-            const int v = stack[--sp];
-            pre[k++] = v;
-            if (R[v] >= 0) { par[R[v]] = v; stack[sp++] = R[v]; }
-            if (L[v] >= 0) { par[L[v]] = v; stack[sp++] = L[v]; }
-        }
         double c = 0.0;
         for (int i = 0; i < 4; ++i) { c += pi_all[(size_t)a * 4 + i]; cum_pi[i] = (float)c; }
         cum_pi[3] = 1.0f;
     }
-    // cumulative P rows: cumP[v][c][i*4 + j] = sum_{j' <= j} P_ij'
+    // cumulative P rows: cumP[(v, c)][i][j] = sum_{j' <= j} P_ij'
     for (int e = tid; e < n_nodes * n_cat * 4; e += kSimThreads) {
         const int i = e % 4, c = (e / 4) % n_cat, v = e / (4 * n_cat);
         const double t = bl[v] * cat_all[(size_t)a * n_cat + c];
+        float* row = cumP + (size_t)e * 4;
         double acc = 0.0;
+        float r[4];
+#pragma unroll
         for (int j = 0; j < 4; ++j) {
             double p = 0.0;
+#pragma unroll
             for (int k = 0; k < 4; ++k) p += V[i * 4 + k] * exp(lam[k] * t) * Vi[k * 4 + j];
             acc += p > 0.0 ? p : 0.0;
-            cumP[v][c][i * 4 + j] = (float)acc;
+            r[j] = (float)acc;
         }
-        const float tot = cumP[v][c][i * 4 + 3];
-        for (int j = 0; j < 4; ++j) cumP[v][c][i * 4 + j] /= tot;
-        cumP[v][c][i * 4 + 3] = 1.0f;
+        const float tot = r[3];
+#pragma unroll
+        for (int j = 0; j < 3; ++j) row[j] = r[j] / tot;
+        row[3] = 1.0f;
     }
     __syncthreads();
     // pair ownership: thread owns pairs p = tid, tid + 256 (496 pairs for 32 taxa)
     const int n_pairs = n_taxa * (n_taxa - 1) / 2;
     int pa[2] = {-1, -1}, pb[2] = {-1, -1};
+#pragma unroll
     for (int q = 0; q < 2; ++q) {
         int p = tid + q * kSimThreads;
         if (p >= n_pairs) continue;
@@ -114,47 +110,51 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         pb[q] = i + 1 + p;
     }
     int joint[2][16];
+#pragma unroll
     for (int q = 0; q < 2; ++q)
+#pragma unroll
         for (int c = 0; c < 16; ++c) joint[q][c] = 0;
-    int basec[4] = {0, 0, 0, 0}, gapc = 0;
+    int base_count = 0;      // threads < 4 n_taxa: state tid % 4 of taxon tid / 4
     for (int s0 = 0; s0 < n_sites; s0 += kSimThreads) {
         const int s = s0 + tid;
-        if (s < n_sites) {
-            const int cat = n_cat > 1 ? min(n_cat - 1, (int)(urand(seed, a, s, 1u << 20) * n_cat)) : 0;
-            const float u = urand(seed, a, s, (1u << 20) + 1);
-            int rs = 3;
-            for (int j = 0; j < 4; ++j)
-                if (u < cum_pi[j]) { rs = j; break; }
-            st[pre[0]][tid] = (unsigned char)rs;
-            for (int k = 1; k < n_nodes; ++k) {
-                const int v = pre[k];
-                const int anc = st[par[v]][tid];
-                const float r = urand(seed, a, s, (uint64_t)v);
-                const float* row = &cumP[v][cat][anc * 4];
-                int x = 3;
-                for (int j = 0; j < 4; ++j)
-                    if (r < row[j]) { x = j; break; }
-                st[v][tid] = (unsigned char)x;
+        const bool live = s < n_sites;      // (the other lanes draw too: the ballots need every lane)
+        const int cat = n_cat > 1 ? min(n_cat - 1, (int)(urand(seed, a, s, 1u << 20) * n_cat)) : 0;
+        const float u = urand(seed, a, s, (1u << 20) + 1);
+        // the first state whose cumulative value exceeds u (3 at the end)
+        int rs = !(u < cum_pi[0]);
+        rs += rs == 1 && !(u < cum_pi[1]);
+        rs += rs == 2 && !(u < cum_pi[2]);
+        st[walk[0] - n_taxa][tid] = (unsigned char)rs;
+        uint32_t cnt = 0;        // tips per state, a byte each
+        for (int k = 1; k < n_nodes; ++k) {
+            const int w = walk[k], v = w & 255;
+            const int anc = st[(w >> 8) - n_taxa][tid];
+            const float r = urand(seed, a, s, (uint64_t)v);
+            const float4 row = *reinterpret_cast<const float4*>(cumP + (((size_t)v * n_cat + cat) * 4 + anc) * 4);
+            int x = !(r < row.x);
+            x += x == 1 && !(r < row.y);
+            x += x == 2 && !(r < row.z);
+            if (v >= n_taxa) {
+                st[v - n_taxa][tid] = (unsigned char)x;
+                continue;
             }
-            // gaps at the tips, site summaries
-            int cnt[4] = {0, 0, 0, 0}, n_ok = 0;
-            for (int t = 0; t < n_taxa; ++t) {
-                if (gap_frac > 0.f && urand(seed, a, s, (2u << 20) + t) < gap_frac) {
-                    st[t][tid] = kGap;
-                    ++gapc;
-                } else {
-                    ++cnt[st[t][tid]];
-                    ++basec[st[t][tid]];
-                    ++n_ok;
-                }
-                if (masks_out)
-                    masks_out[((size_t)a * n_taxa + t) * n_sites + s] = st[t][tid] == kGap ? 15u : (1u << st[t][tid]);
-            }
-            int distinct = 0, mx = 0, sq = 0;
+            // a tip: gaps, its states' words
+            const bool ok = live && !(gap_frac > 0.f && urand(seed, a, s, (2u << 20) + v) < gap_frac);
+            cnt += ok ? 1u << (8 * x) : 0u;
+            const uint64_t m0 = __ballot(ok && x == 0), m1 = __ballot(ok && x == 1), m2 = __ballot(ok && x == 2),
+                           m3 = __ballot(ok && x == 3);
+            if (lane < 4) tip[v][wave][lane] = lane == 0 ? m0 : lane == 1 ? m1 : lane == 2 ? m2 : m3;
+            if (masks_out && live) masks_out[((size_t)a * n_taxa + v) * n_sites + s] = ok ? 1u << x : 15u;
+        }
+        if (live) {
+            int distinct = 0, mx = 0, sq = 0, n_ok = 0;
+#pragma unroll
             for (int j = 0; j < 4; ++j) {
-                distinct += cnt[j] > 0;
-                mx = max(mx, cnt[j]);
-                sq += cnt[j] * cnt[j];
+                const int c = cnt >> (8 * j) & 255;
+                n_ok += c;
+                distinct += c > 0;
+                mx = max(mx, c);
+                sq += c * c;
             }
             if (distinct > 0) atomicAdd(&h_site[distinct - 1], 1);
             if (distinct == 1) atomicAdd(&invariant, 1);
@@ -166,20 +166,29 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
             atomicAdd(&h_site[36 + (n_ok ? min(31, 128 * (nn2 - sq) / (3 * nn2)) : 0)], 1);
         }
         __syncthreads();
-        const int len = min(kSimThreads, n_sites - s0);
+#pragma unroll
         for (int q = 0; q < 2; ++q) {
             if (pa[q] < 0) continue;
-            const unsigned char* x = st[pa[q]];
-            const unsigned char* y = st[pb[q]];
-            for (int k = 0; k < len; ++k)
-                if (x[k] != kGap && y[k] != kGap) ++joint[q][x[k] * 4 + y[k]];
+            for (int w = 0; w < kSimThreads / 64; ++w) {
+                uint64_t x[4], y[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) { x[j] = tip[pa[q]][w][j]; y[j] = tip[pb[q]][w][j]; }
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) joint[q][i * 4 + j] += __popcll(x[i] & y[j]);
+            }
         }
+        if (tid < 4 * n_taxa)
+            for (int w = 0; w < kSimThreads / 64; ++w) base_count += __popcll(tip[tid >> 2][w][tid & 3]);
         __syncthreads();
     }
     // pair statistics
+#pragma unroll
     for (int q = 0; q < 2; ++q) {
         if (pa[q] < 0) continue;
         int n = 0;
+#pragma unroll
         for (int c = 0; c < 16; ++c) n += joint[q][c];
         if (n == 0) continue;
         const float inv = 1.f / n;
@@ -187,8 +196,11 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         const int ts = joint[q][1] + joint[q][4] + joint[q][11] + joint[q][14];     // A<->G, C<->T
         const int tv = n - same - ts;
         const float pd = (n - same) * inv, pts = ts * inv, ptv = tv * inv;
+#pragma unroll
         for (int i = 0; i < 4; ++i)
-            for (int j = 0; j < 4; ++j) atomicAdd(&h_pair[i * 4 + j], 0.5f * (joint[q][i * 4 + j] + joint[q][j * 4 + i]) * inv / n_pairs);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                atomicAdd(&h_pair[i * 4 + j], 0.5f * (joint[q][i * 4 + j] + joint[q][j * 4 + i]) * inv / n_pairs);
         // p-distance in bins of 1/40, transition and transversion distances
         // in bins of 1/80 (integer bin edges)
         atomicAdd(&h_pair[16 + min(31, 40 * (n - same) / n)], 1.f / n_pairs);
@@ -202,8 +214,7 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         const float jc = fminf(3.f, -0.75f * logf(fmaxf(1e-6f, 1.f - pd / 0.75f)));
         atomicAdd(&h_pair[116], jc / n_pairs);
     }
-    for (int j = 0; j < 4; ++j) atomicAdd(&base[j], basec[j]);
-    atomicAdd(&gaps_total, gapc);
+    if (tid < 4 * n_taxa) atomicAdd(&base[tid & 3], base_count);
     __syncthreads();
     float* f = feat + (size_t)a * kFeat;
     for (int i = tid; i < kFeat; i += kSimThreads) {
@@ -218,7 +229,7 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         else if (i == 185) v = sqrtf(fmaxf(0.f, h_pair[113] - h_pair[112] * h_pair[112]));
         else if (i == 186) v = h_pair[114];
         else if (i == 187) v = h_pair[115];
-        else if (i == 188) v = (float)gaps_total / ((float)n_sites * n_taxa);
+        else if (i == 188) v = (float)(n_sites * n_taxa - nb) / ((float)n_sites * n_taxa);
         else if (i == 189) v = h_pair[116];
         else if (i == 190) v = fminf(20.f, h_pair[114] / fmaxf(1e-6f, h_pair[115]));
         else if (i == 191) v = (float)invariant / n_sites;
@@ -675,9 +686,24 @@ int phylo_sim_features(int device, int n_align, int n_taxa, int n_sites, int n_c
     for (long i = 0; i < (long)n_align * nn; ++i)
         if (left[i] < -1 || left[i] >= nn || right[i] < -1 || right[i] >= nn) return PHYLO_ERR_ARG;
     // every tree must be a rooted binary tree over nodes 0..nn-1 with the tips
-    // 0..n_taxa-1 childless: the kernel's preorder stack and state table are
-    // sized by that
-    std::vector<int> n_par(nn);
+    // 0..n_taxa-1 childless: the kernel's walk and state table are sized by
+    // that.  The walk lists the nodes in preorder with their parents.
+    std::vector<int> n_par(nn), stack;
+    // one device block for every input, the features and the masks, filled by one copy
+    size_t off = 0;
+    const auto take = [&](size_t bytes) {
+        const size_t at = off;
+        off += (bytes + 255) & ~size_t(255);
+        return at;
+    };
+    const size_t N = (size_t)n_align;
+    const size_t o_walk = take(N * nn * sizeof(int)), o_blen = take(N * nn * sizeof(double));
+    const size_t o_eig = take(N * 36 * sizeof(double)), o_pi = take(N * 4 * sizeof(double));
+    const size_t o_cat = take(N * n_cat * sizeof(double)), in_bytes = off;
+    const size_t o_feat = take(N * kFeat * sizeof(float));
+    const size_t o_mask = take(masks ? N * n_taxa * n_sites * sizeof(uint32_t) : 0);
+    const std::unique_ptr<unsigned char[]> in(new unsigned char[in_bytes]);
+    int* walk = reinterpret_cast<int*>(in.get() + o_walk);
     for (int k = 0; k < n_align; ++k) {
         const int32_t* L = left + (size_t)k * nn;
         const int32_t* R = right + (size_t)k * nn;
@@ -693,50 +719,48 @@ int phylo_sim_features(int device, int n_align, int n_taxa, int n_sites, int n_c
         }
         for (int v = 0; v < nn; ++v)
             if (n_par[v] != (v == roots[k] ? 0 : 1)) return PHYLO_ERR_ARG;
-        // connected: count nodes reachable from the root
-        std::vector<int> stack{roots[k]};
+        // connected: every node is reached from the root
+        int* out = walk + (size_t)k * nn;
         int seen = 0;
+        stack.assign(1, roots[k]);
         while (!stack.empty()) {
-            const int v = stack.back();
+            const int w = stack.back(), v = w & 255;
             stack.pop_back();
-            if (++seen > nn) return PHYLO_ERR_ARG;
-            if (L[v] >= 0) { stack.push_back(L[v]); stack.push_back(R[v]); }
+            if (seen == nn) return PHYLO_ERR_ARG;
+            out[seen++] = w;
+            if (L[v] >= 0) {
+                stack.push_back(R[v] | v << 8);
+                stack.push_back(L[v] | v << 8);
+            }
         }
         if (seen != nn) return PHYLO_ERR_ARG;
     }
+    std::memcpy(in.get() + o_blen, blen, N * nn * sizeof(double));
+    std::memcpy(in.get() + o_eig, eig, N * 36 * sizeof(double));
+    std::memcpy(in.get() + o_pi, pi, N * 4 * sizeof(double));
+    std::memcpy(in.get() + o_cat, cat_rates, N * n_cat * sizeof(double));
     if (hipSetDevice(device) != hipSuccess) return PHYLO_ERR_HIP;
-    hipStream_t st;
-    if (hipStreamCreateWithFlags(&st, hipStreamNonBlocking) != hipSuccess) return PHYLO_ERR_HIP;
+    const hipStream_t st = hipStreamPerThread;     // (a stream of its own a call, and the staging buffer zeroed, took 80 us)
     int rc = PHYLO_OK;
-    int *dl = nullptr, *dr = nullptr, *droot = nullptr;
-    double *db = nullptr, *de = nullptr, *dp = nullptr, *dc = nullptr;
-    float* df = nullptr;
-    uint32_t* dm = nullptr;
-    auto up = [&](auto*& d, const auto* h, size_t n) {
-        if (hipMalloc(reinterpret_cast<void**>(&d), n * sizeof(*h)) != hipSuccess) return false;
-        return hipMemcpyAsync(d, h, n * sizeof(*h), hipMemcpyHostToDevice, st) == hipSuccess;
-    };
-    if (!up(dl, left, (size_t)n_align * nn) || !up(dr, right, (size_t)n_align * nn) || !up(droot, roots, (size_t)n_align) ||
-        !up(db, blen, (size_t)n_align * nn) || !up(de, eig, (size_t)n_align * 36) || !up(dp, pi, (size_t)n_align * 4) ||
-        !up(dc, cat_rates, (size_t)n_align * n_cat) ||
-        hipMalloc(reinterpret_cast<void**>(&df), (size_t)n_align * kFeat * sizeof(float)) != hipSuccess ||
-        (masks && hipMalloc(reinterpret_cast<void**>(&dm), (size_t)n_align * n_taxa * n_sites * sizeof(uint32_t)) !=
-                      hipSuccess)) {
+    unsigned char* d = nullptr;
+    if (hipMalloc(reinterpret_cast<void**>(&d), off) != hipSuccess ||
+        hipMemcpyAsync(d, in.get(), in_bytes, hipMemcpyHostToDevice, st) != hipSuccess) {
         rc = PHYLO_ERR_HIP;
     } else {
-        hipLaunchKernelGGL(sim_features_kernel, dim3(n_align), dim3(kSimThreads), 0, st, n_taxa, n_sites, n_cat, dl, dr,
-                           droot, db, de, dp, dc, (float)gap_frac, seed, df, dm);
+        const auto dbl = [&](size_t o) { return reinterpret_cast<const double*>(d + o); };
+        float* df = reinterpret_cast<float*>(d + o_feat);
+        uint32_t* dm = masks ? reinterpret_cast<uint32_t*>(d + o_mask) : nullptr;
+        hipLaunchKernelGGL(sim_features_kernel, dim3(n_align), dim3(kSimThreads), (size_t)nn * n_cat * 16 * sizeof(float), st,
+                           n_taxa, n_sites, n_cat, reinterpret_cast<const int*>(d + o_walk), dbl(o_blen), dbl(o_eig),
+                           dbl(o_pi), dbl(o_cat), (float)gap_frac, seed, df, dm);
         if (hipGetLastError() != hipSuccess ||
-            hipMemcpyAsync(features, df, (size_t)n_align * kFeat * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
-            (masks && hipMemcpyAsync(masks, dm, (size_t)n_align * n_taxa * n_sites * sizeof(uint32_t),
-                                     hipMemcpyDeviceToHost, st) != hipSuccess) ||
+            hipMemcpyAsync(features, df, N * kFeat * sizeof(float), hipMemcpyDeviceToHost, st) != hipSuccess ||
+            (masks && hipMemcpyAsync(masks, dm, N * n_taxa * n_sites * sizeof(uint32_t), hipMemcpyDeviceToHost, st) !=
+                          hipSuccess) ||
             hipStreamSynchronize(st) != hipSuccess)
             rc = PHYLO_ERR_HIP;
     }
-    void* bufs[] = {dl, dr, droot, db, de, dp, dc, df, dm};
-    for (void* b : bufs)
-        if (b) (void)hipFree(b);
-    (void)hipStreamDestroy(st);
+    if (d) (void)hipFree(d);
     return rc;
 }
 
