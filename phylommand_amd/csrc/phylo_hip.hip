@@ -635,7 +635,7 @@ struct phylo_ctx {
     Op* d_ops = nullptr; size_t ops_bytes = 0;
     int* d_prog = nullptr; size_t prog_bytes = 0;
     double* d_PmT = nullptr; size_t PmT_bytes = 0;       // P transposed in MFMA operand order (NNI walks)
-    bool have_PmT = false;                                // d_PmT matches d_P
+    bool want_PmT = false;                                // NNI walks have asked for d_PmT
     // NNI walks of the current topology (nni_program.h), rebuilt when it changes
     struct NniWalks {
         int mode = -1;                                    // -1: none built
@@ -1078,11 +1078,11 @@ void host_pmatrices(const phylo_ctx* c, int Sp, std::vector<double>& P) {
 }
 
 int upload_pmatrices(phylo_ctx* c) {
-    const int Sp = padded_states(c->S_model);
+    const int S = c->S_model, Sp = padded_states(S);
     const size_t nP = (size_t)c->n_nodes * c->C * Sp * Sp;
     HIPCHK(c, ensure(c->d_P, c->P_bytes, nP * sizeof(double)));
+    const double *dV = nullptr, *dVi = nullptr, *dl = nullptr, *dr = nullptr, *d_eff = nullptr;
     if (c->builder == PHYLO_P_EIGEN) {
-        const int S = c->S_model;
         const size_t n_eig = 2 * c->V.size() + c->lam.size() + c->cat_rate.size();
         double* h = nullptr;
         HIPCHK(c, stage_acquire(c->stage_P, n_eig + c->eff.size(), &h));
@@ -1095,17 +1095,12 @@ int upload_pmatrices(phylo_ctx* c) {
         HIPCHK(c, ensure(c->d_eig, c->eig_bytes, (n_eig + c->eff.size()) * sizeof(double)));
         HIPCHK(c, hipMemcpyAsync(c->d_eig, h, (n_eig + c->eff.size()) * sizeof(double), hipMemcpyHostToDevice,
                                  c->stream));
-        const double* d_eff = c->d_eig + n_eig;
         HIPCHK(c, stage_release(c->stage_P, c->stream));
-        const double* dV = c->d_eig;
-        const double* dVi = dV + (size_t)S * S;
-        const double* dl = dVi + (size_t)S * S;
-        const double* dr = dl + S;
-        const int threads = 256;
-        const long blocks = ((long)nP + threads - 1) / threads;
-        hipLaunchKernelGGL(pbuild_eigen_kernel, dim3((unsigned)blocks), dim3(threads), 0, c->stream, dV, dVi, dl,
-                           d_eff, dr, S, Sp, c->C, c->n_nodes, c->d_P);
-        HIPCHK(c, hipGetLastError());
+        d_eff = c->d_eig + n_eig;
+        dV = c->d_eig;
+        dVi = dV + (size_t)S * S;
+        dl = dVi + (size_t)S * S;
+        dr = dl + S;
     } else {
         std::vector<double> P;
         host_pmatrices(c, Sp, P);
@@ -1113,14 +1108,24 @@ int upload_pmatrices(phylo_ctx* c) {
         HIPCHK(c, hipStreamSynchronize(c->stream));
     }
     if (Sp > 4) {
-        const int V = mfma_slots(c->S_model), TN = V > 4 ? 2 : 1;
-        const size_t nPm = (size_t)c->n_nodes * c->C * TN * V * 64, nPT = (size_t)c->n_nodes * c->C * (c->S_model + 1) * 4 * V;
+        const int V = mfma_slots(S), TN = V > 4 ? 2 : 1;
+        const size_t nPm = (size_t)c->n_nodes * c->C * TN * V * 64, nPT = (size_t)c->n_nodes * c->C * (S + 1) * 4 * V;
         HIPCHK(c, ensure(c->d_Pm, c->Pm_bytes, nPm * sizeof(double)));
         HIPCHK(c, ensure(c->d_PTm, c->PTm_bytes, nPT * sizeof(double)));
-        HIPCHK(c, mfma_operands(c->d_P, c->S_model, Sp, c->C, c->n_nodes, c->d_Pm, c->d_PTm, c->stream));
+        if (c->want_PmT)
+            if (const hipError_t e = ensure(c->d_PmT, c->PmT_bytes, nPm * sizeof(double)); e != hipSuccess) {
+                c->want_PmT = false;      // plain evaluations do without
+                HIPCHK(c, e);
+            }
+        HIPCHK(c, mfma_matrices(dV, dVi, dl, d_eff, dr, S, Sp, c->C, c->n_nodes, c->d_P, c->d_Pm,
+                                c->want_PmT ? c->d_PmT : nullptr, c->d_PTm, c->stream));
+    } else if (c->builder == PHYLO_P_EIGEN) {
+        const long blocks = ((long)nP + 255) / 256;
+        hipLaunchKernelGGL(pbuild_eigen_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, dV, dVi, dl, d_eff, dr, S,
+                           Sp, c->C, c->n_nodes, c->d_P);
+        HIPCHK(c, hipGetLastError());
     }
     c->dirty_P = false;
-    c->have_PmT = false;
     return PHYLO_OK;
 }
 
@@ -1843,12 +1848,6 @@ int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* l
     a.one.n_var = n_out;
     a.one.nblk = nblk;
     a.n_prog = w.n_prog;
-    if (mfma && !c->have_PmT) {
-        const int S = c->S_model, V = mfma_slots(S), TN = V > 4 ? 2 : 1;
-        HIPCHK(c, ensure(c->d_PmT, c->PmT_bytes, (size_t)c->n_nodes * c->C * TN * V * 64 * sizeof(double)));
-        HIPCHK(c, mfma_transposed(c->d_P, S, padded_states(S), c->C, c->n_nodes, c->d_PmT, c->stream));
-        c->have_PmT = true;
-    }
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     if (mfma) HIPCHK(c, nni_mfma_launch(a, c->S, static_cast<const uint32_t*>(c->d_tips), c->d_Pm, c->d_PmT, c->d_PTm, c->stream));
     else HIPCHK(c, nni4_launch(a, c->stream));
@@ -1870,6 +1869,10 @@ int phylo_nni_score(phylo_ctx* c, int mode, int max_variants, double* lnl, int32
                     int* n_variants, double* base_lnl) {
     if (!c || !n_variants) return PHYLO_ERR_ARG;
     if (mode != 0 && mode != 1) return fail(c, PHYLO_ERR_ARG, "nni_score: mode must be 0 or 1");
+    if (uses_mfma(c) && !c->want_PmT) {
+        c->want_PmT = true;          // the walks read P's transposes too
+        c->dirty_P = true;
+    }
     int rc = prepare(c);
     if (rc) return rc;
     double base = 0.0;

@@ -41,11 +41,11 @@ struct MfmaArgs {
 hipError_t mfma_launch(const MfmaArgs& a, hipStream_t st);
 // Workgroups of the staging walker that one CU holds at once, 0 if unknown.
 int mfma_resident(bool f64, int C, int S);
-// The walker's P operands and tip columns from P (pmfma_kernel, ptm_kernel).
-hipError_t mfma_operands(const double* P, int S, int Sp, int C, int n_nodes, double* Pm, double* PTm, hipStream_t st);
-
-// The same operands of every P's transpose (the NNI walks' way down).
-hipError_t mfma_transposed(const double* P, int S, int Sp, int C, int n_nodes, double* PmT, hipStream_t st);
+// P, the walkers' operands of it (Pm; PmT of the transpose, where set) and the
+// tip columns PTm: from the eigen system and lengths (device memory), or with
+// eff null from P as it is (pwide_kernel).
+hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const double* cat_rate,
+                         int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT, double* PTm, hipStream_t st);
 // NNI walks (nni.h; a.tips, a.P and the batch members unused).
 hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const double* Pm, const double* PmT,
                            const double* PTm, hipStream_t st);

@@ -21,9 +21,9 @@ namespace {
 // MFMA result (tile T, register r) is slot 4T + r of the next op's operand
 // with no shuffles.  V = ceil(S / 4) slots cover the S states; tile 1 exists
 // for S > 16 (for 17..20 states as v_mfma_f64_4x4x4f64 blocks, see
-// pmfma_kernel).  Partials are stored as [slot][cat][site group][V][64 lanes]
+// pwide_kernel).  Partials are stored as [slot][cat][site group][V][64 lanes]
 // (every load and store a full row), P as [node][cat][tile][V][64] doubles
-// (pmfma_kernel).  FP64 matrix cores rather than FP32 ones: the FP32 MFMA
+// (pwide_kernel).  FP64 matrix cores rather than FP32 ones: the FP32 MFMA
 // dot products truncate small addends (about -0.1 ulp per 5-step chain on
 // transition-matrix-shaped operands), which biases every site the same way.
 // Scalers as in the DNA walker: one int32 power of two per (node, category,
@@ -32,48 +32,81 @@ namespace {
 
 typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 
+// The P matrices of one (node, category) a workgroup, in every form the walkers
+// read, from one pass: P itself, the matrix-core operands, the tip columns.
+//
+// P[i][j] = sum_k V[i][k] exp(lam_k r_c t_node) Vinv[k][j], the exponentials
+// taken once (eff set), or P as it lies in memory (eff null: built on the host).
+//
 // Pm[node][cat][T][t][lane] = P[16T + lane % 16][4t + lane / 16] (0 outside S),
 // the A operand of v_mfma_f64_16x16x4f64 for row tile T and K-step t.  With
 // V = 5 (17..20 states) tile 1 holds only rows 16..19 and is instead the A
 // operand of v_mfma_f64_4x4x4f64 (four 4x4 blocks, one per 4 sites): lane l
 // = 4b + 16k + i holds P[16 + i][4t + k] for every block b.  That product
 // lands as D[lane j + 16 i] = row 16 + i of site j, the operand slot of
-// states 16..19, with no padded rows.
-// TR: of the transpose.
-template <bool TR>
-__global__ void pmfma_kernel(const double* __restrict__ P, int S, int Sp, int C, int n_nodes, int V, int TN,
-                             double* __restrict__ Pm) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)n_nodes * C * TN * V * 64;
-    if (gid >= total) return;
-    const int l = gid % 64;
-    const int t = (gid / 64) % V;
-    const int T = (gid / (64L * V)) % TN;
-    const long mat = gid / (64L * V * TN);          // node * C + cat
-    const bool short_tile = V == 5 && T == 1;
-    const int row = 16 * T + (short_tile ? l % 4 : l % 16), col = 4 * t + l / 16;
-    Pm[gid] = (row < S && col < S) ? P[TR ? (mat * Sp + col) * Sp + row : (mat * Sp + row) * Sp + col] : 0.0;
-}
-
+// states 16..19, with no padded rows.  PmT (where set): the same of P's
+// transpose.
+//
 // PTm[node][cat][k][i] = P[i][k] for k < S, PTm[..][S][i] = sum_q P[i][q]
 // (the product with an all-states tip), i < 4V (0 for i >= S): the columns a
 // single-state or all-states tip selects.
-__global__ void ptm_kernel(const double* __restrict__ P, int S, int Sp, int C, int n_nodes, int W,
-                           double* __restrict__ PTm) {
-    const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long total = (long)n_nodes * C * (S + 1) * W;
-    if (gid >= total) return;
-    const int i = gid % W;
-    const int k = (gid / W) % (S + 1);
-    const long mat = gid / ((long)W * (S + 1));
-    const double* row = P + (mat * Sp + i) * Sp;
-    double v = 0.0;
-    if (i < S) {
-        if (k < S) v = row[k];
-        else
-            for (int q = 0; q < S; ++q) v += row[q];
+//
+// Bound by the chain exp -> V exp -> S fma -> layouts and the launch, not by its
+// few MB of stores: 7.2 us for the 127 nodes and 4 categories of a 64-taxon
+// 20-state tree.  As three launches, each entry of P with its own S
+// exponentials, the same took 18 us and two more gaps.
+__global__ __launch_bounds__(256) void pwide_kernel(const double* __restrict__ eig_V, const double* __restrict__ eig_Vinv,
+                                                    const double* __restrict__ lam, const double* __restrict__ eff,
+                                                    const double* __restrict__ cat_rate, int S, int Sp, int C, int V,
+                                                    int TN, double* P, double* __restrict__ Pm, double* __restrict__ PmT,
+                                                    double* __restrict__ PTm) {
+    __shared__ double ex[32], ve[32 * 32], vi[32 * 32], p[32][33];
+    const int mat = blockIdx.x, c = mat % C, node = mat / C;      // node * C + cat
+    const int tid = threadIdx.x;
+    double* Pg = P + (size_t)mat * Sp * Sp;
+    if (eff) {
+        const double t = eff[node] * cat_rate[c];
+        if (tid < S) ex[tid] = exp(lam[tid] * t);
+        __syncthreads();
+        for (int i = tid; i < S * S; i += 256) {
+            ve[i] = eig_V[i] * ex[i % S];
+            vi[i] = eig_Vinv[i];
+        }
+        __syncthreads();
+        for (int e = tid; e < Sp * Sp; e += 256) {
+            const int i = e / Sp, j = e % Sp;
+            double v = 0.0;
+            if (i < S && j < S)
+                for (int k = 0; k < S; ++k) v = fma(ve[i * S + k], vi[k * S + j], v);
+            p[i][j] = v;
+            Pg[e] = v;
+        }
+    } else {
+        for (int e = tid; e < Sp * Sp; e += 256) p[e / Sp][e % Sp] = Pg[e];
     }
-    PTm[gid] = v;
+    __syncthreads();
+    double* pm = Pm + (size_t)mat * TN * V * 64;
+    double* pmt = PmT ? PmT + (size_t)mat * TN * V * 64 : nullptr;
+    for (int e = tid; e < TN * V * 64; e += 256) {
+        const int l = e % 64, t = e / 64 % V, T = e / (64 * V);
+        const bool short_tile = V == 5 && T == 1;
+        const int row = 16 * T + (short_tile ? l % 4 : l % 16), col = 4 * t + l / 16;
+        const bool in = row < S && col < S;
+        pm[e] = in ? p[row][col] : 0.0;
+        if (pmt) pmt[e] = in ? p[col][row] : 0.0;
+    }
+    const int W = 4 * V;
+    double* pt = PTm + (size_t)mat * (S + 1) * W;
+    for (int e = tid; e < (S + 1) * W; e += 256) {
+        const int i = e % W, k = e / W;
+        double v = 0.0;
+        if (i < S) {
+            if (k < S) v = p[i][k];
+            else
+                for (int q = 0; q < S; ++q) v += p[i][q];
+        }
+        pt[e] = v;
+    }
 }
 
 __device__ inline double to_d(float x) { return (double)x; }
@@ -916,20 +949,10 @@ hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const 
     return hipGetLastError();
 }
 
-hipError_t mfma_transposed(const double* P, int S, int Sp, int C, int n_nodes, double* PmT, hipStream_t st) {
-    const int V = mfma_slots(S), TN = V > 4 ? 2 : 1;
-    const long nPm = (long)n_nodes * C * TN * V * 64;
-    hipLaunchKernelGGL((pmfma_kernel<true>), dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, V,
-                       TN, PmT);
-    return hipGetLastError();
-}
-
-hipError_t mfma_operands(const double* P, int S, int Sp, int C, int n_nodes, double* Pm, double* PTm, hipStream_t st) {
-    const int V = mfma_slots(S), TN = V > 4 ? 2 : 1;
-    const long nPm = (long)n_nodes * C * TN * V * 64, nPT = (long)n_nodes * C * (S + 1) * 4 * V;
-    hipLaunchKernelGGL((pmfma_kernel<false>), dim3((unsigned)((nPm + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, V, TN,
-                       Pm);
-    hipLaunchKernelGGL(ptm_kernel, dim3((unsigned)((nPT + 255) / 256)), dim3(256), 0, st, P, S, Sp, C, n_nodes, 4 * V,
-                       PTm);
+hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const double* cat_rate,
+                         int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT, double* PTm, hipStream_t st) {
+    const int slots = mfma_slots(S);
+    hipLaunchKernelGGL(pwide_kernel, dim3(n_nodes * C), dim3(256), 0, st, V, Vinv, lam, eff, cat_rate, S, Sp, C, slots,
+                       slots > 4 ? 2 : 1, P, Pm, PmT, PTm);
     return hipGetLastError();
 }
