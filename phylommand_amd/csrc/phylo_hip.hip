@@ -1458,7 +1458,8 @@ long nni_path_ops(const TV* c, const std::vector<int>& par, int v) {
 
 // Enumerates a neighbourhood and builds its walks (nni_program.h): node / side of
 // every variant in `node` / `side`, the variant of each scored output in
-// `which` (both sides of an edge are scored or neither is).
+// `which` (both sides of an edge are scored or neither is; -1 for the side of
+// a single-child node that would move its missing child: that keeps the tree).
 template <class TV>
 void build_nni(const TV* c, int mode, int max_edges, std::vector<int>& node, std::vector<int>& side,
                std::vector<int>& which, long& path_ops, std::vector<NniOp>& ops, std::vector<int>& begin) {
@@ -1470,8 +1471,8 @@ void build_nni(const TV* c, int mode, int max_edges, std::vector<int>& node, std
     for (size_t k = 0; k + 1 < node.size(); k += 2) {
         if (nni_partner(c, par, node[k]) < 0) continue;
         pair_of[node[k]] = (int)which.size();
-        which.push_back((int)k);
-        which.push_back((int)k + 1);
+        which.push_back(c->left[node[k]] >= 0 ? (int)k : -1);
+        which.push_back(c->right[node[k]] >= 0 ? (int)k + 1 : -1);
         path_ops += 2 * nni_path_ops(c, par, node[k]);
     }
     if (!which.empty()) build_nni_walks(c, pair_of, max_edges, ops, begin);
@@ -1858,7 +1859,8 @@ int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* l
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;
-    for (int q = 0; q < n_out; ++q) lnl[w.which[q]] = c->h_total[q];
+    for (int q = 0; q < n_out; ++q)
+        if (w.which[q] >= 0) lnl[w.which[q]] = c->h_total[q];
     c->nni_ops_last = w.path_ops;
     return PHYLO_OK;
 }
@@ -2723,7 +2725,10 @@ int phylo_batch_run(phylo_batch* b, double* totals, double* nni_lnl) {
             const auto& I = b->inst[i];
             double* dst = nni_lnl + b->var_offsets[i];
             std::fill(dst, dst + I.nni_node.size(), b->h_out[i]);     // no-op variants keep the base tree
-            for (int k : I.nni_which) dst[k] = b->h_out[ni + seg++];
+            for (int k : I.nni_which) {
+                if (k >= 0) dst[k] = b->h_out[ni + seg];
+                ++seg;
+            }
         }
     }
     return PHYLO_OK;

@@ -1,12 +1,14 @@
 """NNI neighbourhoods by the outer-partial walks where their layouts can go
 wrong: state counts around the operand slots and tiles, one category and many,
 site counts around a wave, taxa past what a workgroup stages,
-FP64, site weights, every mode, and lengths changed in between."""
+unary nodes, FP64, site weights, every mode, and lengths changed in between."""
 import numpy as np
 import pytest
 
+import phylommand_amd as P
 from phylommand_amd import synth
 from helpers import gpu_context
+from test_gpu_edge import _tree, _workload
 
 pytestmark = pytest.mark.gpu
 
@@ -72,3 +74,23 @@ def test_both_builders_give_the_same_scores(S):
             base, variants = ctx.nni_score(1)
             got.append([base] + [x[2] for x in variants])
     np.testing.assert_allclose(got[0], got[1], rtol=1e-9)
+
+
+@pytest.mark.parametrize("S,prec", [(4, 0), (4, 1), (20, 0), (20, 1)])
+def test_unary_nodes_pass_their_child(oracle, S, prec):
+    """A unary internal node on a path, inside the neighbourhood: exchanging
+    its missing child keeps the tree, alone and in a batch."""
+    print(f"nni unary S={S} prec={prec}", flush=True)
+    # tips 0..4; 5 = (0,1); 6 = unary above 5; 7 = (2,3); 8 = (6,7); 9 = root (8,4)
+    t = _tree([-1] * 5 + [0, 5, 2, 6, 8], [-1] * 5 + [1, -1, 3, 7, 4], 9,
+              [0.1, 0.2, 0.15, 0.25, 0.05, 0.3, 0.12, 0.2, 0.1, 0.0], 5)
+    wl = _workload(t, 130, C=2, S=S, seed=6)
+    with gpu_context(wl, precision=prec) as ctx:
+        _check(oracle, wl, ctx, 1)
+        single = ctx.nni_score(1)[1]
+    if S == 4:
+        with P.Batch(2, prec) as b:
+            b.add(wl.masks, t.left, t.right, t.root, t.blen, wl.Q, wl.pi, wl.cat_rates, wl.cat_weights, nni_mode=1)
+            b.finalize(autotune=False)
+            nni = b.run()[1]
+        np.testing.assert_allclose(nni, [x[2] for x in single], rtol=1e-9)
