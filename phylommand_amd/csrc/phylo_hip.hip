@@ -522,6 +522,35 @@ __global__ void pbuild_eigen_kernel(const double* __restrict__ V, const double* 
     P[gid] = v;
 }
 
+// The same for a context of at most 4 states (Sp = 4), with nothing copied to
+// the device beforehand: the eigen system, rates and weights are arguments,
+// the lengths are read from the host's pinned memory (one 8-byte read a wave).
+// Bound by the round trip to host memory and the launch: 4.5 us at 32 and at
+// 128 taxa.  A copy in front of it cost 10 us of host time and a 3 us copy
+// kernel; a fit that changes the model each evaluation took two (59 us an
+// evaluation of 32 taxa x 2000 sites then, 37 us now).
+struct Eig4 {
+    double rate[kMaxCat], V[16], Vinv[16], lam[4];
+};
+__global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const double* __restrict__ eff, int S, int C,
+                               int n_nodes, double* __restrict__ P, double* __restrict__ d_roots) {
+    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    if (gid < kRootDoubles) d_roots[gid] = roots.v[gid];
+    if (gid >= n_nodes * C * 16) return;
+    const int j = gid % 4, i = gid / 4 % 4, c = gid / 16 % C, node = gid / (16 * C);
+    double v = 0.0;
+    if (i < S && j < S) {
+        const double t = eff[node] * e.rate[c];
+        for (int k = 0; k < S; ++k) v = fma(e.V[i * S + k] * exp(e.lam[k] * t), e.Vinv[k * S + j], v);
+    }
+    P[gid] = v;
+}
+
+// The root and category weights alone (P is unchanged, or built on the host).
+__global__ void roots_kernel(const RootWeights roots, double* __restrict__ d_roots) {
+    if (threadIdx.x < kRootDoubles) d_roots[threadIdx.x] = roots.v[threadIdx.x];
+}
+
 __device__ inline uint64_t sim_mix(uint64_t z) {
     z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
     z = (z ^ (z >> 27)) * 0x94d049bb133111ebull;
@@ -633,7 +662,7 @@ struct phylo_ctx {
     int* d_scl = nullptr; size_t scl_bytes = 0;
     double* d_P = nullptr; size_t P_bytes = 0;
     Op* d_ops = nullptr; size_t ops_bytes = 0;
-    int* d_prog = nullptr; size_t prog_bytes = 0;
+    int* d_prog = nullptr;                               // in d_ops' buffer, after the ops
     double* d_PmT = nullptr; size_t PmT_bytes = 0;       // P transposed in MFMA operand order (NNI walks)
     bool want_PmT = false;                                // NNI walks have asked for d_PmT
     // NNI walks of the current topology (nni_program.h), rebuilt when it changes
@@ -653,20 +682,23 @@ struct phylo_ctx {
     bool keep_partials = false;                           // loglik stores every node's partial
     double* d_roots = nullptr;
     double* d_sitew = nullptr; size_t sitew_bytes = 0;
-    double* d_sitelnl = nullptr; size_t sitelnl_bytes = 0;
     double* d_partial = nullptr; size_t partial_bytes = 0;
-    double* d_eig = nullptr; size_t eig_bytes = 0;      // V, Vinv, lambda, category rates, edge lengths
+    double* d_eig = nullptr; size_t eig_bytes = 0;      // V, Vinv, lambda (wide states)
+    bool dirty_eig = true;
     double* h_total = nullptr; size_t h_total_bytes = 0;  // pinned, mapped: final_sum_kernel writes here
     double* h_total_dev = nullptr;                        // its device address
-    // Pinned staging for the per-evaluation uploads (eigen system + edge
-    // lengths, root / category weights): copied without a stream
-    // synchronisation; an event guards reuse of the host buffer.
+    // Pinned, mapped host memory that work on the stream reads (edge lengths;
+    // eigen system of wide states, compiled programs) or writes (site values):
+    // no stream synchronisation around it, the evaluation that used it ends
+    // with one.  (Site values copied to the caller's array by the runtime
+    // took 40 us more for 2000 to 4000 sites; the programs of a new topology,
+    // in three pageable copies and a wait, 15 us more.)
     struct Stage {
         double* h = nullptr;
+        double* dev = nullptr;      // its device address
         size_t cap = 0;
-        hipEvent_t ev = nullptr;
-        bool pending = false;
-    } stage_P, stage_roots;
+        bool pending = false;       // work that uses it may be in flight
+    } stage_len, stage_eig, stage_prog, stage_site;
 };
 
 namespace {
@@ -717,50 +749,53 @@ void order_children(std::vector<Op>& ops) {
     }
 }
 
-// Copies a program's ops to the device, children in kind order, followed by
-// one zero op: the walkers read the op after the one they run (up to
-// ops[end] of the last program), the DNA walker to load its P matrices
-// early, the matrix walker to have the descriptor at hand.
-hipError_t upload_ops(Op*& d, size_t& have, std::vector<Op>& ops, hipStream_t st) {
-    static const Op pad{};
-    order_children(ops);
-    hipError_t e = ensure(d, have, (ops.size() + 1) * sizeof(Op));
-    if (e == hipSuccess) e = hipMemcpyAsync(d, ops.data(), ops.size() * sizeof(Op), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(d + ops.size(), &pad, sizeof(Op), hipMemcpyHostToDevice, st);
-    return e;
-}
-
-// Host staging area of n doubles, free to overwrite once the copy that last
-// read it has completed.
-hipError_t stage_acquire(phylo_ctx::Stage& st, size_t n, double** out) {
+// Pinned memory of n doubles, free to overwrite once the work that last used
+// it has completed.
+hipError_t stage_acquire(phylo_ctx* c, phylo_ctx::Stage& st, size_t n) {
     hipError_t e;
     if (st.pending) {
-        if ((e = hipEventSynchronize(st.ev)) != hipSuccess) return e;
+        if ((e = hipStreamSynchronize(c->stream)) != hipSuccess) return e;
         st.pending = false;
     }
-    if (!st.ev && (e = hipEventCreateWithFlags(&st.ev, hipEventDisableTiming)) != hipSuccess) return e;
     if (st.cap < n) {
         if (st.h && (e = hipHostFree(st.h)) != hipSuccess) return e;
         st.h = nullptr;
         st.cap = 0;
-        if ((e = hipHostMalloc(reinterpret_cast<void**>(&st.h), n * sizeof(double))) != hipSuccess) return e;
+        if ((e = hipHostMalloc(reinterpret_cast<void**>(&st.h), n * sizeof(double), hipHostMallocMapped)) != hipSuccess ||
+            (e = hipHostGetDevicePointer(reinterpret_cast<void**>(&st.dev), st.h, 0)) != hipSuccess)
+            return e;
         st.cap = n;
     }
-    *out = st.h;
+    st.pending = true;
     return hipSuccess;
 }
 
-hipError_t stage_release(phylo_ctx::Stage& st, hipStream_t stream) {
-    hipError_t e = hipEventRecord(st.ev, stream);
-    st.pending = e == hipSuccess;
-    return e;
+// Copies the compiled programs to the device in one piece: the ops, children
+// in kind order, one zero op (the walkers read the op after the one they run,
+// up to ops[end] of the last program: the DNA walker to load its P matrices
+// early, the matrix walker to have the descriptor at hand), then the programs'
+// bounds.
+hipError_t upload_programs(phylo_ctx* c) {
+    order_children(c->ops);
+    const size_t n_op = c->ops.size(), op_bytes = (n_op + 1) * sizeof(Op);
+    const size_t bytes = op_bytes + c->prog_begin.size() * sizeof(int);
+    hipError_t e = stage_acquire(c, c->stage_prog, (bytes + sizeof(double) - 1) / sizeof(double));
+    if (e != hipSuccess) return e;
+    Op* h = reinterpret_cast<Op*>(c->stage_prog.h);
+    std::copy(c->ops.begin(), c->ops.end(), h);
+    h[n_op] = Op{};
+    std::copy(c->prog_begin.begin(), c->prog_begin.end(), reinterpret_cast<int*>(h + n_op + 1));
+    if ((e = ensure(c->d_ops, c->ops_bytes, bytes)) != hipSuccess) return e;
+    c->d_prog = reinterpret_cast<int*>(c->d_ops + n_op + 1);
+    return hipMemcpyAsync(c->d_ops, h, bytes, hipMemcpyHostToDevice, c->stream);
 }
 
-void stage_free(phylo_ctx::Stage& st) {
-    if (st.pending && st.ev) (void)hipEventSynchronize(st.ev);
-    if (st.h) (void)hipHostFree(st.h);
-    if (st.ev) (void)hipEventDestroy(st.ev);
-    st = phylo_ctx::Stage{};
+// Waits for everything on the context's stream.
+hipError_t finish(phylo_ctx* c) {
+    const hipError_t e = hipStreamSynchronize(c->stream);
+    if (e == hipSuccess)
+        c->stage_len.pending = c->stage_eig.pending = c->stage_prog.pending = c->stage_site.pending = false;
+    return e;
 }
 
 // States per stored partial: 4 for the DNA walker, else the next supported
@@ -1077,30 +1112,32 @@ void host_pmatrices(const phylo_ctx* c, int Sp, std::vector<double>& P) {
     }
 }
 
+RootWeights root_weights(const phylo_ctx* c) {
+    RootWeights r{};
+    std::copy(c->root_w.begin(), c->root_w.end(), r.v);
+    std::copy(c->cat_w.begin(), c->cat_w.end(), r.v + kRootCatOff);
+    return r;
+}
+
 int upload_pmatrices(phylo_ctx* c) {
     const int S = c->S_model, Sp = padded_states(S);
     const size_t nP = (size_t)c->n_nodes * c->C * Sp * Sp;
     HIPCHK(c, ensure(c->d_P, c->P_bytes, nP * sizeof(double)));
-    const double *dV = nullptr, *dVi = nullptr, *dl = nullptr, *dr = nullptr, *d_eff = nullptr;
-    if (c->builder == PHYLO_P_EIGEN) {
-        const size_t n_eig = 2 * c->V.size() + c->lam.size() + c->cat_rate.size();
-        double* h = nullptr;
-        HIPCHK(c, stage_acquire(c->stage_P, n_eig + c->eff.size(), &h));
-        double* w = std::copy(c->V.begin(), c->V.end(), h);
-        w = std::copy(c->Vinv.begin(), c->Vinv.end(), w);
-        w = std::copy(c->lam.begin(), c->lam.end(), w);
-        w = std::copy(c->cat_rate.begin(), c->cat_rate.end(), w);
-        std::copy(c->eff.begin(), c->eff.end(), w);
-        // eigen system and edge lengths in one buffer: one copy per model or length change
-        HIPCHK(c, ensure(c->d_eig, c->eig_bytes, (n_eig + c->eff.size()) * sizeof(double)));
-        HIPCHK(c, hipMemcpyAsync(c->d_eig, h, (n_eig + c->eff.size()) * sizeof(double), hipMemcpyHostToDevice,
-                                 c->stream));
-        HIPCHK(c, stage_release(c->stage_P, c->stream));
-        d_eff = c->d_eig + n_eig;
-        dV = c->d_eig;
-        dVi = dV + (size_t)S * S;
-        dl = dVi + (size_t)S * S;
-        dr = dl + S;
+    if (!c->d_roots) HIPCHK(c, hipMalloc(&c->d_roots, kRootDoubles * sizeof(double)));
+    const bool eigen = c->builder == PHYLO_P_EIGEN;
+    if (eigen) {
+        HIPCHK(c, stage_acquire(c, c->stage_len, c->eff.size()));
+        std::copy(c->eff.begin(), c->eff.end(), c->stage_len.h);
+        if (Sp > 4 && c->dirty_eig) {     // every workgroup reads all of it: a copy, once a model
+            const size_t n_eig = 2 * c->V.size() + c->lam.size();
+            HIPCHK(c, ensure(c->d_eig, c->eig_bytes, n_eig * sizeof(double)));
+            HIPCHK(c, stage_acquire(c, c->stage_eig, n_eig));
+            double* w = std::copy(c->V.begin(), c->V.end(), c->stage_eig.h);
+            w = std::copy(c->Vinv.begin(), c->Vinv.end(), w);
+            std::copy(c->lam.begin(), c->lam.end(), w);
+            HIPCHK(c, hipMemcpyAsync(c->d_eig, c->stage_eig.h, n_eig * sizeof(double), hipMemcpyHostToDevice, c->stream));
+            c->dirty_eig = false;
+        }
     } else {
         std::vector<double> P;
         host_pmatrices(c, Sp, P);
@@ -1117,13 +1154,23 @@ int upload_pmatrices(phylo_ctx* c) {
                 c->want_PmT = false;      // plain evaluations do without
                 HIPCHK(c, e);
             }
-        HIPCHK(c, mfma_matrices(dV, dVi, dl, d_eff, dr, S, Sp, c->C, c->n_nodes, c->d_P, c->d_Pm,
-                                c->want_PmT ? c->d_PmT : nullptr, c->d_PTm, c->stream));
-    } else if (c->builder == PHYLO_P_EIGEN) {
-        const long blocks = ((long)nP + 255) / 256;
-        hipLaunchKernelGGL(pbuild_eigen_kernel, dim3((unsigned)blocks), dim3(256), 0, c->stream, dV, dVi, dl, d_eff, dr, S,
-                           Sp, c->C, c->n_nodes, c->d_P);
+        PRates rates;
+        std::copy(c->cat_rate.begin(), c->cat_rate.end(), rates.v);
+        const double* dVi = c->d_eig + (size_t)S * S;
+        HIPCHK(c, mfma_matrices(c->d_eig, dVi, dVi + (size_t)S * S, eigen ? c->stage_len.dev : nullptr, rates,
+                                root_weights(c), S, Sp, c->C, c->n_nodes, c->d_P, c->d_Pm,
+                                c->want_PmT ? c->d_PmT : nullptr, c->d_PTm, c->d_roots, c->stream));
+        c->dirty_roots = false;
+    } else if (eigen) {
+        Eig4 e{};
+        std::copy(c->cat_rate.begin(), c->cat_rate.end(), e.rate);
+        std::copy(c->V.begin(), c->V.end(), e.V);
+        std::copy(c->Vinv.begin(), c->Vinv.end(), e.Vinv);
+        std::copy(c->lam.begin(), c->lam.end(), e.lam);
+        hipLaunchKernelGGL(pbuild4_kernel, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0, c->stream, e, root_weights(c),
+                           c->stage_len.dev, S, c->C, c->n_nodes, c->d_P, c->d_roots);
         HIPCHK(c, hipGetLastError());
+        c->dirty_roots = false;
     }
     c->dirty_P = false;
     return PHYLO_OK;
@@ -1170,10 +1217,7 @@ int prepare(phylo_ctx* c) {
         int rc = compile_full_program(c);
         if (rc) return rc;
         if (!root_ops_last(c->ops, c->prog_begin)) return fail(c, PHYLO_ERR_STATE, "internal: root op not last");
-        HIPCHK(c, upload_ops(c->d_ops, c->ops_bytes, c->ops, c->stream));
-        HIPCHK(c, ensure(c->d_prog, c->prog_bytes, c->prog_begin.size() * sizeof(int)));
-        HIPCHK(c, hipMemcpyAsync(c->d_prog, c->prog_begin.data(), c->prog_begin.size() * sizeof(int), hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        HIPCHK(c, upload_programs(c));
         c->dirty_topo = false;
         c->walks.mode = -1;
     }
@@ -1187,15 +1231,9 @@ int prepare(phylo_ctx* c) {
         if (rc) return rc;
     }
     if (c->dirty_roots) {
-        const size_t n_roots = kMaxStates + kMaxCat;
-        double* roots = nullptr;
-        HIPCHK(c, stage_acquire(c->stage_roots, n_roots, &roots));
-        std::fill(roots, roots + n_roots, 0.0);
-        for (int i = 0; i < c->S; ++i) roots[i] = c->root_w[i];
-        for (int k = 0; k < c->C; ++k) roots[kRootCatOff + k] = c->cat_w[k];
-        if (!c->d_roots) HIPCHK(c, hipMalloc(&c->d_roots, n_roots * sizeof(double)));
-        HIPCHK(c, hipMemcpyAsync(c->d_roots, roots, n_roots * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, stage_release(c->stage_roots, c->stream));
+        if (!c->d_roots) HIPCHK(c, hipMalloc(&c->d_roots, kRootDoubles * sizeof(double)));
+        hipLaunchKernelGGL(roots_kernel, dim3(1), dim3(64), 0, c->stream, root_weights(c), c->d_roots);
+        HIPCHK(c, hipGetLastError());
         c->dirty_roots = false;
     }
     return PHYLO_OK;
@@ -1335,10 +1373,11 @@ int run_programs(phylo_ctx* c, const Op* d_ops, const int* d_prog, int n_prog, d
     const bool mfma = uses_mfma(c);
     const int nblk = c->m_pad / (mfma ? 16 * kMfmaGroups : 64);
     HIPCHK(c, ensure(c->d_partial, c->partial_bytes, (size_t)n_prog * nblk * sizeof(double)));
-    if (site_lnl_host) HIPCHK(c, ensure(c->d_sitelnl, c->sitelnl_bytes, (size_t)n_prog * c->m * sizeof(double)));
+    // site values go straight into pinned memory, as the totals do
+    if (site_lnl_host) HIPCHK(c, stage_acquire(c, c->stage_site, (size_t)n_prog * c->m));
     if (int rc = ensure_totals(c, n_prog)) return rc;
     dim3 grid(nblk, n_prog);
-    double* dsite = site_lnl_host ? c->d_sitelnl : nullptr;
+    double* dsite = site_lnl_host ? c->stage_site.dev : nullptr;
     if (!c->d_fold) {
         // cleared on the context's own stream: a null-stream hipMemset is not
         // ordered with this non-blocking stream, and with other host threads
@@ -1363,9 +1402,8 @@ int run_programs(phylo_ctx* c, const Op* d_ops, const int* d_prog, int n_prog, d
                            c->h_total_dev);
         HIPCHK(c, hipGetLastError());
     }
-    if (site_lnl_host)
-        HIPCHK(c, hipMemcpyAsync(site_lnl_host, c->d_sitelnl, (size_t)n_prog * c->m * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, finish(c));
+    if (site_lnl_host) std::memcpy(site_lnl_host, c->stage_site.h, (size_t)n_prog * c->m * sizeof(double));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;
@@ -1533,14 +1571,13 @@ void phylo_destroy(phylo_ctx* c) {
     if (!c) return;
     (void)hipSetDevice(c->device);
     if (c->stream) (void)hipStreamSynchronize(c->stream);
-    void* bufs[] = {c->d_tips, c->d_Pm, c->d_PTm, c->d_clv, c->d_scl, c->d_P, c->d_ops, c->d_prog, c->d_PmT,
-                    c->d_roots, c->d_sitew,
-                    c->d_sitelnl, c->d_partial, c->d_eig, c->d_fold, c->walks.d_ops, c->walks.d_prog, c->walks.d_part};
+    void* bufs[] = {c->d_tips, c->d_Pm, c->d_PTm, c->d_clv, c->d_scl, c->d_P, c->d_ops, c->d_PmT,
+                    c->d_roots, c->d_sitew, c->d_partial, c->d_eig, c->d_fold, c->walks.d_ops, c->walks.d_prog, c->walks.d_part};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     if (c->h_total) (void)hipHostFree(c->h_total);
-    stage_free(c->stage_P);
-    stage_free(c->stage_roots);
+    for (auto* st : {&c->stage_len, &c->stage_eig, &c->stage_prog, &c->stage_site})
+        if (st->h) (void)hipHostFree(st->h);
     if (c->ev0) (void)hipEventDestroy(c->ev0);
     if (c->ev1) (void)hipEventDestroy(c->ev1);
     if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -1662,6 +1699,7 @@ int phylo_set_model(phylo_ctx* c, int n_states, const double* Q, const double* r
     }
     c->have_model = true;
     c->dirty_P = true;
+    c->dirty_eig = true;
     c->clv_valid = false;
     c->dirty_roots = true;
     return PHYLO_OK;
@@ -1855,7 +1893,7 @@ int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* l
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr,
                              (n_out + kNniSumVars - 1) / kNniSumVars, c->h_total_dev, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, finish(c));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;

@@ -36,6 +36,7 @@ constexpr int kMaxCat = 8;
 constexpr int kMaxStates = 32;
 constexpr double kLn2 = 0.69314718055994530942;
 constexpr int kRootCatOff = 32;   // roots[]: per-state weights [0, 32), category weights after
+constexpr int kRootDoubles = kRootCatOff + kMaxCat;
 
 // Workgroups per CU below which a whole-tree launch has too few waves to
 // hide its dependent chain: every site block is then walked as subtree

@@ -41,11 +41,22 @@ struct MfmaArgs {
 hipError_t mfma_launch(const MfmaArgs& a, hipStream_t st);
 // Workgroups of the staging walker that one CU holds at once, 0 if unknown.
 int mfma_resident(bool f64, int C, int S);
+// By value in kernel arguments: nothing to copy to the device beforehand.
+struct RootWeights {
+    double v[40];      // roots[]: per-state weights, category weights from 32
+};
+struct PRates {
+    double v[8];       // category rates
+};
+
 // P, the walkers' operands of it (Pm; PmT of the transpose, where set) and the
-// tip columns PTm: from the eigen system and lengths (device memory), or with
+// tip columns PTm: from the eigen system (device
+// memory) and lengths (device or mapped host memory), or with
 // eff null from P as it is (pwide_kernel).
-hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const double* cat_rate,
-                         int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT, double* PTm, hipStream_t st);
+// Writes the root and category weights `roots` to d_roots too.
+hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const PRates& rates,
+                         const RootWeights& roots, int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT,
+                         double* PTm, double* d_roots, hipStream_t st);
 // NNI walks (nni.h; a.tips, a.P and the batch members unused).
 hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const double* Pm, const double* PmT,
                            const double* PTm, hipStream_t st);

@@ -57,15 +57,17 @@ typedef double mfma_d4 __attribute__((ext_vector_type(4)));
 // exponentials, the same took 18 us and two more gaps.
 __global__ __launch_bounds__(256) void pwide_kernel(const double* __restrict__ eig_V, const double* __restrict__ eig_Vinv,
                                                     const double* __restrict__ lam, const double* __restrict__ eff,
-                                                    const double* __restrict__ cat_rate, int S, int Sp, int C, int V,
-                                                    int TN, double* P, double* __restrict__ Pm, double* __restrict__ PmT,
-                                                    double* __restrict__ PTm) {
+                                                    const PRates rates, const RootWeights roots, int S, int Sp, int C,
+                                                    int V, int TN, double* P, double* __restrict__ Pm,
+                                                    double* __restrict__ PmT, double* __restrict__ PTm,
+                                                    double* __restrict__ d_roots) {
     __shared__ double ex[32], ve[32 * 32], vi[32 * 32], p[32][33];
     const int mat = blockIdx.x, c = mat % C, node = mat / C;      // node * C + cat
     const int tid = threadIdx.x;
     double* Pg = P + (size_t)mat * Sp * Sp;
+    if (mat == 0 && tid < kRootDoubles) d_roots[tid] = roots.v[tid];
     if (eff) {
-        const double t = eff[node] * cat_rate[c];
+        const double t = eff[node] * rates.v[c];
         if (tid < S) ex[tid] = exp(lam[tid] * t);
         __syncthreads();
         for (int i = tid; i < S * S; i += 256) {
@@ -949,10 +951,11 @@ hipError_t nni_mfma_launch(const NniArgs& a, int S, const uint32_t* tips, const 
     return hipGetLastError();
 }
 
-hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const double* cat_rate,
-                         int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT, double* PTm, hipStream_t st) {
+hipError_t mfma_matrices(const double* V, const double* Vinv, const double* lam, const double* eff, const PRates& rates,
+                         const RootWeights& roots, int S, int Sp, int C, int n_nodes, double* P, double* Pm, double* PmT,
+                         double* PTm, double* d_roots, hipStream_t st) {
     const int slots = mfma_slots(S);
-    hipLaunchKernelGGL(pwide_kernel, dim3(n_nodes * C), dim3(256), 0, st, V, Vinv, lam, eff, cat_rate, S, Sp, C, slots,
-                       slots > 4 ? 2 : 1, P, Pm, PmT, PTm);
+    hipLaunchKernelGGL(pwide_kernel, dim3(n_nodes * C), dim3(256), 0, st, V, Vinv, lam, eff, rates, roots, S, Sp, C, slots,
+                       slots > 4 ? 2 : 1, P, Pm, PmT, PTm, d_roots);
     return hipGetLastError();
 }
