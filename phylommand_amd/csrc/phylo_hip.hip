@@ -152,7 +152,7 @@ __device__ __forceinline__ void load_p2(const Op& op, const char* Pcat, double (
 // are loaded into nPl / nPr once this op's products are done: the P
 // registers are free by then, and the loads run under the rest of the op
 // instead of at the start of the next.
-template <typename T, int C, bool TL, bool PIPE>
+template <typename T, int C, bool TL, bool PIPE, bool LOC>
 __device__ __forceinline__ void walk4_op(const Op op, const uint8_t* __restrict__ tips, const uint8_t* tl,
                                          const double2* tipv, const T* plane, size_t slot_stride, int* scl,
                                          const char* Pcat, int m_pad, int s, int lane, int cat,
@@ -172,30 +172,38 @@ __device__ __forceinline__ void walk4_op(const Op op, const uint8_t* __restrict_
     // which the compiler keeps apart from the switch's compare tree)
     double L[4];
     int sc = 0;
+    const int ms = m_pad, si = LOC ? lane : s;     // a slot's sites and this one's index (LOC: in LDS)
     if (op.flags & OP_SH_AT)
-        children4<SRC_CARRY_A, SRC_TIP, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, m_pad, s, lane, cat,
+        children4<SRC_CARRY_A, SRC_TIP, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat,
                                                   cin, sin, xb, sB, Pl, Pr, L, sc);
     else if (op.flags & OP_SH_TT)
-        children4<SRC_TIP, SRC_TIP, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, m_pad, s, lane, cat, cin,
+        children4<SRC_TIP, SRC_TIP, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat, cin,
                                               sin, xb, sB, Pl, Pr, L, sc);
-    else if (op.flags & OP_SH_AB)
-        children4<SRC_CARRY_A, SRC_CARRY_B, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, m_pad, s, lane, cat,
+    else if (!LOC && op.flags & OP_SH_AB)
+        children4<SRC_CARRY_A, SRC_CARRY_B, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat,
                                                       cin, sin, xb, sB, Pl, Pr, L, sc);
     else if (op.flags & OP_SH_AC)
-        children4<SRC_CARRY_A, SRC_CLV, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, m_pad, s, lane, cat,
+        children4<SRC_CARRY_A, SRC_CLV, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat,
                                                   cin, sin, xb, sB, Pl, Pr, L, sc);
     else switch (op.l_kind * 5 + op.r_kind) {
 #define PHYLO_SHAPE(A, B)                                                                                   \
     case A * 5 + B:                                                                                       \
-        children4<A, B, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, m_pad, s, lane, cat, cin, sin, xb, \
+        children4<A, B, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat, cin, sin, xb, \
                                   sB, Pl, Pr, L, sc);                                                     \
+        break;
+#define PHYLO_SHAPE_B(A, B)                                                                                 \
+    case A * 5 + B:                                                                                       \
+        if constexpr (!LOC)                                                                               \
+            children4<A, B, T, C, TL>(op, tips, tl, tipv, plane, slot_stride, scl, ms, si, lane, cat, cin, sin,  \
+                                      xb, sB, Pl, Pr, L, sc);                                             \
         break;
         // the other shapes of children in kind order (carry A, tip, carry B,
         // stored, none)
-        PHYLO_SHAPE(2, 4) PHYLO_SHAPE(0, 3) PHYLO_SHAPE(0, 1) PHYLO_SHAPE(0, 4)
-        PHYLO_SHAPE(3, 1) PHYLO_SHAPE(3, 4) PHYLO_SHAPE(1, 1)
+        PHYLO_SHAPE(2, 4) PHYLO_SHAPE(0, 1) PHYLO_SHAPE(0, 4) PHYLO_SHAPE(1, 1)
+        PHYLO_SHAPE_B(0, 3) PHYLO_SHAPE_B(3, 1) PHYLO_SHAPE_B(3, 4)
         default: PHYLO_SHAPE(1, 4)      // (no other shape occurs: one carry A and one carry B at a time)
 #undef PHYLO_SHAPE
+#undef PHYLO_SHAPE_B
     }
     if constexpr (PIPE) load_p2<C>(nx, Pcat, nPl, nPr);
     // Carried results are FP64 and rescaled lazily: only when the
@@ -223,14 +231,14 @@ __device__ __forceinline__ void walk4_op(const Op op, const uint8_t* __restrict_
 #pragma unroll
         for (int i = 0; i < 4; ++i) r[i] = (T)round_cut(ldexp(L[i], -e), key + 0x9e3779b9u * i, T());
         store4(const_cast<T*>(plane) + op.out_slot * slot_stride, r);
-        scl[((size_t)op.out_slot * C + cat) * m_pad + s] = sc + e;
+        scl[((size_t)op.out_slot * C + cat) * ms + si] = sc + e;
     }
     // carry A takes every result (after an op to carry B nothing reads
     // the old A), so no select between the carries
 #pragma unroll
     for (int i = 0; i < 4; ++i) cout[i] = L[i];
     sout = sc;
-    const bool to_b = op.flags & OP_TO_B;
+    const bool to_b = !LOC && op.flags & OP_TO_B;
     if (to_b) {
         xb[cat][0][lane] = make_double2(L[0], L[1]);
         xb[cat][1][lane] = make_double2(L[2], L[3]);
@@ -242,7 +250,9 @@ __device__ __forceinline__ void walk4_op(const Op op, const uint8_t* __restrict_
 // it one op per turn, the result copied into carry A (the batch kernel,
 // where the second copy of the op body would cost it a resident wave).  The
 // values are the same either way.
-template <typename T, int C, bool TL, bool PAIRS = true>
+// LOC: the stored partials are LDS slots of the workgroup's 64 sites (m_pad =
+// 64; prune4_pieces_kernel), and the programs use carry A alone.
+template <typename T, int C, bool TL, bool PAIRS = true, bool LOC = false>
 __device__ inline void walk4(const Op* __restrict__ ops, int k0, int k1, const uint8_t* __restrict__ tips,
                              const uint8_t* tl, const double2* tipv, T* clv, int* scl, const double* __restrict__ P,
                              const double* __restrict__ roots, int m_pad, int s, int lane, int cat,
@@ -252,7 +262,7 @@ __device__ inline void walk4(const Op* __restrict__ ops, int k0, int k1, const u
     // sits in LDS: xb[cat][][lane], written and read by the same lane)
     double cA[4] = {0.0, 0.0, 0.0, 0.0};
     int sA = 0, sB = 0;
-    const T* plane = clv + ((size_t)cat * m_pad + s) * 4;          // + slot * C * m_pad * 4
+    const T* plane = clv + ((size_t)cat * m_pad + (LOC ? lane : s)) * 4;          // + slot * C * m_pad * 4
     const size_t slot_stride = (size_t)C * m_pad * 4;
     const char* Pcat = reinterpret_cast<const char*>(P + (size_t)cat * 16);
     double cB2[4] = {0.0, 0.0, 0.0, 0.0};
@@ -261,7 +271,7 @@ __device__ inline void walk4(const Op* __restrict__ ops, int k0, int k1, const u
     if constexpr (!PAIRS) {
         double unused[16];
         for (; k < k1; ++k) {
-            walk4_op<T, C, TL, false>(ops[k], tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
+            walk4_op<T, C, TL, false, LOC>(ops[k], tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
                                       cA, sA, sB, cB2, sA2, unused, unused, ops[k], unused, unused);
 #pragma unroll
             for (int i = 0; i < 4; ++i) cA[i] = cB2[i];
@@ -281,14 +291,14 @@ __device__ inline void walk4(const Op* __restrict__ ops, int k0, int k1, const u
         load_p2<C>(cur, Pcat, PA_l, PA_r);
         for (; op + 1 < op_end; op += 2) {
             const Op nx = op[1];
-            walk4_op<T, C, TL, true>(cur, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
+            walk4_op<T, C, TL, true, LOC>(cur, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
                                      cA, sA, sB, cB2, sA2, PA_l, PA_r, nx, PB_l, PB_r);
             cur = op[2];
-            walk4_op<T, C, TL, true>(nx, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat,
+            walk4_op<T, C, TL, true, LOC>(nx, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat,
                                      xb, cB2, sA2, sB, cA, sA, PB_l, PB_r, cur, PA_l, PA_r);
         }
         if (op < op_end) {  // an odd op count: the last op, its result back in cA
-            walk4_op<T, C, TL, true>(cur, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
+            walk4_op<T, C, TL, true, LOC>(cur, tips, tl, tipv, plane, slot_stride, scl, Pcat, m_pad, s, lane, cat, xb,
                                      cA, sA, sB, cB2, sA2, PA_l, PA_r, cur, PB_l, PB_r);
 #pragma unroll
             for (int i = 0; i < 4; ++i) cA[i] = cB2[i];
@@ -311,6 +321,10 @@ __device__ inline void walk4(const Op* __restrict__ ops, int k0, int k1, const u
     }
 }
 
+// log(lc 2^sc), the same bits in every kernel (one that contracts the
+// expression its own way could differ in the last).
+__device__ inline double site_value(double lc, int sc) { return fma((double)sc, kLn2, log(lc)); }
+
 // Site lnL from the categories' root sums (lc, sc) held by the C waves of a
 // workgroup (wave = category): the sums meet in LDS at their largest
 // exponent.  Every wave returns the same value.  REUSE: the caller writes
@@ -331,7 +345,7 @@ __device__ inline double combine_categories(double lc, int sc, int cat, int lane
         if (REUSE) __syncthreads();
         sc = M;
     }
-    return log(lc) + sc * kLn2;
+    return site_value(lc, sc);
 }
 
 // Plain launch (prog_main = -1): grid = (m_pad / 64, n_programs); workgroup
@@ -405,6 +419,78 @@ __global__ __launch_bounds__(64 * C) void prune4_kernel(
         const double v = wave_sum(live ? w * lnl : 0.0);
         if (lane == 0) *dst = v;
     }
+}
+
+// The whole tree of 64 sites in one workgroup of 16 waves: 16 / C groups of C
+// waves walk the pieces of the tree (build_split_programs), group g program
+// prog_begin[g], their results go to LDS slots, and the first group walks the
+// nodes above them (program G).  For problems of so few blocks that latency is
+// all they spend: the pieces' stores and the top program's loads one after
+// another through global memory, and the launch between them, go.  Stored
+// partials are rounded to T as in global memory, so the values are those of
+// the two launches.  n_slots LDS slots of [C][64] partials, then their scalers,
+// then the tips (64 bytes a taxon).
+// Bound by the chain: the tips' and the ops' first loads, the longest share of
+// pieces (four waves a SIMD hide part of it), the top program with one wave a
+// SIMD.  Two launches -> one, us: 32 taxa x 2000 sites, FP64, 4 categories
+// 6.5 + 8.7 -> 12.0; 50 x 4099, FP64, 1 category 6.3 + 9.7 and the sum's 3.6 ->
+// 14.0; 50 x 10,000, FP32, 4 categories 12.4 + 14.5 -> 18.2.
+template <typename T, int C>
+__global__ __launch_bounds__(1024) void prune4_pieces_kernel(
+    const Op* __restrict__ ops, const int* __restrict__ prog_begin, const uint8_t* __restrict__ tips,
+    const double* __restrict__ P, const double* __restrict__ roots, const double* __restrict__ site_w,
+    double* __restrict__ site_lnl, double* __restrict__ partial, int m, int m_pad, int n_taxa, int n_slots,
+    unsigned* fold_counter, double* fold_out) {
+    constexpr int G = 16 / C;
+    __shared__ int xsc[C][64];
+    __shared__ double xroot[C][64];
+    __shared__ double2 tipv[32];
+    __shared__ double2 xb[C][2][64];       // (never used: the programs keep no carry B)
+    extern __shared__ __align__(16) uint8_t dyn[];
+    T* const slots = reinterpret_cast<T*>(dyn);
+    int* const scl = reinterpret_cast<int*>(slots + (size_t)n_slots * C * 256);
+    uint8_t* const tl = reinterpret_cast<uint8_t*>(scl + (size_t)n_slots * C * 64);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cat = wave % C, g = wave / C, s = blockIdx.x * 64 + lane;
+    if (threadIdx.x < 32) {
+        const unsigned code = threadIdx.x & 15, h = (threadIdx.x >> 4) * 2;
+        tipv[threadIdx.x] = make_double2((double)((code >> h) & 1u), (double)((code >> (h + 1)) & 1u));
+    }
+    const uint8_t* blk = tips + (size_t)blockIdx.x * 64;
+    for (int i = threadIdx.x; i < n_taxa * 16; i += 1024) {
+        const uint32_t w = *reinterpret_cast<const uint32_t*>(blk + (size_t)(i >> 4) * m_pad + 4 * (i & 15));
+        reinterpret_cast<uint32_t*>(tl)[i] = (w << 4) & 0xF0F0F0F0u;
+    }
+    __syncthreads();
+    double lc;
+    int sc;
+    walk4<T, C, true, true, true>(ops, prog_begin[g], prog_begin[g + 1], tips, tl, tipv, slots, scl, P, roots, 64, s, lane,
+                                  cat, xb, lc, sc);
+    __syncthreads();
+    if (g == 0) {
+        walk4<T, C, true, true, true>(ops, prog_begin[G], prog_begin[G + 1], tips, tl, tipv, slots, scl, P, roots, 64, s,
+                                      lane, cat, xb, lc, sc);
+        xroot[cat][lane] = lc;
+        xsc[cat][lane] = sc;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        if (C > 1) {
+            int M = xsc[0][lane];
+#pragma unroll
+            for (int c = 1; c < C; ++c) M = max(M, xsc[c][lane]);
+            lc = 0.0;
+#pragma unroll
+            for (int c = 0; c < C; ++c) lc += ldexp(xroot[c][lane], xsc[c][lane] - M);
+            sc = M;
+        }
+        const double lnl = site_value(lc, sc);
+        const bool live = s < m;
+        if (live && site_lnl) site_lnl[s] = lnl;
+        const double v = wave_sum(live ? (site_w ? site_w[s] : 1.0) * lnl : 0.0);
+        if (lane == 0) partial[blockIdx.x] = v;
+    }
+    fold_total(partial, (int)gridDim.x, fold_counter, fold_out);
 }
 
 // Batched scoring: the whole trees of many independent problems in one
@@ -528,13 +614,16 @@ __global__ void pbuild_eigen_kernel(const double* __restrict__ V, const double* 
 // Bound by the round trip to host memory and the launch: 4.5 us at 32 and at
 // 128 taxa.  A copy in front of it cost 10 us of host time and a 3 us copy
 // kernel; a fit that changes the model each evaluation took two (59 us an
-// evaluation of 32 taxa x 2000 sites then, 37 us now).
+// evaluation of 32 taxa x 2000 sites then, 37 us without).  A new topology's
+// programs (prog_words 16-byte words of pinned memory) come along.
 struct Eig4 {
     double rate[kMaxCat], V[16], Vinv[16], lam[4];
 };
 __global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const double* __restrict__ eff, int S, int C,
-                               int n_nodes, double* __restrict__ P, double* __restrict__ d_roots) {
+                               int n_nodes, double* __restrict__ P, double* __restrict__ d_roots,
+                               const int4* __restrict__ prog, int4* __restrict__ d_prog, int prog_words) {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
+    for (int i = gid; i < prog_words; i += gridDim.x * blockDim.x) d_prog[i] = prog[i];
     if (gid < kRootDoubles) d_roots[gid] = roots.v[gid];
     if (gid >= n_nodes * C * 16) return;
     const int j = gid % 4, i = gid / 4 % 4, c = gid / 16 % C, node = gid / (16 * C);
@@ -647,6 +736,8 @@ struct phylo_ctx {
     // tail split of whole-tree DNA walks (build_split_programs): split_K chunk
     // programs from program id split_base[full ? 0 : 1], then one top program
     int split_K = 0, split_base[2] = {0, 0};
+    int fused_base = 0, fused_slots = 0;                  // prune4_pieces_kernel's programs, LDS slots (0: none)
+    int max_lds = 0;                                      // bytes of LDS a workgroup may have
     bool split_all = false;                               // every block walks the pieces (too few blocks)
     bool tail_split = true;                               // phylo_set_tail_split
     int n_cu = 0;                                         // compute units of the device
@@ -663,6 +754,7 @@ struct phylo_ctx {
     double* d_P = nullptr; size_t P_bytes = 0;
     Op* d_ops = nullptr; size_t ops_bytes = 0;
     int* d_prog = nullptr;                               // in d_ops' buffer, after the ops
+    size_t prog_bytes = 0;                               // staged for d_ops' buffer and not yet copied
     double* d_PmT = nullptr; size_t PmT_bytes = 0;       // P transposed in MFMA operand order (NNI walks)
     bool want_PmT = false;                                // NNI walks have asked for d_PmT
     // NNI walks of the current topology (nni_program.h), rebuilt when it changes
@@ -770,16 +862,16 @@ hipError_t stage_acquire(phylo_ctx* c, phylo_ctx::Stage& st, size_t n) {
     return hipSuccess;
 }
 
-// Copies the compiled programs to the device in one piece: the ops, children
+// Stages the compiled programs for one copy to the device: the ops, children
 // in kind order, one zero op (the walkers read the op after the one they run,
 // up to ops[end] of the last program: the DNA walker to load its P matrices
 // early, the matrix walker to have the descriptor at hand), then the programs'
 // bounds.
-hipError_t upload_programs(phylo_ctx* c) {
+hipError_t stage_programs(phylo_ctx* c) {
     order_children(c->ops);
     const size_t n_op = c->ops.size(), op_bytes = (n_op + 1) * sizeof(Op);
-    const size_t bytes = op_bytes + c->prog_begin.size() * sizeof(int);
-    hipError_t e = stage_acquire(c, c->stage_prog, (bytes + sizeof(double) - 1) / sizeof(double));
+    const size_t bytes = (op_bytes + c->prog_begin.size() * sizeof(int) + 15) / 16 * 16;
+    hipError_t e = stage_acquire(c, c->stage_prog, bytes / sizeof(double));
     if (e != hipSuccess) return e;
     Op* h = reinterpret_cast<Op*>(c->stage_prog.h);
     std::copy(c->ops.begin(), c->ops.end(), h);
@@ -787,7 +879,8 @@ hipError_t upload_programs(phylo_ctx* c) {
     std::copy(c->prog_begin.begin(), c->prog_begin.end(), reinterpret_cast<int*>(h + n_op + 1));
     if ((e = ensure(c->d_ops, c->ops_bytes, bytes)) != hipSuccess) return e;
     c->d_prog = reinterpret_cast<int*>(c->d_ops + n_op + 1);
-    return hipMemcpyAsync(c->d_ops, h, bytes, hipMemcpyHostToDevice, c->stream);
+    c->prog_bytes = bytes;       // (to be copied by the P kernel, or prepare)
+    return hipSuccess;
 }
 
 // Waits for everything on the context's stream.
@@ -907,6 +1000,16 @@ bool root_ops_last(const std::vector<Op>& ops, const std::vector<int>& begin) {
     return true;
 }
 
+// Waves of prune4_pieces_kernel's workgroups.
+constexpr int kFusedWaves = 16;
+// LDS of one of its workgroups: dynamic, with its static arrays.
+constexpr size_t kFusedStaticLds = 8192;     // (at most 6736 bytes: 8 categories)
+size_t fused_dyn_lds(const phylo_ctx* c) {
+    const size_t elt = c->prec == PHYLO_PREC_FP64 ? sizeof(double) : sizeof(float);
+    return (size_t)c->fused_slots * c->C * 64 * (4 * elt + sizeof(int)) + tip_lds_bytes(c->n_taxa);
+}
+size_t fused_lds_bytes(const phylo_ctx* c) { return fused_dyn_lds(c) + kFusedStaticLds; }
+
 // Clears the stores of ops[begin, end) whose result no op of that range reads
 // back from memory: results consumed only through the two carries.  With the
 // second carry only results that wait while a branching subtree is walked keep
@@ -946,8 +1049,10 @@ void drop_unread_stores(std::vector<Op>& ops, size_t begin, size_t end) {
 // storing and the lean evaluation, split_K chunk programs and one top program
 // to c->ops / c->prog_begin; split_K stays 0 when no cut keeps the top
 // program short (a caterpillar tree, say) or the tree is small.
+// (For prune4_pieces_kernel also a program for each of its groups of waves and
+// the top program once more, over LDS slots.)
 bool build_split_programs(phylo_ctx* c, int max_chunks, bool split_all) {
-    c->split_K = 0;
+    c->split_K = c->fused_slots = 0;
     const int nt = c->n_taxa, nn = c->n_nodes, root = c->root;
     const std::vector<int> post = internal_postorder(c, c->left, c->right);
     const int ni = (int)post.size();
@@ -959,43 +1064,67 @@ bool build_split_programs(phylo_ctx* c, int max_chunks, bool split_all) {
         if (l >= 0) par[l] = v;
         if (r >= 0) par[r] = v;
     }
-    // pieces: the largest subtrees of at most L internal nodes, in postorder;
-    // a subtree's internal nodes are the size[v] entries of post ending at v
-    const auto cut = [&](int L, std::vector<std::vector<int>>& chunks, std::vector<int>& top) {
-        chunks.clear();
+    // pieces: the largest subtrees of at most L internal nodes, in postorder; a
+    // subtree's internal nodes are the size[v] entries of post ending at v.
+    // Chunk k takes the pieces up to chunk_end[k].
+    struct Piece { int begin, n; };
+    std::vector<Piece> pieces;
+    std::vector<int> chunk_end, top;
+    size_t big = 0;                              // longest chunk
+    const auto cut = [&](int L) {
+        pieces.clear();
+        chunk_end.clear();
         top.clear();
-        std::vector<int> cur;
+        big = 0;
         int cur_n = 0;
         for (int i = 0; i < ni; ++i) {
             const int v = post[i];
             if (size[v] > L) { top.push_back(v); continue; }
             if (v != root && size[par[v]] <= L) continue;     // inside a larger piece
-            if (cur_n > 0 && cur_n + size[v] > L) { chunks.push_back(cur); cur.clear(); cur_n = 0; }
-            for (int k = i - size[v] + 1; k <= i; ++k) cur.push_back(post[k]);
+            if (cur_n > 0 && cur_n + size[v] > L) { chunk_end.push_back((int)pieces.size()); cur_n = 0; }
+            pieces.push_back({i - size[v] + 1, size[v]});
             cur_n += size[v];
+            big = std::max(big, (size_t)cur_n);
         }
-        if (cur_n > 0) chunks.push_back(cur);
+        if (cur_n > 0) chunk_end.push_back((int)pieces.size());
     };
-    int best_L = -1;
-    double best_cost = 1e30;
-    std::vector<std::vector<int>> chunks;
-    std::vector<int> top;
+    // prune4_pieces_kernel's share of the pieces: longest first, each to the
+    // group with the least so far; returns the longest share
+    const int nblk = c->m_pad / 64;
+    const int G = split_all && !uses_mfma(c) && nt <= kTipLdsTaxa && nblk <= c->n_cu ? kFusedWaves / c->C : 0;
+    std::vector<int> by, group_of, load(G);
+    const auto share = [&]() {
+        by.resize(pieces.size());
+        group_of.resize(pieces.size());
+        for (size_t i = 0; i < by.size(); ++i) by[i] = (int)i;
+        std::sort(by.begin(), by.end(), [&](int a, int b) {
+            return pieces[a].n != pieces[b].n ? pieces[a].n > pieces[b].n : a < b;
+        });
+        std::fill(load.begin(), load.end(), 0);
+        for (int i : by) {
+            const int g = (int)(std::min_element(load.begin(), load.end()) - load.begin());
+            group_of[i] = g;
+            load[g] += pieces[i].n;
+        }
+        return *std::max_element(load.begin(), load.end());
+    };
+    int best_L = -1, best_fused_L = -1;
+    double best_cost = 1e30, best_fused = 1e30;
     // piece sizes to try: fractions of the tree, and (so that few large
     // pieces are possible) the sizes of the subtrees near the root
-    std::vector<int> Ls;
-    for (int d : {16, 12, 10, 8, 6, 5, 4, 3, 2}) Ls.push_back(std::max(1, ni / d));
+    int Ls[15], n_L = 0;
+    for (int d : {16, 12, 10, 8, 6, 5, 4, 3, 2}) Ls[n_L++] = std::max(1, ni / d);
     for (int v : {c->left[root], c->right[root]})
         if (v >= nt) {
-            Ls.push_back(size[v]);
+            Ls[n_L++] = size[v];
             for (int w : {c->left[v], c->right[v]})
-                if (w >= nt) Ls.push_back(size[w]);
+                if (w >= nt) Ls[n_L++] = size[w];
         }
-    for (int L : Ls) {
-        if (size[root] <= L) continue;
-        cut(L, chunks, top);
-        size_t big = 0;
-        for (const auto& ch : chunks) big = std::max(big, ch.size());
-        if (chunks.size() < 2 || top.size() > 16 || (int)chunks.size() > max_chunks) continue;
+    for (int k = 0; k < n_L; ++k) {
+        const int L = Ls[k];
+        if (size[root] <= L || std::find(Ls, Ls + k, L) != Ls + k) continue;
+        cut(L);
+        if (chunk_end.size() < 2 || top.size() > 16 || (int)chunk_end.size() > max_chunks) continue;
         // Tail split: the top program runs alone, about 0.7 us per op; a
         // chunk shares a CU with main blocks and costs nothing until it is
         // longer than about 0.4 of the whole walk, then about 0.5 us per op
@@ -1006,35 +1135,89 @@ bool build_split_programs(phylo_ctx* c, int max_chunks, bool split_all) {
         const double over = std::max(0.0, (double)big - 0.4 * ni);
         const double cost = split_all ? (double)big + (double)top.size() : (double)top.size() + 0.7 * over;
         if (cost < best_cost) { best_cost = cost; best_L = L; }
+        if (G > 0)
+            if (const double f = (double)share() + (double)top.size(); f < best_fused) { best_fused = f; best_fused_L = L; }
     }
     if (best_L < 0) return false;
-    cut(best_L, chunks, top);
-    const auto emit = [&](const std::vector<int>& nodes, bool store_all) {
-        for (size_t i = 0; i < nodes.size(); ++i) {
+    // One workgroup a block for all pieces, or one a chunk: the first saves a
+    // launch and the global round trips, the second spreads the chain over idle
+    // CUs.  us an evaluation, two launches / one, 4 categories, FP32, 2000
+    // sites (32 blocks): 20 taxa 25 / 23, 50 taxa 29 / 28, 120 taxa (chains of
+    // about 28 and 38 ops) 33 / 38, 250 taxa 42 / 56; 9000 sites (144 blocks,
+    // which leave the chunks few idle CUs): 29 / 25, 35 / 30, 44 / 40, 63 / 58;
+    // 16,384 (256 blocks): 32 / 27, 41 / 33, 55 / 42, 79 / 60.  One category
+    // (16 groups, and the total folded in): 28 / 21, 32 / 24, 38 / 26, 48 / 33
+    // at 2000 sites.  Past a block a CU it loses (50 taxa, 1 category, 768
+    // blocks: 38 / 48).
+    bool fused = G > 0 && (best_fused <= best_cost + 3.0 || 2 * nblk >= c->n_cu);
+    // with free_slots (prune4_pieces_kernel): lean, stores to LDS slots
+    std::vector<int> lds_slot(fused ? nn : 0, -1);
+    const auto emit = [&](const int* nodes, int n, bool store_all, std::vector<int>* free_slots = nullptr) {
+        for (int i = 0; i < n; ++i) {
             const int v = nodes[i], l = c->left[v], r = c->right[v];
             const auto src = [&](int ch, int& kind, int& idx) {
                 if (ch < 0) { kind = SRC_NONE; idx = 0; }
                 else if (ch < nt) { kind = SRC_TIP; idx = ch; }
                 else if (i > 0 && nodes[i - 1] == ch) { kind = SRC_CARRY_A; idx = 0; }
-                else { kind = SRC_CLV; idx = ch - nt; }
+                else if (!free_slots) { kind = SRC_CLV; idx = ch - nt; }
+                else {
+                    kind = SRC_CLV;
+                    idx = lds_slot[ch];
+                    free_slots->push_back(idx);      // its one reader
+                }
             };
             Op op{};
             op.l_node = l;
             op.r_node = r < 0 ? 0 : r;
             src(l, op.l_kind, op.l_idx);
             src(r, op.r_kind, op.r_idx);
-            const bool next_reads = i + 1 < nodes.size() && par[v] == nodes[i + 1];
+            const bool next_reads = i + 1 < n && par[v] == nodes[i + 1];
             op.out_slot = (store_all || !next_reads) ? v - nt : -1;
+            if (free_slots && op.out_slot >= 0) {
+                if (v == root) op.out_slot = -1;     // (nothing reads it)
+                else if (free_slots->empty()) op.out_slot = lds_slot[v] = c->fused_slots++;
+                else {
+                    op.out_slot = lds_slot[v] = free_slots->back();
+                    free_slots->pop_back();
+                }
+            }
             op.flags = v == root ? OP_ROOT : 0;
             c->ops.push_back(op);
         }
-        c->prog_begin.push_back((int)c->ops.size());
     };
-    c->split_K = (int)chunks.size();
+    const auto end_program = [&]() { c->prog_begin.push_back((int)c->ops.size()); };
+    if (fused) {
+        const size_t n_ops = c->ops.size(), n_prog = c->prog_begin.size();
+        cut(best_fused_L);
+        (void)share();
+        c->fused_base = (int)n_prog - 1;
+        std::vector<int> spare, mine;              // free slots: of all groups (for the top program), of one
+        for (int g = 0; g < G; ++g) {
+            mine.clear();
+            for (size_t p = 0; p < pieces.size(); ++p)
+                if (group_of[p] == g) emit(&post[pieces[p].begin], pieces[p].n, false, &mine);
+            end_program();
+            spare.insert(spare.end(), mine.begin(), mine.end());
+        }
+        emit(top.data(), (int)top.size(), false, &spare);
+        end_program();
+        fused = fused_lds_bytes(c) <= (size_t)c->max_lds;
+        if (!fused) {                              // too many results at once for the LDS
+            c->ops.resize(n_ops);
+            c->prog_begin.resize(n_prog);
+            c->fused_slots = 0;
+        }
+    }
+    if (!fused) cut(best_L);
+    c->split_K = (int)chunk_end.size();
     for (int mode = 0; mode < 2; ++mode) {     // 0: store every partial, 1: lean
         c->split_base[mode] = (int)c->prog_begin.size() - 1;
-        for (const auto& ch : chunks) emit(ch, mode == 0);
-        emit(top, mode == 0);
+        for (size_t k = 0, p = 0; k < chunk_end.size(); ++k) {
+            for (; (int)p < chunk_end[k]; ++p) emit(&post[pieces[p].begin], pieces[p].n, mode == 0);
+            end_program();
+        }
+        emit(top.data(), (int)top.size(), mode == 0);
+        end_program();
     }
     return true;
 }
@@ -1168,8 +1351,11 @@ int upload_pmatrices(phylo_ctx* c) {
         std::copy(c->Vinv.begin(), c->Vinv.end(), e.Vinv);
         std::copy(c->lam.begin(), c->lam.end(), e.lam);
         hipLaunchKernelGGL(pbuild4_kernel, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0, c->stream, e, root_weights(c),
-                           c->stage_len.dev, S, c->C, c->n_nodes, c->d_P, c->d_roots);
+                           c->stage_len.dev, S, c->C, c->n_nodes, c->d_P, c->d_roots,
+                           reinterpret_cast<const int4*>(c->stage_prog.dev), reinterpret_cast<int4*>(c->d_ops),
+                           (int)(c->prog_bytes / 16));
         HIPCHK(c, hipGetLastError());
+        c->prog_bytes = 0;
         c->dirty_roots = false;
     }
     c->dirty_P = false;
@@ -1217,7 +1403,7 @@ int prepare(phylo_ctx* c) {
         int rc = compile_full_program(c);
         if (rc) return rc;
         if (!root_ops_last(c->ops, c->prog_begin)) return fail(c, PHYLO_ERR_STATE, "internal: root op not last");
-        HIPCHK(c, upload_programs(c));
+        HIPCHK(c, stage_programs(c));
         c->dirty_topo = false;
         c->walks.mode = -1;
     }
@@ -1229,6 +1415,10 @@ int prepare(phylo_ctx* c) {
     if (c->dirty_P) {
         int rc = upload_pmatrices(c);
         if (rc) return rc;
+    }
+    if (c->prog_bytes) {
+        HIPCHK(c, hipMemcpyAsync(c->d_ops, c->stage_prog.h, c->prog_bytes, hipMemcpyHostToDevice, c->stream));
+        c->prog_bytes = 0;
     }
     if (c->dirty_roots) {
         if (!c->d_roots) HIPCHK(c, hipMalloc(&c->d_roots, kRootDoubles * sizeof(double)));
@@ -1256,6 +1446,14 @@ void launch_prune4(phylo_ctx* c, dim3 grid, double* site_lnl) {
     const double* sw = c->have_site_w ? c->d_sitew : nullptr;
     if (c->run_whole_tree && c->n_taxa <= kTipLdsTaxa) {
         const int nblk = (int)grid.x;
+        if (c->tail_split && c->fused_slots > 0 && !c->run_full && grid.y == 1 &&
+            fused_lds_bytes(c) <= (size_t)c->max_lds) {      // (the precision may have changed since)
+            hipLaunchKernelGGL((prune4_pieces_kernel<T, C>), grid, dim3(64 * kFusedWaves), fused_dyn_lds(c), c->stream,
+                               c->d_ops, c->d_prog + c->fused_base, tips, c->d_P, c->d_roots, sw, site_lnl, c->d_partial,
+                               c->m, c->m_pad, c->n_taxa, c->fused_slots, c->d_fold, c->h_total_dev);
+            c->folded = true;
+            return;
+        }
         const int main_b = split_main_blocks(c, nblk), tail = nblk - main_b;
         if (c->tail_split && c->split_K > 0 && grid.y == 1 && tail > 0) {
             // the main blocks and the tail's pieces, then the tail's top program
@@ -1559,7 +1757,8 @@ int phylo_create(int device, phylo_ctx** out) {
     c->device = device;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&c->ev0) != hipSuccess || hipEventCreate(&c->ev1) != hipSuccess ||
-        hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) {
+        hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+        hipDeviceGetAttribute(&c->max_lds, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess) {
         phylo_destroy(c);
         return PHYLO_ERR_HIP;
     }
@@ -1711,6 +1910,7 @@ int phylo_set_categories(phylo_ctx* c, int n_cat, const double* rates, const dou
     for (int k = 0; k < n_cat; ++k)
         if (!(rates[k] >= 0.0) || !(weights[k] >= 0.0) || !std::isfinite(rates[k]))
             return fail(c, PHYLO_ERR_ARG, "set_categories: rates and weights must be finite and >= 0");
+    if (n_cat != c->C) c->dirty_topo = true;      // the split programs depend on it
     c->C = n_cat;
     c->cat_rate.assign(rates, rates + n_cat);
     c->cat_w.assign(weights, weights + n_cat);

@@ -143,14 +143,14 @@ __device__ inline void two_sum_add(double& hi, double& lo, double b, double bl) 
 // Threads of the compensated sum: one workgroup per program.
 constexpr int kSumThreads = 256;
 
-// Compensated fixed-order sum of partial[0, n) by one workgroup of
-// kSumThreads.  Each thread issues its loads eight at a time before adding
+// Compensated fixed-order sum of partial[0, n) by the first kSumThreads
+// threads of one workgroup.  Each thread issues its loads eight at a time before adding
 // them (Kahan), so their latencies overlap instead of queueing; the threads'
 // (sum, error) pairs then meet by two-sum, in a butterfly within each wave
 // and in LDS across the waves.  Thread 0 returns the total.
 __device__ inline double block_total(const double* partial, int n) {
     double s = 0.0, comp = 0.0;
-    for (int base = threadIdx.x; base < n; base += 8 * kSumThreads) {
+    for (int base = threadIdx.x < kSumThreads ? (int)threadIdx.x : n; base < n; base += 8 * kSumThreads) {
         double v[8];
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
@@ -172,7 +172,7 @@ __device__ inline double block_total(const double* partial, int n) {
     for (int o = 32; o > 0; o >>= 1) two_sum_add(hi, lo, __shfl_xor(hi, o, 64), __shfl_xor(lo, o, 64));
     __shared__ double red_hi[kSumThreads / 64], red_lo[kSumThreads / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    if (lane == 0) { red_hi[wid] = hi; red_lo[wid] = lo; }
+    if (lane == 0 && wid < kSumThreads / 64) { red_hi[wid] = hi; red_lo[wid] = lo; }
     __syncthreads();
     hi = red_hi[0];
     lo = red_lo[0];
@@ -201,7 +201,7 @@ __device__ inline void block_sum_store(double v, double* dst) {
 // partial in block_total's order (so the total equals final_sum_kernel's),
 // writes it to the host-mapped total and returns the counter to zero.  The
 // fences publish the few partials this launch wrote and drop stale copies
-// before the sum reads them.  Workgroups of kSumThreads threads only.
+// before the sum reads them.  Workgroups of kSumThreads threads or more only.
 __device__ inline void fold_total(const double* partial, int n_part, unsigned* counter, double* total) {
     __shared__ int last;
     if (threadIdx.x == 0) {
