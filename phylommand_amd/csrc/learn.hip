@@ -20,10 +20,11 @@
 
 namespace {
 
-constexpr int kSimThreads = 256;
+constexpr int kSimThreads = 512;
 constexpr int kMaxSimTaxa = 32;
 constexpr int kMaxSimNodes = 2 * kMaxSimTaxa - 1;
 constexpr int kMaxSimCat = 8;
+constexpr int kSimPairs = (kMaxSimTaxa * (kMaxSimTaxa - 1) / 2 + kSimThreads - 1) / kSimThreads;   // a thread, at most
 constexpr int kFeat = 256;
 
 __device__ inline uint64_t mix64(uint64_t z) {
@@ -40,13 +41,17 @@ __device__ inline float urand(uint64_t seed, uint64_t a, uint64_t b, uint64_t c)
 // One workgroup per alignment.  Per-alignment inputs (eig = V[16], Vinv[16],
 // lam[4]; pi[4]; cat_rates[C]) give P(t) = V exp(lam r t) Vinv in LDS as
 // cumulative rows; walk holds the nodes in preorder as node | parent << 8.
-// Each thread simulates one site of a 256-site chunk down the tree; a tip's
-// states leave as four ballot words a wave (one bit a site and state), so the
-// joint state counts of a pair of taxa are 16 popcounts of ANDed words per 64
-// sites.  (A byte a site, counted site by site into an array indexed at run
-// time, which lies in scratch memory, took 1.42 ms for 512 alignments of 32
-// taxa x 2,000 sites.)  What is left is the generator: three 64-bit mixes a
-// draw, 94 draws a site.
+// Each thread simulates one site of a chunk down the tree; a tip's states leave
+// as four ballot words a wave (one bit a site and state), so the joint state
+// counts of a pair of taxa are 16 popcounts of ANDed words per 64 sites.  (A
+// byte a site, counted site by site into an array indexed at run time, which
+// lies in scratch memory, took 1.42 ms for 512 alignments of 32 taxa x 2,000
+// sites.)  Bound by the generator, three 64-bit mixes a draw, 94 draws a site,
+// and by the chain of states down the tree behind it: eight waves a workgroup,
+// so that 512 alignments give every SIMD four (four waves, two a SIMD, 0.40 ms;
+// eight 0.31; sixteen 0.34, half of them without a pair to count).  A table of
+// the innermost mixes, which the alignments share, made the kernel a tenth
+// faster and its own launch and allocation took that back.
 __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
     int n_taxa, int n_sites, int n_cat, const int* __restrict__ walk, const double* __restrict__ blen,
     const double* __restrict__ eig, const double* __restrict__ pi_all, const double* __restrict__ cat_all,
@@ -56,7 +61,7 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
     const int n_nodes = 2 * n_taxa - 1;
     extern __shared__ __align__(16) float cumP[];       // [n_nodes][n_cat][4][4]
     __shared__ unsigned char st[kMaxSimNodes - kMaxSimTaxa][kSimThreads];   // inner nodes' states
-    __shared__ __align__(16) uint64_t tip[kMaxSimTaxa][kSimThreads / 64][4];    // [taxon][wave][state]
+    __shared__ uint64_t tip[kMaxSimTaxa][kSimThreads / 16 + 1];    // [taxon][wave, state]; odd rows: no bank conflicts
     __shared__ float cum_pi[4];
     __shared__ int h_site[4 + 32 + 32];
     __shared__ float h_pair[16 + 32 + 32 + 32 + 8];
@@ -97,11 +102,12 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         row[3] = 1.0f;
     }
     __syncthreads();
-    // pair ownership: thread owns pairs p = tid, tid + 256 (496 pairs for 32 taxa)
+    // pair ownership: thread owns pairs p = tid, tid + kSimThreads, ... (496 pairs for 32 taxa)
     const int n_pairs = n_taxa * (n_taxa - 1) / 2;
-    int pa[2] = {-1, -1}, pb[2] = {-1, -1};
+    int pa[kSimPairs], pb[kSimPairs];
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < kSimPairs; ++q) {
+        pa[q] = pb[q] = -1;
         int p = tid + q * kSimThreads;
         if (p >= n_pairs) continue;
         int i = 0;
@@ -109,70 +115,72 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
         pa[q] = i;
         pb[q] = i + 1 + p;
     }
-    int joint[2][16];
+    int joint[kSimPairs][16];
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < kSimPairs; ++q)
 #pragma unroll
         for (int c = 0; c < 16; ++c) joint[q][c] = 0;
     int base_count = 0;      // threads < 4 n_taxa: state tid % 4 of taxon tid / 4
     for (int s0 = 0; s0 < n_sites; s0 += kSimThreads) {
-        const int s = s0 + tid;
-        const bool live = s < n_sites;      // (the other lanes draw too: the ballots need every lane)
-        const int cat = n_cat > 1 ? min(n_cat - 1, (int)(urand(seed, a, s, 1u << 20) * n_cat)) : 0;
-        const float u = urand(seed, a, s, (1u << 20) + 1);
-        // the first state whose cumulative value exceeds u (3 at the end)
-        int rs = !(u < cum_pi[0]);
-        rs += rs == 1 && !(u < cum_pi[1]);
-        rs += rs == 2 && !(u < cum_pi[2]);
-        st[walk[0] - n_taxa][tid] = (unsigned char)rs;
-        uint32_t cnt = 0;        // tips per state, a byte each
-        for (int k = 1; k < n_nodes; ++k) {
-            const int w = walk[k], v = w & 255;
-            const int anc = st[(w >> 8) - n_taxa][tid];
-            const float r = urand(seed, a, s, (uint64_t)v);
-            const float4 row = *reinterpret_cast<const float4*>(cumP + (((size_t)v * n_cat + cat) * 4 + anc) * 4);
-            int x = !(r < row.x);
-            x += x == 1 && !(r < row.y);
-            x += x == 2 && !(r < row.z);
-            if (v >= n_taxa) {
-                st[v - n_taxa][tid] = (unsigned char)x;
-                continue;
+        const int s = s0 + tid, waves = min(kSimThreads / 64, (n_sites - s0 + 63) / 64);    // (that have a site)
+        const bool live = s < n_sites;      // (its wave's other lanes draw too: the ballots need every lane)
+        if (wave < waves) {
+            const int cat = n_cat > 1 ? min(n_cat - 1, (int)(urand(seed, a, s, 1u << 20) * n_cat)) : 0;
+            const float u = urand(seed, a, s, (1u << 20) + 1);
+            // the first state whose cumulative value exceeds u (3 at the end)
+            int rs = !(u < cum_pi[0]);
+            rs += rs == 1 && !(u < cum_pi[1]);
+            rs += rs == 2 && !(u < cum_pi[2]);
+            st[walk[0] - n_taxa][tid] = (unsigned char)rs;
+            uint32_t cnt = 0;        // tips per state, a byte each
+            for (int k = 1; k < n_nodes; ++k) {
+                const int w = walk[k], v = w & 255;
+                const int anc = st[(w >> 8) - n_taxa][tid];
+                const float r = urand(seed, a, s, (uint64_t)v);
+                const float4 row = *reinterpret_cast<const float4*>(cumP + (((size_t)v * n_cat + cat) * 4 + anc) * 4);
+                int x = !(r < row.x);
+                x += x == 1 && !(r < row.y);
+                x += x == 2 && !(r < row.z);
+                if (v >= n_taxa) {
+                    st[v - n_taxa][tid] = (unsigned char)x;
+                    continue;
+                }
+                // a tip: gaps, its states' words
+                const bool ok = live && !(gap_frac > 0.f && urand(seed, a, s, (2u << 20) + v) < gap_frac);
+                cnt += ok ? 1u << (8 * x) : 0u;
+                const uint64_t m0 = __ballot(ok && x == 0), m1 = __ballot(ok && x == 1), m2 = __ballot(ok && x == 2),
+                               m3 = __ballot(ok && x == 3);
+                if (lane < 4) tip[v][4 * wave + lane] = lane == 0 ? m0 : lane == 1 ? m1 : lane == 2 ? m2 : m3;
+                if (masks_out && live) masks_out[((size_t)a * n_taxa + v) * n_sites + s] = ok ? 1u << x : 15u;
             }
-            // a tip: gaps, its states' words
-            const bool ok = live && !(gap_frac > 0.f && urand(seed, a, s, (2u << 20) + v) < gap_frac);
-            cnt += ok ? 1u << (8 * x) : 0u;
-            const uint64_t m0 = __ballot(ok && x == 0), m1 = __ballot(ok && x == 1), m2 = __ballot(ok && x == 2),
-                           m3 = __ballot(ok && x == 3);
-            if (lane < 4) tip[v][wave][lane] = lane == 0 ? m0 : lane == 1 ? m1 : lane == 2 ? m2 : m3;
-            if (masks_out && live) masks_out[((size_t)a * n_taxa + v) * n_sites + s] = ok ? 1u << x : 15u;
-        }
-        if (live) {
-            int distinct = 0, mx = 0, sq = 0, n_ok = 0;
+            if (live) {
+                int distinct = 0, mx = 0, sq = 0, n_ok = 0;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = cnt >> (8 * j) & 255;
-                n_ok += c;
-                distinct += c > 0;
-                mx = max(mx, c);
-                sq += c * c;
+                for (int j = 0; j < 4; ++j) {
+                    const int c = cnt >> (8 * j) & 255;
+                    n_ok += c;
+                    distinct += c > 0;
+                    mx = max(mx, c);
+                    sq += c * c;
+                }
+                if (distinct > 0) atomicAdd(&h_site[distinct - 1], 1);
+                if (distinct == 1) atomicAdd(&invariant, 1);
+                // minor-allele fraction (n - max) / n in bins of 1/64 and
+                // Gini-Simpson diversity 1 - sum f^2 in bins of 3/128, both from
+                // integers so the bin edges are exact
+                const int nn2 = n_ok * n_ok;
+                atomicAdd(&h_site[4 + (n_ok ? min(31, 64 * (n_ok - mx) / n_ok) : 0)], 1);
+                atomicAdd(&h_site[36 + (n_ok ? min(31, 128 * (nn2 - sq) / (3 * nn2)) : 0)], 1);
             }
-            if (distinct > 0) atomicAdd(&h_site[distinct - 1], 1);
-            if (distinct == 1) atomicAdd(&invariant, 1);
-            // minor-allele fraction (n - max) / n in bins of 1/64 and
-            // Gini-Simpson diversity 1 - sum f^2 in bins of 3/128, both from
-            // integers so the bin edges are exact
-            const int nn2 = n_ok * n_ok;
-            atomicAdd(&h_site[4 + (n_ok ? min(31, 64 * (n_ok - mx) / n_ok) : 0)], 1);
-            atomicAdd(&h_site[36 + (n_ok ? min(31, 128 * (nn2 - sq) / (3 * nn2)) : 0)], 1);
         }
         __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < kSimPairs; ++q) {
             if (pa[q] < 0) continue;
-            for (int w = 0; w < kSimThreads / 64; ++w) {
+            for (int w = 0; w < waves; ++w) {
                 uint64_t x[4], y[4];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) { x[j] = tip[pa[q]][w][j]; y[j] = tip[pb[q]][w][j]; }
+                for (int j = 0; j < 4; ++j) { x[j] = tip[pa[q]][4 * w + j]; y[j] = tip[pb[q]][4 * w + j]; }
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -180,12 +188,12 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
             }
         }
         if (tid < 4 * n_taxa)
-            for (int w = 0; w < kSimThreads / 64; ++w) base_count += __popcll(tip[tid >> 2][w][tid & 3]);
+            for (int w = 0; w < waves; ++w) base_count += __popcll(tip[tid >> 2][4 * w + (tid & 3)]);
         __syncthreads();
     }
     // pair statistics
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < kSimPairs; ++q) {
         if (pa[q] < 0) continue;
         int n = 0;
 #pragma unroll
