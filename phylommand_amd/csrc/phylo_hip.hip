@@ -1923,7 +1923,7 @@ int phylo_set_categories(phylo_ctx* c, int n_cat, const double* rates, const dou
 namespace {
 // One evaluation of the current inputs; `full` stores every internal node's
 // partial, otherwise only those the walk reads back.
-int evaluate(phylo_ctx* c, bool full, double* site_lnl, double* total) {
+static int evaluate(phylo_ctx* c, bool full, double* site_lnl, double* total) {
     int rc = prepare(c);
     if (rc) return rc;
     c->clv_valid = false;
@@ -2034,7 +2034,7 @@ namespace {
 
 // A neighbourhood: every variant by the outer-partial walks, against the
 // stored partials of an evaluation that kept them all.
-int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* lnl, int32_t* node, int32_t* side,
+static int score_walks(phylo_ctx* c, int mode, int max_variants, double base, double* lnl, int32_t* node, int32_t* side,
                 int* n_variants, double* base_lnl) {
     auto& w = c->walks;
     const bool mfma = uses_mfma(c);
