@@ -105,8 +105,9 @@ int phylo_set_keep_partials(phylo_ctx *ctx, int keep);
  * evenly among the GPU's CUs walks the blocks past the last full round (the
  * tail) as subtree pieces beside the other blocks plus a short second launch
  * for the nodes above the cut (enable != 0, the default), or as whole-tree
- * workgroups.  Values differ only by the FP32 rounding of the extra stored
- * partials of the tail sites (FP64 storage: bit-identical).  No counterpart
+ * workgroups; with few blocks it walks every block that way, in one workgroup
+ * where that is faster.  Values differ only by the FP32 rounding of the extra
+ * stored partials of the sites walked in pieces (FP64 storage: bit-identical).  No counterpart
  * in the reference (a launch-shape choice); kept switchable for tests. */
 int phylo_set_tail_split(phylo_ctx *ctx, int enable);
 
@@ -132,9 +133,10 @@ int phylo_get_pmatrix(phylo_ctx *ctx, int node, double *P);
  * treebender --nni all emits after the original (internal branches 2..n-3,
  * left then right swap, 2*(n-4) variants; treebender.cpp:897-915 with
  * tree::nni / tree::interchange, tree.cpp:2480-2548); mode 1: the full
- * unrooted neighbourhood, 2*(n-3) variants.  Each variant recomputes only the
- * two re-attached nodes and the path to the root against the stored partials
- * of the current tree (evaluated first if stale), all variants in one launch.
+ * unrooted neighbourhood, 2*(n-3) variants.  One preorder walk carries the
+ * partial of everything outside each subtree and scores both interchanges of
+ * an edge from it and the stored partials of the current tree (evaluated first
+ * if stale).  Exchanging the missing child of a single-child node keeps the tree.
  * Branch lengths move with their subtrees, as in interchange.  lnl: one total
  * per variant (capacity max_variants); node/side (nullable): the interchanged
  * node and side (0 left, 1 right); *n_variants: the count; base_lnl
@@ -156,8 +158,9 @@ int phylo_nni_score(phylo_ctx *ctx, int mode, int max_variants, double *lnl, int
  * clock and cannot be reproduced. */
 int phylo_simulate(phylo_ctx *ctx, int n_sites, const double *root_freq, uint64_t seed, uint8_t *states);
 
-/* Number of partial-recompute ops the last phylo_nni_score ran (updates
- * per site and category), for throughput accounting. */
+/* Number of partial updates (per site and category) that recomputing every
+ * variant of the last phylo_nni_score along its path to the root would take,
+ * for throughput accounting. */
 int phylo_nni_ops(phylo_ctx *ctx, long *n_ops);
 
 /* Waits for all work on the context's device (hipDeviceSynchronize). */
@@ -192,9 +195,9 @@ int phylo_loglik_noalloc(phylo_ctx *ctx, int n_taxa, int n_sites, int n_states, 
 
 /* ---- Batched scoring ------------------------------------------------------
  * Many independent DNA problems (S <= 4) of uneven taxon and site counts,
- * each optionally with its whole NNI neighbourhood, scored by two persistent
- * work-queue launches (full evaluations, then partial-recompute variants)
- * captured once into a HIP graph and replayed by phylo_batch_run.  All
+ * each optionally with its whole NNI neighbourhood, scored by one persistent
+ * work-queue launch (full evaluations) and one of NNI walks over the partials
+ * it stored, captured once into a HIP graph and replayed by phylo_batch_run.  All
  * problems share the number of rate categories and the precision.
  * Replaces: running treeator once per tree file / per treebender --nni tree
  * (treeator.cpp:705-990), which has no batching. */
@@ -220,8 +223,8 @@ int phylo_batch_set_tiling(phylo_batch *b, int sites_per_item, int category_wave
 /* Uploads everything, builds the work lists and captures the graph.  With
  * autotune != 0 it first times 64, 128, 256 and 512 sites per work item with
  * one rate category per wave, then one wave walking every category at the
- * best size and twice it, then up to three fewer resident workgroups per CU,
- * and keeps the fastest (phylo_batch_tiling). */
+ * best size and twice it, then up to three fewer resident workgroups per CU
+ * (the full evaluations' launch), and keeps the fastest (phylo_batch_tiling). */
 int phylo_batch_finalize(phylo_batch *b, int autotune);
 
 /* Replays the graph.  totals: one lnL per problem; nni_lnl (nullable): every
