@@ -19,8 +19,8 @@ struct NniInst {
 struct NniItem {
     int inst, prog, block, pad;
 };
-// A group of kNniSumVars variants of one instance to be totalled into
-// out[out0 ..].
+// A group of up to kNniSumVars variants of one batch instance to be totalled
+// into out[out0 ..].
 struct NniSum {
     int inst, var0, out0, pad;
 };

@@ -274,14 +274,19 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
 }
 
 // total = sum over site blocks of log(mantissa product) + exponent ln 2 (or
-// of the weighted sums): 32 slices of a variant's blocks, kNniSumVars variants
-// side by side so that a slice's loads are one 128-byte run; Kahan within a
-// slice, then two-sums over the slices in order.
+// of the weighted sums): 256 / W slices of a variant's blocks, W variants side by
+// side; Kahan within a slice, then two-sums over the slices in a fixed order.
+// Bound by a slice's chain of loads and logarithms where there are few
+// workgroups (250 variants x 1564 blocks: W = 8 30 us, 4 17, 2 10.9; 74 x 640:
+// 6.8, 5.0, 3.8), by the width of its loads (16 W bytes) where there are many
+// (5200 variants of 24 alignments: 8.4, 9.1, 11.1).
+template <int W>
 __global__ __launch_bounds__(256) void nni_sum_kernel(const double2* __restrict__ part, int weighted,
                                                       const NniInst* __restrict__ insts, NniInst one,
                                                       const NniSum* __restrict__ sums, double* __restrict__ out) {
-    constexpr int W = kNniSumVars, SL = 256 / W;
-    __shared__ double hi[SL][W], lo[SL][W];
+    constexpr int SL = 256 / W;
+    static_assert(64 % W == 0, "a wave holds whole slices");
+    __shared__ double hi[4][W], lo[4][W];
     NniSum g{0, (int)blockIdx.x * W, (int)blockIdx.x * W, 0};
     NniInst I = one;
     if (sums) {
@@ -309,12 +314,16 @@ __global__ __launch_bounds__(256) void nni_sum_kernel(const double2* __restrict_
             }
         }
     }
-    hi[sl][w] = s;
-    lo[sl][w] = -comp;
+    double h = s, l = -comp;
+#pragma unroll
+    for (int o = W; o < 64; o <<= 1) two_sum_add(h, l, __shfl_xor(h, o, 64), __shfl_xor(l, o, 64));
+    if ((threadIdx.x & 63) < W) {
+        hi[threadIdx.x >> 6][w] = h;
+        lo[threadIdx.x >> 6][w] = l;
+    }
     __syncthreads();
-    if (sl == 0 && var < I.n_var) {
-        double h = hi[0][w], l = lo[0][w];
-        for (int q = 1; q < SL; ++q) two_sum_add(h, l, hi[q][w], lo[q][w]);
+    if (threadIdx.x < W && var < I.n_var) {
+        for (int q = 1; q < 4; ++q) two_sum_add(h, l, hi[q][w], lo[q][w]);
         out[g.out0 + w] = h + l;
     }
 }
@@ -355,6 +364,12 @@ hipError_t nni4_launch(const NniArgs& a, hipStream_t st) {
 
 hipError_t nni_sum_launch(const double2* part, bool weighted, const NniInst* insts, const NniInst& one,
                           const NniSum* sums, int n_sums, double* out, hipStream_t st) {
-    hipLaunchKernelGGL(nni_sum_kernel, dim3(n_sums), dim3(256), 0, st, part, weighted ? 1 : 0, insts, one, sums, out);
+    const auto launch = [&](auto* kernel, int n) {
+        hipLaunchKernelGGL(kernel, dim3(n), dim3(256), 0, st, part, weighted ? 1 : 0, insts, one, sums, out);
+    };
+    // one neighbourhood: narrow groups until they alone fill the chip
+    if (sums) launch(nni_sum_kernel<kNniSumVars>, n_sums);
+    else if (one.n_var <= 1024) launch(nni_sum_kernel<2>, (one.n_var + 1) / 2);
+    else launch(nni_sum_kernel<kNniSumVars>, (one.n_var + kNniSumVars - 1) / kNniSumVars);
     return hipGetLastError();
 }

@@ -2091,8 +2091,8 @@ static int score_walks(phylo_ctx* c, int mode, int max_variants, double base, do
     if (mfma) HIPCHK(c, nni_mfma_launch(a, c->S, static_cast<const uint32_t*>(c->d_tips), c->d_Pm, c->d_PmT, c->d_PTm, c->stream));
     else HIPCHK(c, nni4_launch(a, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr,
-                             (n_out + kNniSumVars - 1) / kNniSumVars, c->h_total_dev, c->stream));
+    HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr, 0, c->h_total_dev,
+                             c->stream));
     HIPCHK(c, finish(c));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));

@@ -45,7 +45,7 @@ def _check(oracle, wl, ctx, mode, eff=None, w=None, n_check=6, seed=0):
     (9, 65, 4, 1, 0, 1), (11, 64, 4, 8, 1, 0), (13, 1, 4, 2, 0, 1), (7, 257, 2, 4, 1, 1), (300, 130, 4, 4, 0, 1),
     (6, 17, 5, 1, 0, 1), (8, 16, 8, 2, 1, 0), (8, 15, 9, 4, 0, 1), (9, 33, 16, 4, 1, 1), (9, 63, 17, 1, 0, 0),
     (9, 1, 19, 8, 1, 1), (10, 48, 21, 2, 0, 1), (8, 49, 24, 4, 1, 1), (8, 31, 25, 1, 0, 1), (8, 80, 32, 4, 0, 1),
-    (140, 20, 20, 4, 1, 1),
+    (140, 20, 20, 4, 1, 1), (530, 70, 4, 1, 1, 1),      # (more than 1024 variants)
 ])
 def test_walks_match_the_oracle_at_layout_edges(oracle, n, m, S, C, prec, mode):
     print(f"nni walks n={n} m={m} S={S} C={C} prec={prec} mode={mode}", flush=True)
