@@ -511,7 +511,7 @@ def main():
                    "n_taxa": n, "n_sites": m, "n_patterns": int(np.unique(wl.masks, axis=1).shape[1]),
                    "n_cat": C, "clv_storage": "f64" if args.fp64 else "f32", "arithmetic": "f64", "lnL": lnl},
         "end_to_end": {"ms_per_step": e2e_ms, "steps": e2e_steps,
-                       "what": "set_edge_lengths with new lengths (read from pinned host memory, "
+                       "what": "set_edge_lengths with new lengths (kernel arguments, "
                                "P rebuilt on the device) + loglik, alternating two length sets"},
         # What binds the DNA walker is FP64 arithmetic issue, not HBM: it keeps
         # all but a few partials in registers and LDS, so it moves a tenth of

@@ -609,19 +609,28 @@ __global__ void pbuild_eigen_kernel(const double* __restrict__ V, const double* 
 }
 
 // The same for a context of at most 4 states (Sp = 4), with nothing copied to
-// the device beforehand: the eigen system, rates and weights are arguments,
-// the lengths are read from the host's pinned memory (one 8-byte read a wave).
-// Bound by the round trip to host memory and the launch: 4.5 us at 32 and at
-// 128 taxa.  A copy in front of it cost 10 us of host time and a 3 us copy
-// kernel; a fit that changes the model each evaluation took two (59 us an
-// evaluation of 32 taxa x 2000 sites then, 37 us without).  A new topology's
-// programs (prog_words 16-byte words of pinned memory) come along.
+// the device beforehand: the eigen system, rates and weights are arguments, and
+// so are the lengths of up to kArgLengths nodes (arguments end at 4 KB); those of
+// larger trees are read from the host's pinned memory, one 8-byte read a wave.
+// Bound by the round trips to host memory, for the arguments and then for the
+// lengths, and the launch: 3.2 us with the lengths as arguments, 4.4 with them in
+// pinned memory, at 32 and at 128 taxa.  A copy in front of it cost 10 us of host
+// time and a 3 us copy kernel; a fit that changes the model each evaluation took
+// two (59 us an evaluation of 32 taxa x 2000 sites then, 34 us now).  A new
+// topology's programs (prog_words 16-byte words of pinned memory) come along.
 struct Eig4 {
     double rate[kMaxCat], V[16], Vinv[16], lam[4];
 };
-__global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const double* __restrict__ eff, int S, int C,
-                               int n_nodes, double* __restrict__ P, double* __restrict__ d_roots,
-                               const int4* __restrict__ prog, int4* __restrict__ d_prog, int prog_words) {
+template <int NL>
+struct Lengths {
+    double v[NL];
+};
+constexpr int kArgLengths = 384;
+template <int NL>
+__global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const Lengths<NL> len,
+                               const double* __restrict__ eff, int S, int C, int n_nodes, double* __restrict__ P,
+                               double* __restrict__ d_roots, const int4* __restrict__ prog, int4* __restrict__ d_prog,
+                               int prog_words) {
     const int gid = blockIdx.x * blockDim.x + threadIdx.x;
     for (int i = gid; i < prog_words; i += gridDim.x * blockDim.x) d_prog[i] = prog[i];
     if (gid < kRootDoubles) d_roots[gid] = roots.v[gid];
@@ -629,7 +638,7 @@ __global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const doub
     const int j = gid % 4, i = gid / 4 % 4, c = gid / 16 % C, node = gid / (16 * C);
     double v = 0.0;
     if (i < S && j < S) {
-        const double t = eff[node] * e.rate[c];
+        const double t = (NL > 1 ? len.v[node] : eff[node]) * e.rate[c];
         for (int k = 0; k < S; ++k) v = fma(e.V[i * S + k] * exp(e.lam[k] * t), e.Vinv[k * S + j], v);
     }
     P[gid] = v;
@@ -1308,9 +1317,12 @@ int upload_pmatrices(phylo_ctx* c) {
     HIPCHK(c, ensure(c->d_P, c->P_bytes, nP * sizeof(double)));
     if (!c->d_roots) HIPCHK(c, hipMalloc(&c->d_roots, kRootDoubles * sizeof(double)));
     const bool eigen = c->builder == PHYLO_P_EIGEN;
+    const bool arg_lengths = Sp == 4 && c->n_nodes <= kArgLengths;
     if (eigen) {
-        HIPCHK(c, stage_acquire(c, c->stage_len, c->eff.size()));
-        std::copy(c->eff.begin(), c->eff.end(), c->stage_len.h);
+        if (!arg_lengths) {
+            HIPCHK(c, stage_acquire(c, c->stage_len, c->eff.size()));
+            std::copy(c->eff.begin(), c->eff.end(), c->stage_len.h);
+        }
         if (Sp > 4 && c->dirty_eig) {     // every workgroup reads all of it: a copy, once a model
             const size_t n_eig = 2 * c->V.size() + c->lam.size();
             HIPCHK(c, ensure(c->d_eig, c->eig_bytes, n_eig * sizeof(double)));
@@ -1350,10 +1362,15 @@ int upload_pmatrices(phylo_ctx* c) {
         std::copy(c->V.begin(), c->V.end(), e.V);
         std::copy(c->Vinv.begin(), c->Vinv.end(), e.Vinv);
         std::copy(c->lam.begin(), c->lam.end(), e.lam);
-        hipLaunchKernelGGL(pbuild4_kernel, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0, c->stream, e, root_weights(c),
-                           c->stage_len.dev, S, c->C, c->n_nodes, c->d_P, c->d_roots,
-                           reinterpret_cast<const int4*>(c->stage_prog.dev), reinterpret_cast<int4*>(c->d_ops),
-                           (int)(c->prog_bytes / 16));
+        const auto launch = [&](auto len) {
+            if (sizeof len > sizeof(double)) std::copy(c->eff.begin(), c->eff.end(), len.v);
+            hipLaunchKernelGGL(pbuild4_kernel<sizeof len / sizeof(double)>, dim3((unsigned)((nP + 255) / 256)), dim3(256), 0,
+                               c->stream, e, root_weights(c), len, c->stage_len.dev, S, c->C, c->n_nodes, c->d_P, c->d_roots,
+                               reinterpret_cast<const int4*>(c->stage_prog.dev), reinterpret_cast<int4*>(c->d_ops),
+                               (int)(c->prog_bytes / 16));
+        };
+        if (arg_lengths) launch(Lengths<kArgLengths>{});
+        else launch(Lengths<1>{});
         HIPCHK(c, hipGetLastError());
         c->prog_bytes = 0;
         c->dirty_roots = false;

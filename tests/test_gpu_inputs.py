@@ -27,8 +27,18 @@ def _fresh(wl, prec, builder):
     (5, 8, 1, P.P_EIGEN), (20, 4, 0, P.P_EIGEN), (32, 1, 1, P.P_EIGEN), (20, 2, 0, P.P_PADE),
 ])
 def test_changed_inputs_match_a_fresh_context(S, C, prec, builder):
-    print(f"inputs S={S} C={C} prec={prec} builder={builder}", flush=True)
-    a, b = _wl(9, 130, S, C, 50 + S), _wl(9, 130, S, C, 70 + S)
+    _changed_inputs(9, S, C, prec, builder)
+
+
+@pytest.mark.parametrize("n", [192, 193])
+def test_lengths_at_the_limit_of_the_arguments(n):
+    """383 nodes' lengths are kernel arguments, 385 nodes' are in pinned memory."""
+    _changed_inputs(n, 4, 2, 1, P.P_EIGEN)
+
+
+def _changed_inputs(n, S, C, prec, builder):
+    print(f"inputs n={n} S={S} C={C} prec={prec} builder={builder}", flush=True)
+    a, b = _wl(n, 130, S, C, 50 + S), _wl(n, 130, S, C, 70 + S)
     b.tree, b.masks = a.tree, a.masks
     want = [_fresh(x, prec, builder) for x in (a, b)]
     n = a.tree.n_nodes
