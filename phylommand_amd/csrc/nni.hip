@@ -174,8 +174,9 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
         }
     };
 
-    // An op's operands are fetched during the op before it (ops[k1] is always
-    // readable: the next program's first op or the pad at the end).
+    // An op's operands are fetched during the op before it; after a program's
+    // last op those of the next program, but in a batch none: it may be
+    // another tree's.
     double O[4] = {}, B[4] = {};
     int sO = 0, sB = 0;
     const int k0 = prog_begin[prog], k1 = prog_begin[prog + 1];
@@ -186,7 +187,7 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
     fetch(nx.y, ry, rsy);
     for (int k = k0; k < k1; ++k) {
         const NniOp op = nx;
-        nx = ops[k + 1];
+        nx = BATCH ? nni_ahead(ops, k, k1) : ops[k + 1];
         double X[4], Y[4];
         factor(op.x, rx, X);
         factor(op.y, ry, Y);

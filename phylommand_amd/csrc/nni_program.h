@@ -45,6 +45,16 @@ struct alignas(16) NniOp {
 constexpr int nni_pop_slot(int flags) { return flags >> 8 & 15; }
 constexpr int nni_save_slot(int flags) { return flags >> 12 & 15; }
 
+// The op after ops[k] of a program that ends at k1, for a walk that fetches its
+// operands x and y ahead.  Past the end it names none: in a batch the op there
+// begins another tree's walk, whose nodes this tree's offsets do not reach.
+// (ops[k1] is always readable: the next program's first op or a last pad.)
+constexpr NniOp nni_ahead(const NniOp* ops, int k, int k1) {
+    NniOp o = ops[k + 1];
+    if (k + 1 >= k1) o.x = o.y = -1;
+    return o;
+}
+
 // Save slots a walk may hold (LDS; an edge whose upper node is no longer held
 // is reached again from its nearest held ancestor).  One slot leaves a DNA
 // workgroup of 128 taxa 27 KB of LDS, five a CU; two left four a CU and ran
