@@ -276,7 +276,8 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
 
 // total = sum over site blocks of log(mantissa product) + exponent ln 2 (or
 // of the weighted sums): 256 / W slices of a variant's blocks, W variants side by
-// side; Kahan within a slice, then two-sums over the slices in a fixed order.
+// side; Kahan within a slice, then two-sums over the slices in a fixed order
+// (infinite values as in block_total).
 // Bound by a slice's chain of loads and logarithms where there are few
 // workgroups (250 variants x 1564 blocks: W = 8 30 us, 4 17, 2 10.9; 74 x 640:
 // 6.8, 5.0, 3.8), by the width of its loads (16 W bytes) where there are many
@@ -295,29 +296,38 @@ __global__ __launch_bounds__(256) void nni_sum_kernel(const double2* __restrict_
         I = insts[g.inst];
     }
     const int w = threadIdx.x % W, sl = threadIdx.x / W, var = g.var0 + w;
+    const double2* p = part + I.part_off + var;
+    const int nblk = var < I.n_var ? I.nblk : 0;
+    const auto value = [&](double2 v) { return weighted ? v.x : log(v.x) + v.y * kLn2; };
     double s = 0.0, comp = 0.0;
-    if (var < I.n_var) {
-        const double2* p = part + I.part_off + var;
-        for (int b0 = sl; b0 < I.nblk; b0 += 4 * SL) {
-            double2 v[4];
+    for (int b0 = sl; b0 < nblk; b0 += 4 * SL) {
+        double2 v[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int b = b0 + u * SL;
-                v[u] = b < I.nblk ? p[(size_t)b * I.n_var] : make_double2(weighted ? 0.0 : 1.0, 0.0);
-            }
+        for (int u = 0; u < 4; ++u) {
+            const int b = b0 + u * SL;
+            v[u] = b < nblk ? p[(size_t)b * I.n_var] : make_double2(weighted ? 0.0 : 1.0, 0.0);
+        }
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double l = weighted ? v[u].x : log(v[u].x) + v[u].y * kLn2;
-                const double x = l - comp;
-                const double t = s + x;
-                comp = (t - s) - x;
-                s = t;
-            }
+        for (int u = 0; u < 4; ++u) {
+            const double x = value(v[u]) - comp;
+            const double t = s + x;
+            comp = (t - s) - x;
+            s = t;
         }
     }
     double h = s, l = -comp;
 #pragma unroll
     for (int o = W; o < 64; o <<= 1) two_sum_add(h, l, __shfl_xor(h, o, 64), __shfl_xor(l, o, 64));
+    if (__any(!(h + l == h + l))) {
+        double q = 0.0;
+        for (int b = sl; b < nblk; b += SL) q += value(p[(size_t)b * I.n_var]);
+#pragma unroll
+        for (int o = W; o < 64; o <<= 1) q += __shfl_xor(q, o, 64);
+        if (!(h + l == h + l)) {
+            h = q;
+            l = 0.0;
+        }
+    }
     if ((threadIdx.x & 63) < W) {
         hi[threadIdx.x >> 6][w] = h;
         lo[threadIdx.x >> 6][w] = l;
@@ -325,7 +335,8 @@ __global__ __launch_bounds__(256) void nni_sum_kernel(const double2* __restrict_
     __syncthreads();
     if (threadIdx.x < W && var < I.n_var) {
         for (int q = 1; q < 4; ++q) two_sum_add(h, l, hi[q][w], lo[q][w]);
-        out[g.out0 + w] = h + l;
+        const double t = h + l;
+        out[g.out0 + w] = t == t ? t : (hi[0][w] + hi[1][w]) + (hi[2][w] + hi[3][w]);
     }
 }
 

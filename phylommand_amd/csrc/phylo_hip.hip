@@ -1618,6 +1618,11 @@ int run_programs(phylo_ctx* c, const Op* d_ops, const int* d_prog, int n_prog, d
         HIPCHK(c, hipGetLastError());
     }
     HIPCHK(c, finish(c));
+    if (c->folded && std::isnan(c->h_total[0])) {     // an infinite site value, perhaps (fold_total)
+        hipLaunchKernelGGL(final_sum_kernel, dim3(1), dim3(kSumThreads), 0, c->stream, c->d_partial, nblk, c->h_total_dev);
+        HIPCHK(c, hipGetLastError());
+        HIPCHK(c, finish(c));
+    }
     if (site_lnl_host) std::memcpy(site_lnl_host, c->stage_site.h, (size_t)n_prog * c->m * sizeof(double));
     float ms = 0.f;
     HIPCHK(c, hipEventElapsedTime(&ms, c->ev0, c->ev1));

@@ -142,12 +142,17 @@ __device__ inline void two_sum_add(double& hi, double& lo, double b, double bl) 
 
 // Threads of the compensated sum: one workgroup per program.
 constexpr int kSumThreads = 256;
+static_assert(kSumThreads == 4 * 64, "block_total: four waves");
 
 // Compensated fixed-order sum of partial[0, n) by the first kSumThreads
 // threads of one workgroup.  Each thread issues its loads eight at a time before adding
 // them (Kahan), so their latencies overlap instead of queueing; the threads'
 // (sum, error) pairs then meet by two-sum, in a butterfly within each wave
 // and in LDS across the waves.  Thread 0 returns the total.
+// An infinite value (a site of likelihood zero) has no compensation: inf - inf
+// is no number.  With INF a wave that ends with none adds its values again
+// without, and so do the waves' sums.
+template <bool INF = true>
 __device__ inline double block_total(const double* partial, int n) {
     double s = 0.0, comp = 0.0;
     for (int base = threadIdx.x < kSumThreads ? (int)threadIdx.x : n; base < n; base += 8 * kSumThreads) {
@@ -170,6 +175,11 @@ __device__ inline double block_total(const double* partial, int n) {
     double hi = s, lo = -comp;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) two_sum_add(hi, lo, __shfl_xor(hi, o, 64), __shfl_xor(lo, o, 64));
+    if (INF && !(hi + lo == hi + lo)) {      // (the same in every lane)
+        hi = lo = 0.0;
+        for (int i = threadIdx.x; i < n; i += kSumThreads) hi += partial[i];
+        hi = wave_sum(hi);
+    }
     __shared__ double red_hi[kSumThreads / 64], red_lo[kSumThreads / 64];
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (lane == 0 && wid < kSumThreads / 64) { red_hi[wid] = hi; red_lo[wid] = lo; }
@@ -178,7 +188,8 @@ __device__ inline double block_total(const double* partial, int n) {
     lo = red_lo[0];
 #pragma unroll
     for (int w = 1; w < kSumThreads / 64; ++w) two_sum_add(hi, lo, red_hi[w], red_lo[w]);
-    return hi + lo;
+    const double t = hi + lo;
+    return !INF || t == t ? t : (red_hi[0] + red_hi[1]) + (red_hi[2] + red_hi[3]);
 }
 
 // Sums v over the workgroup (any multiple of 64 threads); thread 0 stores it.
@@ -202,6 +213,8 @@ __device__ inline void block_sum_store(double v, double* dst) {
 // writes it to the host-mapped total and returns the counter to zero.  The
 // fences publish the few partials this launch wrote and drop stale copies
 // before the sum reads them.  Workgroups of kSumThreads threads or more only.
+// (Without block_total's second pass over infinite values: the host sums again
+// where the total is no number, and the walkers stay as they are.)
 __device__ inline void fold_total(const double* partial, int n_part, unsigned* counter, double* total) {
     __shared__ int last;
     if (threadIdx.x == 0) {
@@ -211,7 +224,7 @@ __device__ inline void fold_total(const double* partial, int n_part, unsigned* c
     }
     __syncthreads();
     if (last) {
-        const double t = block_total(partial, n_part);
+        const double t = block_total<false>(partial, n_part);
         if (threadIdx.x == 0) {
             *total = t;
             *counter = 0u;
