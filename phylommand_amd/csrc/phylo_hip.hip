@@ -1150,15 +1150,18 @@ bool build_split_programs(phylo_ctx* c, int max_chunks, bool split_all) {
     if (best_L < 0) return false;
     // One workgroup a block for all pieces, or one a chunk: the first saves a
     // launch and the global round trips, the second spreads the chain over idle
-    // CUs.  us an evaluation, two launches / one, 4 categories, FP32, 2000
-    // sites (32 blocks): 20 taxa 25 / 23, 50 taxa 29 / 28, 120 taxa (chains of
-    // about 28 and 38 ops) 33 / 38, 250 taxa 42 / 56; 9000 sites (144 blocks,
-    // which leave the chunks few idle CUs): 29 / 25, 35 / 30, 44 / 40, 63 / 58;
-    // 16,384 (256 blocks): 32 / 27, 41 / 33, 55 / 42, 79 / 60.  One category
-    // (16 groups, and the total folded in): 28 / 21, 32 / 24, 38 / 26, 48 / 33
-    // at 2000 sites.  Past a block a CU it loses (50 taxa, 1 category, 768
-    // blocks: 38 / 48).
-    bool fused = G > 0 && (best_fused <= best_cost + 3.0 || 2 * nblk >= c->n_cu);
+    // CUs.  us an evaluation, two launches / one, FP32.  4 categories, 2000
+    // sites (32 blocks): 17 taxa 33 / 30, 50 taxa 36 / 36, 120 taxa (chains of
+    // 28 and 37 ops) 43 / 46, 250 taxa 54 / 65; 8200 sites (132 blocks, which
+    // leave the chunks few idle CUs): 36 / 31, 41 / 37, 53 / 47, 69 / 67;
+    // 16,384 (256 blocks): 39 / 34, 45 / 39, 61 / 49, 80 / 71.  One category
+    // (16 groups, and the total folded in), 2000 sites: 36 / 28, 39 / 31,
+    // 47 / 36, 58 / 44.  8 categories have two groups, so that one workgroup's
+    // chain may be twice the chunks': 8200 sites, chains of 16 and 28 ops 48 / 43, 23 and 46 54 / 53, 31 and 65 61 / 63, 46 and 94
+    // 73 / 80, 59 and 128 (250 taxa) 87 / 101; from 160 blocks on the chunks are
+    // longer, 98 and 142 109 / 106, 256 blocks 120 / 107.  Past a block a CU one
+    // workgroup loses (50 taxa, 1 category, 768 blocks: 38 / 48).
+    bool fused = G > 0 && (best_fused <= best_cost + 3.0 || (2 * nblk >= c->n_cu && best_fused <= 2.0 * best_cost));
     // with free_slots (prune4_pieces_kernel): lean, stores to LDS slots
     std::vector<int> lds_slot(fused ? nn : 0, -1);
     const auto emit = [&](const int* nodes, int n, bool store_all, std::vector<int>* free_slots = nullptr) {
