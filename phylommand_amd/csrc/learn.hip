@@ -284,31 +284,31 @@ __device__ __forceinline__ void tile_products(TileLds& t, const float* __restric
                                               float (&acc)[2][2]) {
     constexpr int NA = kTileM * kTileK / kTileThreads, NB = kTileN * kTileK / kTileThreads;
     const int tid = threadIdx.x;
-    // staging: A by k runs of 64 (K_MINOR) or rows of 16, B by rows of 32.  A
-    // load is a uniform base and the thread's own 32-bit offset, so that a
-    // piece's 24 addresses cost the vector unit nothing.
-    const int ak = K_MINOR ? tid & 63 : tid >> 4, ar = K_MINOR ? tid >> 6 : tid & 15;
+    // staging: A by k runs of 64 (K_MINOR: a wave's rows are its own, so their
+    // addresses are uniform) or rows of 16, B by rows of 32.  A load is a uniform
+    // base and the thread's own offset, so that a piece's 24 addresses cost the
+    // vector unit one instruction each.  Rows are reached in 64 bits: those of a
+    // minibatch may lie anywhere in the training set.
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int ak = K_MINOR ? tid & 63 : tid >> 4, ar = K_MINOR ? wave : tid & 15;
     const int bk = tid >> 5, bc = min(col0 + (tid & 31), N - 1);
-    uint32_t aoff[K_MINOR ? NA : 1];
+    const float* arow[K_MINOR ? NA : 1];
     if constexpr (K_MINOR) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int r = min(row0 + ar + 2 * i, M - 1);
-            aoff[i] = (uint32_t)(rows ? rows[r] - rows[0] : r) * (uint32_t)lda + (uint32_t)ak;
+            const int r = min(row0 + wave + 2 * i, M - 1);
+            arow[i] = A + (size_t)(rows ? rows[r] : r) * lda;
         }
-    } else {
-        aoff[0] = (uint32_t)ak * (uint32_t)lda + (uint32_t)min(row0 + ar, M - 1);
     }
-    const float* a0 = K_MINOR && rows ? A + (size_t)rows[0] * lda : A;
-    const uint32_t boff = (uint32_t)bk * (uint32_t)ldb + (uint32_t)bc;
+    const size_t aoff = (size_t)ak * lda + min(row0 + ar, M - 1), boff = (size_t)bk * ldb + bc;
     float ra[2][NA], rb[2][NB];
     const auto load = [&](int k0, int h) {
         if (k0 + kTileK <= K) {
 #pragma unroll
             for (int i = 0; i < NA; ++i) {
-                if constexpr (K_MINOR) ra[h][i] = (a0 + k0)[(int)aoff[i]];
+                if constexpr (K_MINOR) ra[h][i] = (arow[i] + k0)[ak];
                 else if (rows) ra[h][i] = A[(size_t)rows[k0 + ak + 8 * i] * lda + min(row0 + ar, M - 1)];
-                else ra[h][i] = (A + (size_t)(k0 + 8 * i) * lda)[aoff[0]];
+                else ra[h][i] = (A + (size_t)(k0 + 8 * i) * lda)[aoff];
             }
 #pragma unroll
             for (int i = 0; i < NB; ++i) rb[h][i] = (B + (size_t)(k0 + 4 * i) * ldb)[boff];
@@ -316,7 +316,7 @@ __device__ __forceinline__ void tile_products(TileLds& t, const float* __restric
 #pragma unroll
             for (int i = 0; i < NA; ++i) {
                 if constexpr (K_MINOR) {
-                    ra[h][i] = (a0 + (min(k0 + ak, K - 1) - ak))[(int)aoff[i]];
+                    ra[h][i] = arow[i][min(k0 + ak, K - 1)];
                 } else {
                     const int k = min(k0 + ak + 8 * i, K - 1);
                     ra[h][i] = A[(size_t)(rows ? rows[k] : k) * lda + min(row0 + ar, M - 1)];
