@@ -267,10 +267,11 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
 
 constexpr int kTileM = 16, kTileN = 32, kTileK = 64, kTileThreads = 128;
 
-struct TileLds {
+struct alignas(16) TileLds {
     float a[kTileK][kTileM + 2];
     float b[kTileK][kTileN];
 };
+static_assert(alignof(TileLds) >= alignof(float2), "read two values at once");
 
 // The thread's four sums over k (ascending) of A(row, k) B(k, col) for rows
 // row0 + 2 p, + 1 and columns col0 + 2 q, + 1 (p = thread / 16, q = thread % 16).

@@ -56,7 +56,8 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
     __shared__ int xs[C > 1 ? EP : 1][C][64];        // (both variants of an edge have one scaler)
     __shared__ double2 sv[kNniSaves][C][2][64];
     __shared__ int svs[kNniSaves][C][64];
-    __shared__ T tipv[TL ? 64 : 1];      // the four 0/1 state values of each code
+    __shared__ __align__(16) T tipv[TL ? 64 : 1];      // the four 0/1 state values of each code
+    static_assert(__alignof__(tipv) >= 16, "read four values at once (load_raw4)");
     extern __shared__ __align__(16) uint8_t tl[];
     const int lane = threadIdx.x & 63;
     const int cat = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
