@@ -1157,10 +1157,11 @@ bool build_split_programs(phylo_ctx* c, int max_chunks, bool split_all) {
     // 16,384 (256 blocks): 39 / 34, 45 / 39, 61 / 49, 80 / 71.  One category
     // (16 groups, and the total folded in), 2000 sites: 36 / 28, 39 / 31,
     // 47 / 36, 58 / 44.  8 categories have two groups, so that one workgroup's
-    // chain may be twice the chunks': 8200 sites, chains of 16 and 28 ops 48 / 43, 23 and 46 54 / 53, 31 and 65 61 / 63, 46 and 94
-    // 73 / 80, 59 and 128 (250 taxa) 87 / 101; from 160 blocks on the chunks are
-    // longer, 98 and 142 109 / 106, 256 blocks 120 / 107.  Past a block a CU one
-    // workgroup loses (50 taxa, 1 category, 768 blocks: 38 / 48).
+    // chain may be twice the chunks': 8200 sites, chains of 16 and 28 ops
+    // 48 / 43, 23 and 46 54 / 53, 31 and 65 61 / 63, 46 and 94 73 / 80, 59 and
+    // 128 (250 taxa) 87 / 101; from 160 blocks on the chunks are longer, 98 and
+    // 142 109 / 106, 256 blocks 120 / 107.  Past a block a CU one workgroup
+    // loses (50 taxa, 1 category, 768 blocks: 38 / 48).
     bool fused = G > 0 && (best_fused <= best_cost + 3.0 || (2 * nblk >= c->n_cu && best_fused <= 2.0 * best_cost));
     // with free_slots (prune4_pieces_kernel): lean, stores to LDS slots
     std::vector<int> lds_slot(fused ? nn : 0, -1);
@@ -2068,8 +2069,8 @@ static int score_walks(phylo_ctx* c, int mode, int max_variants, double base, do
         w.mode = -1;
         std::vector<NniOp> ops;
         std::vector<int> begin{0};
-        build_nni(c, mode, nni_segment_edges((double)(c->n_nodes - c->n_taxa) * nblk, c->n_cu), w.node, w.side, w.which,
-                  w.path_ops, ops, begin);
+        build_nni(c, mode, nni_segment_edges((double)(c->n_nodes - c->n_taxa) * nblk, c->C, mfma, c->n_cu), w.node, w.side,
+                  w.which, w.path_ops, ops, begin);
         w.n_prog = (int)begin.size() - 1;
         if (w.n_prog > 0) {
             ops.push_back(NniOp{});     // the walks read the op after the one they run
@@ -2761,7 +2762,7 @@ int phylo_batch_finalize(phylo_batch* b, int autotune) {
         if (I.nni_mode >= 0) edge_blocks += (double)(I.n_nodes - I.n_taxa) * (I.m_pad / 64);
     hipDeviceProp_t prop;
     HIPCHK(b, hipGetDeviceProperties(&prop, b->device));
-    const int max_edges = nni_segment_edges(edge_blocks, prop.multiProcessorCount);
+    const int max_edges = nni_segment_edges(edge_blocks, b->C, false, prop.multiProcessorCount);
     std::vector<NniOp> walk_ops;
     std::vector<int> walk_begin{0};
     std::vector<NniInst> walk_inst;
