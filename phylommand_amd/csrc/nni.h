@@ -72,6 +72,8 @@ inline int nni_segment_edges(double edge_blocks, int C, bool wide, int n_cu) {
 hipError_t nni4_launch(const NniArgs& a, hipStream_t st);
 
 // Totals of the variants from those pairs, in a fixed order with
-// compensation.
+// compensation.  A batch's trees are totalled by the same launch: out[k] = sum
+// of tree_part[seg[k] .. seg[k + 1]), k < n_seg.
 hipError_t nni_sum_launch(const double2* part, bool weighted, const NniInst* insts, const NniInst& one,
-                          const NniSum* sums, int n_sums, double* out, hipStream_t st);
+                          const NniSum* sums, int n_sums, const double* tree_part, const int* seg, int n_seg, double* out,
+                          hipStream_t st);

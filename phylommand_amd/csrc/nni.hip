@@ -282,13 +282,22 @@ __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
 // Bound by a slice's chain of loads and logarithms where there are few
 // workgroups (250 variants x 1564 blocks: W = 8 30 us, 4 17, 2 10.9; 74 x 640:
 // 6.8, 5.0, 3.8), by the width of its loads (16 W bytes) where there are many
-// (5200 variants of 24 alignments: 8.4, 9.1, 11.1).
+// (5200 variants of 24 alignments: 8.4, 9.1, 11.1).  A batch's tree totals come
+// along (their own launch added 5 to 8 us to every run, most of it the gap).
 template <int W>
 __global__ __launch_bounds__(256) void nni_sum_kernel(const double2* __restrict__ part, int weighted,
                                                       const NniInst* __restrict__ insts, NniInst one,
-                                                      const NniSum* __restrict__ sums, double* __restrict__ out) {
+                                                      const NniSum* __restrict__ sums, int n_sums,
+                                                      const double* __restrict__ tree_part, const int* __restrict__ seg,
+                                                      double* __restrict__ out) {
     constexpr int SL = 256 / W;
     static_assert(64 % W == 0, "a wave holds whole slices");
+    if ((int)blockIdx.x >= n_sums) {      // a batch's trees, after the variants
+        const int k = (int)blockIdx.x - n_sums;
+        const double t = block_total(tree_part + seg[k], seg[k + 1] - seg[k]);
+        if (threadIdx.x == 0) out[k] = t;
+        return;
+    }
     __shared__ double hi[4][W], lo[4][W];
     NniSum g{0, (int)blockIdx.x * W, (int)blockIdx.x * W, 0};
     NniInst I = one;
@@ -376,12 +385,15 @@ hipError_t nni4_launch(const NniArgs& a, hipStream_t st) {
 }
 
 hipError_t nni_sum_launch(const double2* part, bool weighted, const NniInst* insts, const NniInst& one,
-                          const NniSum* sums, int n_sums, double* out, hipStream_t st) {
+                          const NniSum* sums, int n_sums, const double* tree_part, const int* seg, int n_seg, double* out,
+                          hipStream_t st) {
+    static_assert(kSumThreads == 256, "trees and variants by the same workgroups");
     const auto launch = [&](auto* kernel, int n) {
-        hipLaunchKernelGGL(kernel, dim3(n), dim3(256), 0, st, part, weighted ? 1 : 0, insts, one, sums, out);
+        hipLaunchKernelGGL(kernel, dim3(n + n_seg), dim3(256), 0, st, part, weighted ? 1 : 0, insts, one, sums, n, tree_part,
+                           seg, out);
     };
     // one neighbourhood: narrow groups until they alone fill the chip
-    if (sums) launch(nni_sum_kernel<kNniSumVars>, n_sums);
+    if (sums || n_seg) launch(nni_sum_kernel<kNniSumVars>, n_sums);
     else if (one.n_var <= 1024) launch(nni_sum_kernel<2>, (one.n_var + 1) / 2);
     else launch(nni_sum_kernel<kNniSumVars>, (one.n_var + kNniSumVars - 1) / kNniSumVars);
     return hipGetLastError();

@@ -569,17 +569,6 @@ __global__ __launch_bounds__(64 * CW) void batch4_kernel(const WorkItem* __restr
     }
 }
 
-// Segmented compensated sums: out[k] = sum partial[seg[k] .. seg[k+1]), one
-// workgroup a segment (one thread a segment took 20 us for 24 alignments, its
-// loads one after another).
-__global__ __launch_bounds__(kSumThreads) void segment_sum_kernel(const double* __restrict__ partial,
-                                                                 const int* __restrict__ seg,
-                                                                 double* __restrict__ out) {
-    const int k = blockIdx.x;
-    const double t = block_total(partial + seg[k], seg[k + 1] - seg[k]);
-    if (threadIdx.x == 0) out[k] = t;
-}
-
 // Compensated fixed-order sum of the per-workgroup partials of each program
 // (one workgroup per program, block_total).
 __global__ __launch_bounds__(kSumThreads) void final_sum_kernel(const double* __restrict__ partial, int n_part,
@@ -2117,7 +2106,7 @@ static int score_walks(phylo_ctx* c, int mode, int max_variants, double base, do
     if (mfma) HIPCHK(c, nni_mfma_launch(a, c->S, static_cast<const uint32_t*>(c->d_tips), c->d_Pm, c->d_PmT, c->d_PTm, c->stream));
     else HIPCHK(c, nni4_launch(a, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
-    HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr, 0, c->h_total_dev,
+    HIPCHK(c, nni_sum_launch(w.d_part, a.site_w != nullptr, nullptr, a.one, nullptr, 0, nullptr, nullptr, 0, c->h_total_dev,
                              c->stream));
     HIPCHK(c, finish(c));
     float ms = 0.f;
@@ -2639,14 +2628,9 @@ int upload_work_lists(phylo_batch* b) {
 int enqueue_batch_run(phylo_batch* b) {
     int rc = enqueue_batch_trees(b, b->blocks_per_item);
     if (rc) return rc;
-    if (b->n_sums) {
-        HIPCHK(b, nni4_launch(b->nni, b->stream));
-        HIPCHK(b, nni_sum_launch(b->d_nni_part, false, b->d_walk_inst, b->nni.one, b->d_sums, b->n_sums, b->d_out,
-                                 b->stream));
-    }
-    hipLaunchKernelGGL(segment_sum_kernel, dim3(b->n_seg1), dim3(kSumThreads), 0, b->stream, b->d_partial, b->d_seg1,
-                       b->d_out);
-    HIPCHK(b, hipGetLastError());
+    if (b->n_sums) HIPCHK(b, nni4_launch(b->nni, b->stream));
+    HIPCHK(b, nni_sum_launch(b->d_nni_part, false, b->d_walk_inst, b->nni.one, b->d_sums, b->n_sums, b->d_partial, b->d_seg1,
+                             b->n_seg1, b->d_out, b->stream));
     HIPCHK(b, hipMemcpyAsync(b->h_out, b->d_out, (size_t)(b->n_seg1 + b->n_scored) * sizeof(double),
                              hipMemcpyDeviceToHost, b->stream));
     return PHYLO_OK;
