@@ -667,16 +667,18 @@ float sum_loss(const float* part, unsigned n) {
     return (float)s;
 }
 
-// Grows a device buffer to n elements.
+// Grows a device buffer to n elements; the old one stays if there is no memory
+// for the new (the loss parts serve phylo_mlp_grad too).
 template <typename T>
 hipError_t grow(T*& d, size_t& have, size_t n) {
     if (n <= have) return hipSuccess;
+    T* bigger = nullptr;
+    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&bigger), n * sizeof(T));
+    if (e != hipSuccess) return e;
     if (d) (void)hipFree(d);
-    d = nullptr;
-    have = 0;
-    const hipError_t e = hipMalloc(reinterpret_cast<void**>(&d), n * sizeof(T));
-    if (e == hipSuccess) have = n;
-    return e;
+    d = bigger;
+    have = n;
+    return hipSuccess;
 }
 
 }  // namespace
@@ -868,6 +870,15 @@ int phylo_mlp_set_data(phylo_mlp* p, int n, const float* x, const float* t) {
     if (!p || n < 1 || !x || !t) return PHYLO_ERR_ARG;
     MCHK(p, hipSetDevice(p->device));
     p->n_data = 0;
+    // (a larger set needs no room beside the one it replaces)
+    const auto make_room = [](float*& d, size_t& have, size_t n) {
+        if (n <= have) return;
+        if (d) (void)hipFree(d);
+        d = nullptr;
+        have = 0;
+    };
+    make_room(p->d_data_x, p->data_x_cap, (size_t)n * p->n_in);
+    make_room(p->d_data_t, p->data_t_cap, (size_t)n * p->n_out);
     MCHK(p, grow(p->d_data_x, p->data_x_cap, (size_t)n * p->n_in));
     MCHK(p, grow(p->d_data_t, p->data_t_cap, (size_t)n * p->n_out));
     MCHK(p, hipMemcpy(p->d_data_x, x, (size_t)n * p->n_in * sizeof(float), hipMemcpyHostToDevice));
