@@ -849,7 +849,7 @@ hipError_t stage_acquire(phylo_ctx* c, phylo_ctx::Stage& st, size_t n) {
     }
     if (st.cap < n) {
         if (st.h && (e = hipHostFree(st.h)) != hipSuccess) return e;
-        st.h = nullptr;
+        st.h = st.dev = nullptr;
         st.cap = 0;
         if ((e = hipHostMalloc(reinterpret_cast<void**>(&st.h), n * sizeof(double), hipHostMallocMapped)) != hipSuccess ||
             (e = hipHostGetDevicePointer(reinterpret_cast<void**>(&st.dev), st.h, 0)) != hipSuccess)
@@ -866,6 +866,7 @@ hipError_t stage_acquire(phylo_ctx* c, phylo_ctx::Stage& st, size_t n) {
 // early, the matrix walker to have the descriptor at hand), then the programs'
 // bounds.
 hipError_t stage_programs(phylo_ctx* c) {
+    c->prog_bytes = 0;           // (programs of an older topology that were never copied)
     order_children(c->ops);
     const size_t n_op = c->ops.size(), op_bytes = (n_op + 1) * sizeof(Op);
     const size_t bytes = (op_bytes + c->prog_begin.size() * sizeof(int) + 15) / 16 * 16;

@@ -1,4 +1,4 @@
-// Every allocation of a few call sequences made to fail in turn, under a
+// Every allocation of a few call sequences, and every two, made to fail, under a
 // stand-in for the HIP runtime (hip_stand_in.h): the call that meets the failure
 // returns an error, and it and the calls after it launch nothing on memory that
 // is not there.  Prints "ok" or the sequence, the failure and what was launched.
@@ -11,25 +11,25 @@
 
 static int bad = 0, runs = 0;
 
-// runs body with no failure, then with each of its allocations failing
+// runs body with no failure, then with each of its allocations failing, and each
+// two of them
 static void sequence(const char* name, const std::function<void()>& body) {
-    for (long k = -1;; k = k < 0 ? 1 : k + 1) {
+    const auto run = [&](long a, long b) {
         stand_in::allocs = 0;
-        stand_in::fail_at = k;
+        stand_in::fail_at[0] = a;
+        stand_in::fail_at[1] = b;
         stand_in::faults.clear();
         body();
         ++runs;
-        for (const std::string& f : stand_in::faults) {
-            printf("%s, allocation %ld failing: %s\n", name, k, f.c_str());
-            ++bad;
-        }
-        if (!stand_in::live.empty()) {
-            printf("%s, allocation %ld failing: %zu buffers left\n", name, k, stand_in::live.size());
-            ++bad;
-            stand_in::live.clear();
-        }
-        if (k >= 0 && stand_in::allocs < k) return;      // no such allocation any more
-    }
+        if (!stand_in::live.empty()) stand_in::faults.push_back(std::to_string(stand_in::live.size()) + " buffers left");
+        stand_in::live.clear();
+        for (const std::string& f : stand_in::faults) printf("%s, allocations %ld, %ld failing: %s\n", name, a, b, f.c_str());
+        bad += (int)stand_in::faults.size();
+        return stand_in::allocs;
+    };
+    run(-1, -1);
+    for (long a = 1; run(a, -1) >= a; ++a)
+        for (long b = a + 1; run(a, b) >= b; ++b) {}
 }
 
 static void mlp() {
@@ -49,8 +49,74 @@ static void mlp() {
     phylo_mlp_destroy(p);
 }
 
+struct Tree {
+    int n = 0, root = -1;
+    std::vector<int32_t> left, right;
+    std::vector<double> len;
+    // a caterpillar (or, paired, a balanced tree) of n_taxa tips
+    Tree(int n_taxa, bool paired) : n(2 * n_taxa - 1), left(n, -1), right(n, -1), len(n, 0.1) {
+        std::vector<int> f;
+        for (int i = 0; i < n_taxa; ++i) f.push_back(i);
+        for (int v = n_taxa; v < n; ++v) {
+            left[v] = f[0];
+            right[v] = f[1];
+            f.erase(f.begin(), f.begin() + 2);
+            f.insert(paired ? f.end() : f.begin(), v);
+        }
+        root = f[0];
+    }
+};
+
+// one context through new trees, neighbourhoods, simulation and precisions, on
+// an alphabet of S states
+static void context(int S) {
+    const int n = 20, m = 300;
+    const std::vector<uint32_t> masks(n * m, 1);
+    std::vector<double> Q(S * S, 1.0 / (S - 1)), pi(S, 1.0 / S), site(m), lnl(200), P(8 * S * S), clv(m * 8 * S);
+    for (int i = 0; i < S; ++i) Q[i * S + i] = -1.0;
+    const double rates[4] = {0.2, 0.6, 1.1, 2.1}, w[4] = {0.25, 0.25, 0.25, 0.25};
+    std::vector<uint8_t> states(400 * 50);
+    phylo_ctx* c = nullptr;
+    if (phylo_create(0, &c) != PHYLO_OK) return;
+    double total;
+    int nv;
+    const Tree small(n, true), other(n, false);
+    phylo_set_tips(c, n, m, S, masks.data());
+    for (const Tree* t : {&small, &other, &small}) {
+        phylo_set_topology(c, t->n, t->root, t->left.data(), t->right.data());
+        phylo_set_edge_lengths(c, t->len.data());
+        phylo_set_model(c, S, Q.data(), pi.data(), pi.data(), PHYLO_P_EIGEN);
+        phylo_set_categories(c, 4, rates, w);
+        phylo_loglik(c, site.data(), &total);
+        phylo_set_edge_lengths(c, t->len.data());
+        phylo_simulate(c, 50, pi.data(), 1, states.data());
+        phylo_nni_score(c, 1, 200, lnl.data(), nullptr, nullptr, &nv, nullptr);
+        phylo_set_precision(c, t == &other ? PHYLO_PREC_FP32 : PHYLO_PREC_FP64);
+        phylo_loglik(c, nullptr, &total);
+        phylo_node_partials(c, n + 1, clv.data(), nullptr);
+        phylo_get_pmatrix(c, 1, P.data());
+    }
+    // more taxa, and more again: larger programs, first met by whatever failed
+    // above, the ones before perhaps never copied
+    const std::vector<uint32_t> more(100 * m, 2);
+    for (int taxa : {50, 100}) {
+        const Tree t(taxa, true);
+        phylo_set_tips(c, taxa, m, S, more.data());
+        phylo_set_topology(c, t.n, t.root, t.left.data(), t.right.data());
+        phylo_set_edge_lengths(c, t.len.data());
+        phylo_loglik(c, site.data(), &total);
+        if (taxa == 50) continue;
+        phylo_set_edge_lengths(c, t.len.data());
+        phylo_simulate(c, 50, pi.data(), 1, states.data());
+        phylo_loglik(c, site.data(), &total);
+    }
+    phylo_destroy(c);
+}
+
 int main() {
     sequence("mlp", mlp);
+    sequence("context, 4 states", [] { context(4); });
+    sequence("context, 20 states", [] { context(20); });
     if (stand_in::launches < 100 || runs < 20) {
         printf("too little ran: %ld launches, %d runs\n", stand_in::launches, runs);
         return 1;

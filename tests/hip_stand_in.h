@@ -1,6 +1,6 @@
 // A stand-in for the HIP runtime on the CPU: device memory is host memory, no
 // kernel runs.  Linked into a test program ahead of the library, it takes the
-// library's calls; the n-th allocation can be made to fail, and every launch and
+// library's calls; one or two allocations can be made to fail, and every launch and
 // copy is checked: a pointer a kernel gets must be null or lie in memory that
 // is allocated at that time, and what a launch's other arguments need must be
 // there.  Host C++ only.
@@ -24,11 +24,12 @@ inline std::map<const void*, std::string>& kernels() {     // demangled, by host
     return k;
 }
 inline std::vector<std::string> faults;
-inline long allocs = 0, fail_at = -1, launches = 0;        // the allocation that fails (1 = next)
+inline long allocs = 0, launches = 0, fail_at[2] = {-1, -1};     // the allocations that fail (from 1)
 
 inline hipError_t get(void** p, size_t n) {
     *p = nullptr;
-    if (++allocs == fail_at) return hipErrorOutOfMemory;
+    ++allocs;
+    if (allocs == fail_at[0] || allocs == fail_at[1]) return hipErrorOutOfMemory;
     *p = calloc(n ? n : 1, 1);
     live[(char*)*p] = n;
     return *p ? hipSuccess : hipErrorOutOfMemory;
@@ -87,9 +88,9 @@ inline void launch(const void* fn, void** args) {
     const auto is = [&](const char* k) { return name.find(k) != std::string::npos; };
     // what may be null in some launches and not in others
     if (is("::output_kernel(") && ptr(6) && !(ptr(9) && ptr(10))) faults.push_back(name + ": targets without dY or loss");
-    if (is("::pbuild4_kernel<") && num(10) > 0) {
-        need(ptr(8), 16 * (size_t)num(10), name + ": programs are not staged");
-        need(ptr(9), 16 * (size_t)num(10), name + ": programs do not fit");
+    if (is("::pbuild4_kernel<") && num(11) > 0) {
+        need(ptr(9), 16 * (size_t)num(11), name + ": programs are not staged");
+        need(ptr(10), 16 * (size_t)num(11), name + ": programs do not fit");
     }
 }
 
