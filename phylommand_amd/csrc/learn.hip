@@ -11,6 +11,7 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <new>
 #include <random>
 #include <string>
 #include <vector>
@@ -713,7 +714,8 @@ int phylo_sim_features(int device, int n_align, int n_taxa, int n_sites, int n_c
     const size_t o_cat = take(N * n_cat * sizeof(double)), in_bytes = off;
     const size_t o_feat = take(N * kFeat * sizeof(float));
     const size_t o_mask = take(masks ? N * n_taxa * n_sites * sizeof(uint32_t) : 0);
-    const std::unique_ptr<unsigned char[]> in(new unsigned char[in_bytes]);
+    const std::unique_ptr<unsigned char[]> in(new (std::nothrow) unsigned char[in_bytes]);
+    if (!in) return PHYLO_ERR_HIP;
     int* walk = reinterpret_cast<int*>(in.get() + o_walk);
     for (int k = 0; k < n_align; ++k) {
         const int32_t* L = left + (size_t)k * nn;

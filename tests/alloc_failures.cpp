@@ -4,12 +4,28 @@
 // is not there.  Prints "ok" or the sequence, the failure and what was launched.
 #include "hip_stand_in.h"
 
+#include <cstdint>
 #include <functional>
+#include <new>
 
 #include "../include/phylo_hip.h"
 #include "../include/phylo_learn.h"
 
 static int bad = 0, runs = 0;
+
+// host allocations above the limit fail
+static size_t host_limit = SIZE_MAX;
+void* operator new(size_t n, const std::nothrow_t&) noexcept { return n > host_limit ? nullptr : malloc(n); }
+void* operator new[](size_t n, const std::nothrow_t&) noexcept { return n > host_limit ? nullptr : malloc(n); }
+void* operator new(size_t n) {
+    if (void* p = operator new(n, std::nothrow)) return p;
+    throw std::bad_alloc();
+}
+void* operator new[](size_t n) { return operator new(n); }
+void operator delete(void* p) noexcept { free(p); }
+void operator delete[](void* p) noexcept { free(p); }
+void operator delete(void* p, size_t) noexcept { free(p); }
+void operator delete[](void* p, size_t) noexcept { free(p); }
 
 // runs body with no failure, then with each of its allocations failing, and each
 // two of them
@@ -113,10 +129,56 @@ static void context(int S) {
     phylo_destroy(c);
 }
 
+static void batch() {
+    const int m = 300;
+    const std::vector<uint32_t> masks(60 * m, 1);
+    std::vector<double> Q(16, 1.0 / 3), w(4, 0.25), tot(3), lnl(400);
+    for (int i = 0; i < 4; ++i) Q[5 * i] = -1.0;
+    phylo_batch* b = nullptr;
+    if (phylo_batch_create(0, 4, PHYLO_PREC_FP32, &b) != PHYLO_OK) return;
+    for (int n : {8, 60, 5}) {
+        const Tree t(n, n == 60);
+        phylo_batch_add(b, n, m, 4, masks.data(), t.n, t.root, t.left.data(), t.right.data(), t.len.data(), Q.data(), w.data(),
+                        w.data(), w.data(), w.data(), n == 5 ? -1 : 1, nullptr);
+    }
+    if (phylo_batch_finalize(b, 1) == PHYLO_OK) phylo_batch_run(b, tot.data(), lnl.data());
+    phylo_batch_destroy(b);
+}
+
+static int features(int n_align, bool limited) {
+    const int n = 6;
+    const Tree t(n, true);
+    std::vector<int32_t> left, right, roots(n_align, t.root);
+    std::vector<double> len, eig(36 * n_align, 0.1), pi(4 * n_align, 0.25), rates(2 * n_align, 1.0);
+    for (int k = 0; k < n_align; ++k) {
+        left.insert(left.end(), t.left.begin(), t.left.end());
+        right.insert(right.end(), t.right.begin(), t.right.end());
+        len.insert(len.end(), t.len.begin(), t.len.end());
+    }
+    std::vector<float> out(256 * n_align);
+    std::vector<uint32_t> masks(n_align * n * 40);
+    if (limited) host_limit = (size_t)n_align * 256;      // (past the library's small vectors)
+    int rc = 1;
+    try {
+        rc = phylo_sim_features(0, n_align, n, 40, 2, left.data(), right.data(), roots.data(), len.data(), eig.data(), pi.data(),
+                                rates.data(), 0.0, 1, out.data(), masks.data());
+    } catch (const std::bad_alloc&) {
+        stand_in::faults.push_back("an exception left phylo_sim_features");
+    }
+    host_limit = SIZE_MAX;
+    return rc;
+}
+
 int main() {
     sequence("mlp", mlp);
     sequence("context, 4 states", [] { context(4); });
     sequence("context, 20 states", [] { context(20); });
+    sequence("batch", batch);
+    sequence("features", [] { features(64, false); });
+    // the copy of its inputs on the host fails
+    sequence("features, no host memory", [] {
+        if (features(64, true) == PHYLO_OK) stand_in::faults.push_back("no error from phylo_sim_features");
+    });
     if (stand_in::launches < 100 || runs < 20) {
         printf("too little ran: %ld launches, %d runs\n", stand_in::launches, runs);
         return 1;
