@@ -620,11 +620,11 @@ __global__ void pbuild4_kernel(const Eig4 e, const RootWeights roots, const Leng
                                const double* __restrict__ eff, int S, int C, int n_nodes, double* __restrict__ P,
                                double* __restrict__ d_roots, const int4* __restrict__ prog, int4* __restrict__ d_prog,
                                int prog_words) {
-    const int gid = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int i = gid; i < prog_words; i += gridDim.x * blockDim.x) d_prog[i] = prog[i];
+    const unsigned gid = blockIdx.x * blockDim.x + threadIdx.x;      // (a launch has less than 2^32 threads)
+    for (unsigned i = gid; i < (unsigned)prog_words; i += gridDim.x * blockDim.x) d_prog[i] = prog[i];
     if (gid < kRootDoubles) d_roots[gid] = roots.v[gid];
-    if (gid >= n_nodes * C * 16) return;
-    const int j = gid % 4, i = gid / 4 % 4, c = gid / 16 % C, node = gid / (16 * C);
+    if (gid >= 16u * C * n_nodes) return;
+    const int j = gid % 4, i = gid / 4 % 4, c = gid / 16 % C, node = gid / (16u * C);
     double v = 0.0;
     if (i < S && j < S) {
         const double t = (NL > 1 ? len.v[node] : eff[node]) * e.rate[c];
