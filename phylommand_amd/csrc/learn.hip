@@ -264,41 +264,61 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
 // while the next two pieces are on their way into registers (what a launch reads
 // was written by the launch before, on other XCDs, so it comes from beyond L2).  (Rows by scalar loads
 // and columns from L1 waited in every 16-long piece: 18 us for 256 x 512 x 512.)
+// Wide layers and batches take 64 x 64 tiles, 4 x 4 a thread (large_tiles): the
+// same sums in the same order.
 // ---------------------------------------------------------------------------
 
-constexpr int kTileM = 16, kTileN = 32, kTileK = 64, kTileThreads = 128;
+constexpr int kTileK = 64;
 
-struct alignas(16) TileLds {
-    float a[kTileK][kTileM + 2];
-    float b[kTileK][kTileN];
+// R x R outputs a thread, 16 threads a tile row.
+template <int R_, int THREADS_>
+struct Tile {
+    static constexpr int R = R_, THREADS = THREADS_, M = THREADS_ / 16 * R_, N = 16 * R_;
+    static constexpr int U = R_ == 2 ? 16 : 4;       // k read ahead of their sums
+    struct alignas(16) Lds {
+        float a[kTileK][M + R_];
+        float b[kTileK][N];
+    };
+    static_assert(alignof(Lds) >= R_ * sizeof(float), "read R values at once");
 };
-static_assert(alignof(TileLds) >= alignof(float2), "read two values at once");
+typedef Tile<2, 128> Small;      // 16 x 32
+typedef Tile<4, 256> Large;      // 64 x 64
 
-// The thread's four sums over k (ascending) of A(row, k) B(k, col) for rows
-// row0 + 2 p, + 1 and columns col0 + 2 q, + 1 (p = thread / 16, q = thread % 16).
+__device__ __forceinline__ void read_values(const float* p, float (&v)[2]) {
+    const float2 x = *reinterpret_cast<const float2*>(p);
+    v[0] = x.x; v[1] = x.y;
+}
+__device__ __forceinline__ void read_values(const float* p, float (&v)[4]) {
+    const float4 x = *reinterpret_cast<const float4*>(p);
+    v[0] = x.x; v[1] = x.y; v[2] = x.z; v[3] = x.w;
+}
+
+// The thread's sums over k (ascending) of A(row, k) B(k, col) for rows
+// row0 + R p .. and columns col0 + R q .. (p = thread / 16, q = thread % 16).
 // A is row-major (K_MINOR: element (row, k) at A[row * lda + k], storage row
 // rows[row] where set) or its transpose (A[k * lda + row], storage row rows[k]).
 // B(k, col) is B[k * ldb + col].  Rows past M and columns past N repeat the last.
-template <bool K_MINOR>
-__device__ __forceinline__ void tile_products(TileLds& t, const float* __restrict__ A, int lda,
+template <class T, bool K_MINOR>
+__device__ __forceinline__ void tile_products(typename T::Lds& t, const float* __restrict__ A, int lda,
                                               const int* __restrict__ rows, int row0, int M, int K,
                                               const float* __restrict__ B, int ldb, int col0, int N,
-                                              float (&acc)[2][2]) {
-    constexpr int NA = kTileM * kTileK / kTileThreads, NB = kTileN * kTileK / kTileThreads;
+                                              float (&acc)[T::R][T::R]) {
+    constexpr int R = T::R, NA = T::M * kTileK / T::THREADS, NB = T::N * kTileK / T::THREADS;
+    constexpr int SA = K_MINOR ? T::THREADS / 64 : T::THREADS / T::M, SB = T::THREADS / T::N;   // rows a step
     const int tid = threadIdx.x;
     // staging: A by k runs of 64 (K_MINOR: a wave's rows are its own, so their
-    // addresses are uniform) or rows of 16, B by rows of 32.  A load is a uniform
-    // base and the thread's own offset, so that a piece's 24 addresses cost the
-    // vector unit one instruction each.  Rows are reached in 64 bits: those of a
-    // minibatch may lie anywhere in the training set.
+    // addresses are uniform) or rows of the tile, B by rows of the tile.  A load
+    // is a uniform base and the thread's own offset, so that a piece's addresses
+    // cost the vector unit one instruction each.  Rows are reached in 64 bits:
+    // those of a minibatch may lie anywhere in the training set.
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int ak = K_MINOR ? tid & 63 : tid >> 4, ar = K_MINOR ? wave : tid & 15;
-    const int bk = tid >> 5, bc = min(col0 + (tid & 31), N - 1);
+    const int ak = K_MINOR ? tid & 63 : tid / T::M, ar = K_MINOR ? wave : tid % T::M;
+    const int bk = tid / T::N, bc = min(col0 + tid % T::N, N - 1);
     const float* arow[K_MINOR ? NA : 1];
     if constexpr (K_MINOR) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int r = min(row0 + wave + 2 * i, M - 1);
+            const int r = min(row0 + wave + SA * i, M - 1);
             arow[i] = A + (size_t)(rows ? rows[r] : r) * lda;
         }
     }
@@ -309,57 +329,58 @@ __device__ __forceinline__ void tile_products(TileLds& t, const float* __restric
 #pragma unroll
             for (int i = 0; i < NA; ++i) {
                 if constexpr (K_MINOR) ra[h][i] = (arow[i] + k0)[ak];
-                else if (rows) ra[h][i] = A[(size_t)rows[k0 + ak + 8 * i] * lda + min(row0 + ar, M - 1)];
-                else ra[h][i] = (A + (size_t)(k0 + 8 * i) * lda)[aoff];
+                else if (rows) ra[h][i] = A[(size_t)rows[k0 + ak + SA * i] * lda + min(row0 + ar, M - 1)];
+                else ra[h][i] = (A + (size_t)(k0 + SA * i) * lda)[aoff];
             }
 #pragma unroll
-            for (int i = 0; i < NB; ++i) rb[h][i] = (B + (size_t)(k0 + 4 * i) * ldb)[boff];
+            for (int i = 0; i < NB; ++i) rb[h][i] = (B + (size_t)(k0 + SB * i) * ldb)[boff];
         } else {
 #pragma unroll
             for (int i = 0; i < NA; ++i) {
                 if constexpr (K_MINOR) {
                     ra[h][i] = arow[i][min(k0 + ak, K - 1)];
                 } else {
-                    const int k = min(k0 + ak + 8 * i, K - 1);
+                    const int k = min(k0 + ak + SA * i, K - 1);
                     ra[h][i] = A[(size_t)(rows ? rows[k] : k) * lda + min(row0 + ar, M - 1)];
                 }
             }
 #pragma unroll
-            for (int i = 0; i < NB; ++i) rb[h][i] = B[(size_t)min(k0 + bk + 4 * i, K - 1) * ldb + bc];
+            for (int i = 0; i < NB; ++i) rb[h][i] = B[(size_t)min(k0 + bk + SB * i, K - 1) * ldb + bc];
         }
     };
     const int p = tid >> 4, q = tid & 15;
-    acc[0][0] = acc[0][1] = acc[1][0] = acc[1][1] = 0.f;
+#pragma unroll
+    for (int i = 0; i < R; ++i)
+#pragma unroll
+        for (int j = 0; j < R; ++j) acc[i][j] = 0.f;
+    const auto add = [&](const float (&x)[R], const float (&y)[R]) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+#pragma unroll
+            for (int j = 0; j < R; ++j) acc[i][j] = fmaf(x[i], y[j], acc[i][j]);
+    };
     const auto piece = [&](int k0, int h) {
         if (k0) __syncthreads();
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            if constexpr (K_MINOR) t.a[ak][ar + 2 * i] = ra[h][i];
-            else t.a[ak + 8 * i][ar] = ra[h][i];
+            if constexpr (K_MINOR) t.a[ak][ar + SA * i] = ra[h][i];
+            else t.a[ak + SA * i][ar] = ra[h][i];
         }
 #pragma unroll
-        for (int i = 0; i < NB; ++i) t.b[bk + 4 * i][tid & 31] = rb[h][i];
+        for (int i = 0; i < NB; ++i) t.b[bk + SB * i][tid % T::N] = rb[h][i];
         __syncthreads();
         if (k0 + 2 * kTileK < K) load(k0 + 2 * kTileK, h);
         const int n = min(kTileK, K - k0);
-        const auto step = [&](int k) {
-            const float2 x = *reinterpret_cast<const float2*>(&t.a[k][2 * p]);
-            const float2 y = *reinterpret_cast<const float2*>(&t.b[k][2 * q]);
-            acc[0][0] = fmaf(x.x, y.x, acc[0][0]);
-            acc[0][1] = fmaf(x.x, y.y, acc[0][1]);
-            acc[1][0] = fmaf(x.y, y.x, acc[1][0]);
-            acc[1][1] = fmaf(x.y, y.y, acc[1][1]);
-        };
         if (n == kTileK) {
-            // 16 k read ahead of their sums (one wave a SIMD: each read waited
+            // U k read ahead of their sums (few waves a SIMD: each read waited
             // for by itself costs the LDS latency, 3.3 us a piece of 64)
-            constexpr int U = 16;
-            float2 x[2][U], y[2][U];
+            constexpr int U = T::U;
+            float x[2][U][R], y[2][U][R];
             const auto read = [&](int k, int h) {
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
-                    x[h][u] = *reinterpret_cast<const float2*>(&t.a[k + u][2 * p]);
-                    y[h][u] = *reinterpret_cast<const float2*>(&t.b[k + u][2 * q]);
+                    read_values(&t.a[k + u][R * p], x[h][u]);
+                    read_values(&t.b[k + u][R * q], y[h][u]);
                 }
             };
             read(0, 0);
@@ -369,16 +390,16 @@ __device__ __forceinline__ void tile_products(TileLds& t, const float* __restric
                 if (k + U < kTileK) read(k + U, 1 - h);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int u = 0; u < U; ++u) {
-                    acc[0][0] = fmaf(x[h][u].x, y[h][u].x, acc[0][0]);
-                    acc[0][1] = fmaf(x[h][u].x, y[h][u].y, acc[0][1]);
-                    acc[1][0] = fmaf(x[h][u].y, y[h][u].x, acc[1][0]);
-                    acc[1][1] = fmaf(x[h][u].y, y[h][u].y, acc[1][1]);
-                }
+                for (int u = 0; u < U; ++u) add(x[h][u], y[h][u]);
                 __builtin_amdgcn_sched_barrier(0);
             }
         } else {
-            for (int k = 0; k < n; ++k) step(k);
+            for (int k = 0; k < n; ++k) {
+                float x[R], y[R];
+                read_values(&t.a[k][R * p], x);
+                read_values(&t.b[k][R * q], y);
+                add(x, y);
+            }
         }
     };
     load(0, 0);
@@ -390,37 +411,39 @@ __device__ __forceinline__ void tile_products(TileLds& t, const float* __restric
 }
 
 // epi(row, col, value) for the thread's elements inside M x N
-template <class Epi>
-__device__ __forceinline__ void tile_out(const float (&acc)[2][2], int row0, int M, int col0, int N, Epi&& epi) {
+template <int R, class Epi>
+__device__ __forceinline__ void tile_out(const float (&acc)[R][R], int row0, int M, int col0, int N, Epi&& epi) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < R; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int r = row0 + 2 * (threadIdx.x >> 4) + i, c = col0 + 2 * (threadIdx.x & 15) + j;
+        for (int j = 0; j < R; ++j) {
+            const int r = row0 + R * (threadIdx.x >> 4) + i, c = col0 + R * (threadIdx.x & 15) + j;
             if (r < M && c < N) epi(r, c, acc[i][j]);
         }
 }
 
 // H = relu(X W + b), X's rows through `rows` where set.
-__global__ __launch_bounds__(kTileThreads) void layer_kernel(int M, int N, int K, const float* __restrict__ X,
+template <class T>
+__global__ __launch_bounds__(T::THREADS) void layer_kernel(int M, int N, int K, const float* __restrict__ X,
                                                              const int* __restrict__ rows, const float* __restrict__ W,
                                                              const float* __restrict__ b, float* __restrict__ H) {
-    __shared__ TileLds t;
-    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
-    float acc[2][2];
-    tile_products<true>(t, X, K, rows, row0, M, K, W, N, col0, N, acc);
+    __shared__ typename T::Lds t;
+    const int nx = (N + T::N - 1) / T::N, row0 = blockIdx.x / nx * T::M, col0 = blockIdx.x % nx * T::N;
+    float acc[T::R][T::R];
+    tile_products<T, true>(t, X, K, rows, row0, M, K, W, N, col0, N, acc);
     tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) { H[(size_t)r * N + c] = fmaxf(v + b[c], 0.f); });
 }
 
 // dZ = (dY W^T) x (H > 0), from the transposed weights WT: the gradient
 // through a layer and its input's ReLU.
-__global__ __launch_bounds__(kTileThreads) void back_kernel(int M, int N, int K, const float* __restrict__ dY,
+template <class T>
+__global__ __launch_bounds__(T::THREADS) void back_kernel(int M, int N, int K, const float* __restrict__ dY,
                                                             const float* __restrict__ WT, const float* __restrict__ H,
                                                             float* __restrict__ dZ) {
-    __shared__ TileLds t;
-    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
-    float acc[2][2];
-    tile_products<true>(t, dY, K, nullptr, row0, M, K, WT, N, col0, N, acc);
+    __shared__ typename T::Lds t;
+    const int nx = (N + T::N - 1) / T::N, row0 = blockIdx.x / nx * T::M, col0 = blockIdx.x % nx * T::N;
+    float acc[T::R][T::R];
+    tile_products<T, true>(t, dY, K, nullptr, row0, M, K, WT, N, col0, N, acc);
     tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) {
         const size_t i = (size_t)r * N + c;
         dZ[i] = H[i] > 0.f ? v : 0.f;
@@ -429,16 +452,16 @@ __global__ __launch_bounds__(kTileThreads) void back_kernel(int M, int N, int K,
 
 // The output layer: Y = H W + b; with targets also dY = 2 (Y - T) / (M N) and
 // the workgroup's share of the loss.
-__global__ __launch_bounds__(kTileThreads) void output_kernel(int M, int N, int K, const float* __restrict__ H,
+__global__ __launch_bounds__(Small::THREADS) void output_kernel(int M, int N, int K, const float* __restrict__ H,
                                                               const float* __restrict__ W, const float* __restrict__ b,
                                                               const float* __restrict__ T, const int* __restrict__ rows,
                                                               float* __restrict__ Y, float* __restrict__ dY,
                                                               float* __restrict__ loss_part) {
-    __shared__ TileLds t;
+    __shared__ Small::Lds t;
     __shared__ float wave_loss[2];
-    const int nx = (N + kTileN - 1) / kTileN, row0 = blockIdx.x / nx * kTileM, col0 = blockIdx.x % nx * kTileN;
+    const int nx = (N + Small::N - 1) / Small::N, row0 = blockIdx.x / nx * Small::M, col0 = blockIdx.x % nx * Small::N;
     float acc[2][2], loss = 0.f;
-    tile_products<true>(t, H, K, nullptr, row0, M, K, W, N, col0, N, acc);
+    tile_products<Small, true>(t, H, K, nullptr, row0, M, K, W, N, col0, N, acc);
     tile_out(acc, row0, M, col0, N, [&](int r, int c, float v) {
         const float y = v + b[c];
         Y[(size_t)r * N + c] = y;
@@ -509,27 +532,28 @@ __device__ __forceinline__ void put_gradient(const Adam& a, float* __restrict__ 
 
 // Every weight gradient A^T dZ and bias gradient (column sums of dZ) of the
 // step, and the Adam updates (and W2's transpose kept up with them).
-// Workgroups: the layers' tiles in turn, then kTileThreads bias columns each.
+// Workgroups: the layers' tiles in turn, then a thread a bias column.
 struct GradArgs {
     int n_in, n_hid, n_out, M;
     int tile[3], bias[3];              // first workgroup of each layer's tiles, of its biases
     size_t w_off[3], b_off[3];
 };
-__global__ __launch_bounds__(kTileThreads) void gradient_kernel(
+template <class T>
+__global__ __launch_bounds__(T::THREADS) void gradient_kernel(
     GradArgs a, const float* __restrict__ X, const int* __restrict__ rows, const float* __restrict__ H1,
     const float* __restrict__ H2, const float* __restrict__ dZ1, const float* __restrict__ dZ2,
     const float* __restrict__ dY, Adam adam, float* __restrict__ g, float* __restrict__ W2T) {
-    __shared__ TileLds t;
+    __shared__ typename T::Lds t;
     const int blk = blockIdx.x;
     if (blk < a.bias[0]) {
         const int l = blk >= a.tile[2] ? 2 : blk >= a.tile[1] ? 1 : 0;
         const float* A = l == 0 ? X : l == 1 ? H1 : H2;
         const float* D = l == 0 ? dZ1 : l == 1 ? dZ2 : dY;
         const int n_a = l == 0 ? a.n_in : a.n_hid, n_d = l == 2 ? a.n_out : a.n_hid;
-        const int nx = (n_d + kTileN - 1) / kTileN, tile = blk - a.tile[l];
-        const int row0 = tile / nx * kTileM, col0 = tile % nx * kTileN;
-        float acc[2][2];
-        tile_products<false>(t, A, n_a, l == 0 ? rows : nullptr, row0, n_a, a.M, D, n_d, col0, n_d, acc);
+        const int nx = (n_d + T::N - 1) / T::N, tile = blk - a.tile[l];
+        const int row0 = tile / nx * T::M, col0 = tile % nx * T::N;
+        float acc[T::R][T::R];
+        tile_products<T, false>(t, A, n_a, l == 0 ? rows : nullptr, row0, n_a, a.M, D, n_d, col0, n_d, acc);
         tile_out(acc, row0, n_a, col0, n_d, [&](int r, int c, float v) {
             const size_t i = a.w_off[l] + (size_t)r * n_d + c;
             put_gradient(adam, g, i, v);
@@ -539,7 +563,7 @@ __global__ __launch_bounds__(kTileThreads) void gradient_kernel(
     }
     const int l = blk >= a.bias[2] ? 2 : blk >= a.bias[1] ? 1 : 0;
     const float* D = l == 0 ? dZ1 : l == 1 ? dZ2 : dY;
-    const int n_d = l == 2 ? a.n_out : a.n_hid, j = (blk - a.bias[l]) * kTileThreads + threadIdx.x;
+    const int n_d = l == 2 ? a.n_out : a.n_hid, j = (blk - a.bias[l]) * T::THREADS + threadIdx.x;
     if (j >= n_d) return;
     float s = 0.f;
     int i = 0;
@@ -561,7 +585,7 @@ __global__ __launch_bounds__(kTileThreads) void gradient_kernel(
 // ---------------------------------------------------------------------------
 
 struct phylo_mlp {
-    int device = 0;
+    int device = 0, n_cu = 0;
     int n_in = 0, n_hid = 0, n_out = 0, max_batch = 0;
     long n_params = 0;
     hipStream_t stream = nullptr;
@@ -618,7 +642,17 @@ Views views(phylo_mlp* p, float* base) {
 unsigned tiles(int n, int t) { return (unsigned)((n + t - 1) / t); }
 
 // Workgroups of the output layer, each with a part of the loss.
-unsigned loss_parts(const phylo_mlp* p, int B) { return tiles(B, kTileM) * tiles(p->n_out, kTileN); }
+unsigned loss_parts(const phylo_mlp* p, int B) { return tiles(B, Small::M) * tiles(p->n_out, Small::N); }
+
+// Whether an M x N product takes the large tiles: from one a CU on.  They read A
+// half and B a quarter as often, which is what binds there; with fewer, CUs stand
+// idle.  Kernel us, small / large, of the second layer: batch 1024 x 512 hidden
+// (128 tiles) 24 / 32, 256 x 4096 (256) 318 / 231, 1024 x 1024 (256) 97 / 63,
+// 1024 x 4096 1200 / 589; of the gradients at batch 1024: 512 hidden (64) 66 / 134,
+// 1024 (256) 144 / 137, 4096 1830 / 978.
+bool large_tiles(const phylo_mlp* p, int M, int N) {
+    return (size_t)tiles(M, Large::M) * tiles(N, Large::N) >= (size_t)p->n_cu;
+}
 
 // One pass over B rows of X (through `rows` where set): the forward layers
 // and the output; with targets also the loss parts and the gradients of the
@@ -626,15 +660,21 @@ unsigned loss_parts(const phylo_mlp* p, int B) { return tiles(B, kTileM) * tiles
 void pass(phylo_mlp* p, int B, const float* X, const int* rows, const float* T, float* loss) {
     const Views w = views(p, p->d_w);
     const int H = p->n_hid;
-    const dim3 grid(tiles(H, kTileN) * tiles(B, kTileM)), block(kTileThreads);
-    hipLaunchKernelGGL(layer_kernel, grid, block, 0, p->stream, B, H, p->n_in, X, rows, w.W1, w.b1, p->d_h1);
-    hipLaunchKernelGGL(layer_kernel, grid, block, 0, p->stream, B, H, H, p->d_h1, nullptr, w.W2, w.b2, p->d_h2);
-    hipLaunchKernelGGL(output_kernel, dim3(loss_parts(p, B)), block, 0, p->stream, B, p->n_out, H, p->d_h2, w.W3, w.b3, T,
-                       rows, p->d_y, p->d_dy, loss);
+    const bool large = large_tiles(p, B, H);
+    const dim3 grid(large ? tiles(H, Large::N) * tiles(B, Large::M) : tiles(H, Small::N) * tiles(B, Small::M));
+    const dim3 block(large ? Large::THREADS : Small::THREADS);
+    const auto layer = [&](int n_in, const float* in, const int* in_rows, const float* W, const float* b, float* out) {
+        hipLaunchKernelGGL(large ? layer_kernel<Large> : layer_kernel<Small>, grid, block, 0, p->stream, B, H, n_in, in, in_rows,
+                           W, b, out);
+    };
+    layer(p->n_in, X, rows, w.W1, w.b1, p->d_h1);
+    layer(H, p->d_h1, nullptr, w.W2, w.b2, p->d_h2);
+    hipLaunchKernelGGL(output_kernel, dim3(loss_parts(p, B)), dim3(Small::THREADS), 0, p->stream, B, p->n_out, H, p->d_h2, w.W3,
+                       w.b3, T, rows, p->d_y, p->d_dy, loss);
     if (!T) return;
     hipLaunchKernelGGL(output_back_kernel, dim3(tiles(H, 64) * tiles(B, 8)), dim3(64), 0, p->stream, B, H, p->n_out, p->d_dy,
                        w.W3, p->d_h2, p->d_dh2);
-    hipLaunchKernelGGL(back_kernel, grid, block, 0, p->stream, B, H, H, p->d_dh2, p->d_w2t, p->d_h1, p->d_dh1);
+    hipLaunchKernelGGL(large ? back_kernel<Large> : back_kernel<Small>, grid, block, 0, p->stream, B, H, H, p->d_dh2, p->d_w2t, p->d_h1, p->d_dh1);
 }
 
 void transpose_w2(phylo_mlp* p) {
@@ -648,16 +688,19 @@ void gradients(phylo_mlp* p, int B, const float* X, const int* rows, const Adam&
     const auto off = [&](const float* q) { return (size_t)(q - p->d_w); };
     GradArgs a{p->n_in, p->n_hid, p->n_out, B, {}, {}, {off(o.W1), off(o.W2), off(o.W3)}, {off(o.b1), off(o.b2), off(o.b3)}};
     const int n_a[3] = {p->n_in, p->n_hid, p->n_hid}, n_d[3] = {p->n_hid, p->n_hid, p->n_out};
+    const bool large = large_tiles(p, p->n_hid, p->n_hid);
+    const int tile_m = large ? Large::M : Small::M, tile_n = large ? Large::N : Small::N;
+    const int threads = large ? Large::THREADS : Small::THREADS;
     int n = 0;
     for (int l = 0; l < 3; ++l) {
         a.tile[l] = n;
-        n += tiles(n_a[l], kTileM) * tiles(n_d[l], kTileN);
+        n += tiles(n_a[l], tile_m) * tiles(n_d[l], tile_n);
     }
     for (int l = 0; l < 3; ++l) {
         a.bias[l] = n;
-        n += tiles(n_d[l], kTileThreads);
+        n += tiles(n_d[l], threads);
     }
-    hipLaunchKernelGGL(gradient_kernel, dim3(n), dim3(kTileThreads), 0, p->stream, a, X, rows, p->d_h1, p->d_h2, p->d_dh1, p->d_dh2,
+    hipLaunchKernelGGL(large ? gradient_kernel<Large> : gradient_kernel<Small>, dim3(n), dim3(threads), 0, p->stream, a, X, rows, p->d_h1, p->d_h2, p->d_dh1, p->d_dh2,
                        p->d_dy, adam, p->d_g, p->d_w2t);
 }
 
@@ -790,6 +833,7 @@ int phylo_mlp_create(int device, int n_in, int n_hidden, int n_out, int max_batc
     auto alloc = [&](auto*& d, size_t n) { return hipMalloc(reinterpret_cast<void**>(&d), n * sizeof(*d)) == hipSuccess; };
     const size_t B = max_batch;
     if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&p->stream, hipStreamNonBlocking) != hipSuccess ||
+        hipDeviceGetAttribute(&p->n_cu, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
         !alloc(p->d_w, p->n_params) || !alloc(p->d_g, p->n_params) || !alloc(p->d_m, p->n_params) ||
         !alloc(p->d_v, p->n_params) || !alloc(p->d_x, B * n_in) || !alloc(p->d_t, B * n_out) ||
         !alloc(p->d_h1, B * n_hidden) || !alloc(p->d_h2, B * n_hidden) || !alloc(p->d_y, B * n_out) ||
