@@ -20,6 +20,10 @@ HIP_FLAGS = [
     # Packed FP32 instructions are kept out of every kernel.
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-command-line-argument",
+    # Host functions on cache lines: what one runs at then does not change with
+    # the code before it (the weights' generator of a new MLP: 456,000 values in
+    # 16.0 ms at offsets 0 and 32 of a line, 27.4 ms at 48).
+    "-Xarch_host", "-falign-functions=64",
 ]
 
 
