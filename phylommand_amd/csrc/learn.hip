@@ -262,8 +262,9 @@ __global__ __launch_bounds__(kSimThreads) void sim_features_kernel(
 // multiply-adds.  A workgroup of two waves owns a 16 x 32 tile (256 of them for
 // 256 x 512 outputs, 2 x 2 a thread) and stages 64 k of both operands in LDS
 // while the next two pieces are on their way into registers (what a launch reads
-// was written by the launch before, on other XCDs, so it comes from beyond L2).  (Rows by scalar loads
-// and columns from L1 waited in every 16-long piece: 18 us for 256 x 512 x 512.)
+// was written by the launch before, on other XCDs, so it comes from beyond L2):
+// 13.2 us for 256 x 512 x 512.  (Rows by scalar loads and columns from L1 waited
+// in every 16-long piece: 18 us.)
 // Wide layers and batches take 64 x 64 tiles, 4 x 4 a thread (large_tiles): the
 // same sums in the same order.
 // ---------------------------------------------------------------------------

@@ -51,10 +51,9 @@ struct NniArgs {
 // (site blocks x walks; 5 are resident): each segment repeats the walk from
 // the root to its start, so few segments move less memory (128 taxa x 100,000
 // sites: 64 edges a walk 0.538 ms, 32 0.585, 16 0.599; 6 to 18 workgroups
-// within 2 %), but a launch of few
-// site blocks needs the segments to fill the CUs.  One edge a walk where even
-// those leave a CU at most 16 waves (wide states, two products a wave: 8): the
-// launch then takes one chain's time whatever else it repeats.  Kernel us, 6
+// within 2 %), but a launch of few site blocks needs the segments to fill the
+// CUs.  One edge a walk where even those leave a CU at most 16 waves (wide
+// states: 8): the launch then takes one chain's time whatever else it repeats.  Kernel us, 6
 // edges / 1, 4 categories, 8 taxa x 64 sites 14.2 / 8.7, 120 x 500 (15 waves)
 // 27.8 / 17.8, 60 x 2000 (30) 21.2 / 22.9; 1 category, 120 x 2000 (15) 28.7 /
 // 19.8; 20 states, 8 x 64 26.9 / 14.4, 28 x 250 (7) 33.9 / 27.4, 28 x 500 (14)

@@ -42,9 +42,11 @@ __device__ __forceinline__ void matvec4t(const double* __restrict__ P, const dou
 // An edge issues about 220 vector instructions, 108 of them the FP64 products,
 // and reads two stored partials; issue (58 % busy) and the reads (1.0 GB of
 // partials, re-read once for the siblings) bind together, so five waves a
-// SIMD are asked for (80 registers; four 0.69, five 0.52 ms).  250 variants
-// of 128 taxa x 100,000 sites: 0.52 ms, 2.206 ms as one path-to-root program
-// a variant.
+// SIMD are asked for (FP32 80 registers, FP64 94; four 0.69, five 0.52 ms).
+// 250 variants of 128 taxa x 100,000 sites: 0.52 to 0.57 ms, 2.206 ms as one
+// path-to-root program a variant.  (The FP64 walk with site weights spills 6 to
+// 13 of its 96 registers: a call at 128 x 20,000 takes 0.365 ms, 0.336 without
+// weights.)
 template <typename T, int C, bool TL, bool BATCH, bool WEIGHTED>
 __global__ __launch_bounds__(64 * C, 5) void nni4_kernel(
     const NniOp* __restrict__ ops, const int* __restrict__ prog_begin, const NniInst* __restrict__ insts, NniInst one,

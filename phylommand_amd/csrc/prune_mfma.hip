@@ -592,9 +592,10 @@ __global__ __launch_bounds__(64 * C, (V <= 5 ? 3 : 1)) void prune_mfma_kernel(
 // (PmT, the same operand order) carries the outer partial down.  The outer
 // partial and one child factor stay in registers between edges.  One site
 // group a wave: two need 168 registers and spill 188 in the loop, one fits 128
-// (20 states), four waves a SIMD to hide the chain of dependent products that
-// binds it.  74 variants of 40 taxa x 5,000 sites, 20 states: 0.176 ms, 0.44 ms
-// as one path-to-root program a variant.
+// (up to 20 states), four waves a SIMD to hide the chain of dependent products
+// that binds it (29 to 32 states: 168 registers at three waves, 8 to 10 spilled).
+// 74 variants of 40 taxa x 5,000 sites, 20 states: 0.18 ms, 0.44 ms as one
+// path-to-root program a variant.
 template <typename T, int C, int V, int G>
 __global__ __launch_bounds__(64 * C, (V <= 5 ? 4 : 3)) void nni_mfma_kernel(
     const NniOp* __restrict__ ops, const int* __restrict__ prog_begin, int n_prog, const uint32_t* __restrict__ tips,
